@@ -22,6 +22,7 @@ Keys of a case:
 import math
 
 import numpy as np
+import torch
 
 import graphchallenge21_amd as gc
 
@@ -131,20 +132,24 @@ def _answers(case):
     return max(1, min(case["batch"], int(1.25 * case["survive"] * case["batch"])))
 
 
+def _layers(case, rng):
+    """The distinct layers of a network that is set up from arrays, in the order in which they repeat."""
+    kind, n, layers = case["kind"], case["neuron"], case["layers"]
+    if kind == "irregular":
+        return [_irregular_layer(rng, n, case["nnz"]) for _ in range(min(layers, 6))]
+    perm = rng.permutation(n).astype(np.int32) if kind == "radix-common" else None
+    strides = [16 << k for k in range(int(math.log2(n // 16)))]
+    return [_radix_layer(rng, n, s, perm) for s in strides[:layers]]
+
+
 def prepare(case, seed):
     kind, n, layers, batch = case["kind"], case["neuron"], case["layers"], case["batch"]
     rng = np.random.default_rng(seed)
     net = gc.Network(n, batch, layers, bias=_bias(n))
     if kind == "band":
         net.synth_layers(seed, nnz_per_row=case["nnz"], value=2.0 / case["nnz"])
-    elif kind == "irregular":
-        kinds = [_irregular_layer(rng, n, case["nnz"]) for _ in range(min(layers, 6))]
-        for l in range(layers):
-            net.set_layer_csr(l, *kinds[l % len(kinds)])
     else:
-        perm = rng.permutation(n).astype(np.int32) if kind == "radix-common" else None
-        strides = [16 << k for k in range(int(math.log2(n // 16)))]
-        kinds = [_radix_layer(rng, n, s, perm) for s in strides[:layers]]
+        kinds = _layers(case, rng)
         for l in range(layers):
             net.set_layer_csr(l, *kinds[l % len(kinds)])
     net.inspect()
@@ -166,6 +171,40 @@ def run(state):
     survived = np.zeros(state["batch"], bool)
     survived[ids] = True
     return {"survived": survived, "activations": net.activations(np.resize(ids, state["answers"]))}
+
+
+def exact(case, seed):
+    """The layer chain in 64 bits (the inputs are the generators' own, the arithmetic is torch's)."""
+    n, layers, batch = case["neuron"], case["layers"], case["batch"]
+    if batch * n > 1 << 26:
+        return None
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    kinds = [] if case["kind"] == "band" else _layers(case, np.random.default_rng(seed))
+    y = torch.from_numpy(gc.synth_features_host(seed, n, 0, batch, *_densities(case))).to(dev, torch.float64).T.contiguous()
+    rows = torch.arange(batch, device=dev)
+    bias = float(np.float32(_bias(n)))
+    for l in range(layers):
+        rowptr, col, val = kinds[l % len(kinds)] if kinds else gc.synth_layer_csr(seed, l, n, case["nnz"], 2.0 / case["nnz"])
+        length = np.diff(rowptr)
+        out = torch.zeros_like(y)
+        for k in range(int(length.max())):
+            at = np.flatnonzero(length > k)
+            i = torch.from_numpy(at).to(dev)
+            c = torch.from_numpy(col[rowptr[at] + k].astype(np.int64)).to(dev)
+            w = torch.from_numpy(val[rowptr[at] + k].astype(np.float64)).to(dev)
+            out[i] += w[:, None] * y[c]
+        out += bias
+        if (out.amax(dim=0).abs() < 1e-5).any():
+            return None   # a row on the edge of dying: rounding decides whether it is among the answers
+        y = out.clamp_(0.0, 32.0)
+        if case["prune"]:
+            live = (y != 0).any(dim=0)
+            y, rows = y[:, live].contiguous(), rows[live]
+    live = (y != 0).any(dim=0)
+    ids = rows[live].cpu().numpy()
+    survived = np.zeros(batch, bool)
+    survived[ids] = True
+    return {"survived": survived, "activations": np.resize(y[:, live].T.cpu().numpy(), (_answers(case), n))}
 
 
 def work(case):
