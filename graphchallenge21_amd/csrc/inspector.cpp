@@ -1038,4 +1038,35 @@ void link_layers(LayerPlan& cur, const std::vector<int32_t>* next_in_pos) {
     link(cur.alt_out_at, cur.alt_dst);
 }
 
+int sum_groups(const LayerPlan& p) {
+    if (p.kernel == SPDNN_KERNEL_BAND && p.alt_ngroups > 0) return p.alt_ngroups;
+    if (p.kernel == SPDNN_KERNEL_BLOCK && p.wmode == 0) return p.ngroups;
+    return 0;
+}
+
+void link_sums(const LayerPlan& prev, LayerPlan& cur, int N) {
+    cur.sum_cols.clear();
+    const int G = sum_groups(cur);
+    if (G == 0 || sum_groups(prev) != G) return;
+    const bool alt = cur.kernel == SPDNN_KERNEL_BAND, palt = prev.kernel == SPDNN_KERNEL_BAND;
+    const std::vector<int32_t>& cols = alt ? cur.alt_cols : cur.blk_cols;
+    const std::vector<int32_t>& cnt = alt ? cur.alt_cnt : cur.blk_cnt;
+    const std::vector<int32_t>& pdst = palt ? prev.alt_dst : prev.dst;
+    const bool full = alt ? cur.alt_full : cur.blk_full;
+    if (G + (full ? 0 : 1) > 4096 || (int)pdst.size() < 16 * G) return;
+    std::vector<int32_t> owner((size_t)N, -1);   // group of `prev` that computes a physical column of cur's input
+    for (int s = 0; s < 16 * G; ++s)
+        if (pdst[(size_t)s] >= 0) owner[(size_t)pdst[(size_t)s]] = s / 16;
+    std::vector<uint16_t> out((size_t)G * 32);
+    for (int g = 0; g < G; ++g) {
+        const int c = full ? 32 : cnt[(size_t)g];
+        for (int k = 0; k < 32; ++k) {
+            const int o = k < c ? owner[(size_t)cols[(size_t)g * 32 + k]] : G;
+            if (o < 0) return;
+            out[((size_t)(k / 8) * G + g) * 8 + (k % 8)] = (uint16_t)(o * 16);
+        }
+    }
+    cur.sum_cols.swap(out);
+}
+
 }  // namespace spdnn

@@ -85,6 +85,11 @@ struct LayerPlan {
     // the column's slot in the panel as raw bits, weight)
     int ntiles = 0;
     int rc_cycles = 0;         // run chains: cycles of groups the layer's own labelling found
+    // Where this layer and the one before it are both made of groups of equal outputs (BLOCK form, one exact weight): the
+    // group sum of the layer before that each of a group's inputs is, in accumulation order - [4][ngroups][8] as
+    // (number of that group) * 16, lists of fewer than 32 padded with ngroups * 16, the place of a zero.  Empty where
+    // there is no such form (see link_sums).
+    std::vector<uint16_t> sum_cols;
     bool self_aligned = false;
     bool pair_twins = false;   // BAND, one exact weight: the two outputs of every pair use the same inputs
     bool fuse_next = false;
@@ -161,5 +166,11 @@ bool pair_fusable(const LayerPlan& a, const LayerPlan& b, int N);
 
 // dst[slot] = physical column (in the next buffer) of the neuron computed at `slot`.
 void link_layers(LayerPlan& cur, const std::vector<int32_t>* next_in_pos);
+
+// Groups of equal outputs in the BLOCK form of a layer with one exact weight: how many, 0 without such a form.
+int sum_groups(const LayerPlan& p);
+// cur.sum_cols from the layer before it (linked to cur already); empty where one of the two has no groups of equal
+// outputs, their numbers of groups differ or there are more of them than 16-bit byte offsets of 16 hold.
+void link_sums(const LayerPlan& prev, LayerPlan& cur, int N);
 
 }  // namespace spdnn

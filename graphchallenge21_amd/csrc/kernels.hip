@@ -426,6 +426,7 @@ __device__ __forceinline__ float relu_clamp(float y, float clampv) {
 // ------------------------------------------------------------------------------------------
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 load_const_u4(const __attribute__((address_space(4))) uint32_t* p) {
     const u32x4_t v = *(const __attribute__((address_space(4))) u32x4_t*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
@@ -2014,6 +2015,225 @@ __global__ __launch_bounds__(1024) void block_resident_kernel(ResidentArgs a) {
     if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
 }
 
+// ------------------------------------------------------------------------------------------
+// Group sums (see launch_sums_head): layers of equal groups behind one another carry one column per group.
+// ------------------------------------------------------------------------------------------
+// The first layer of such a run: block_kernel's loads and sums, one store per group.
+// Every column is read by two groups; at 60000 x 65536 (15.7 GB) 4.5 ms, where the walk that writes full columns takes 5.25.
+template <int RL, bool FULL>
+__global__ __launch_bounds__(256) void sums_head_kernel(
+    Feat yin_all, Feat yout_all, const int32_t* __restrict__ grp_cols, const int32_t* __restrict__ grp_cnt,
+    int32_t* __restrict__ active, int32_t* __restrict__ count_prev, int N, int ngroups, int gpw, int stamp,
+    int prev_stamp, int check_dead, float wu, float bias, float clampv, Publish pub) {
+    using V = typename VecOf<RL>::type;
+    constexpr int RB = 64 * RL;
+    publish_counts(pub);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int rb = blockIdx.x;
+    if (enter_row_block<RL>(active, (size_t)rb * RB + lane * RL, prev_stamp, stamp, check_dead, count_prev,
+                            blockIdx.y == 0 && wave == 0))
+        return;
+    const int loff = lane * RL;
+    const float* __restrict__ yin = block_base(yin_all, rb, (size_t)N * RB) + loff;
+    float* __restrict__ yout = block_base(yout_all, rb, (size_t)ngroups * RB) + loff;
+    const int g0 = (blockIdx.y * 4 + wave) * gpw;
+    const int g1 = min(ngroups, g0 + gpw);
+    float nz[RL];
+#pragma unroll
+    for (int q = 0; q < RL; ++q) nz[q] = 0.0f;
+    for (int g = g0; g < g1; ++g) {
+        const int S = FULL ? 32 : grp_cnt[g];
+        const int32_t* cp = grp_cols + (size_t)g * 32;
+        float x[32][RL];
+#pragma unroll
+        for (int m = 0; m < 32; ++m) {
+            if (FULL || m < S) {
+                vec_to_arr<RL>(*reinterpret_cast<const V*>(yin + (size_t)cp[m] * RB), x[m]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < RL; ++q) x[m][q] = 0.0f;
+            }
+        }
+        float acc[RL];
+#pragma unroll
+        for (int q = 0; q < RL; ++q) acc[q] = 0.0f;
+#pragma unroll
+        for (int m = 0; m < 32; ++m) {
+            if (FULL || m < S) {
+#pragma unroll
+                for (int q = 0; q < RL; ++q) acc[q] = mac<0>(acc[q], x[m][q], wu);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < RL; ++q) {
+            acc[q] = relu_clamp(acc[q] + bias, clampv);
+            nz[q] = nz_merge(nz[q], acc[q]);
+        }
+        *reinterpret_cast<V*>(yout + (size_t)g * RB) = arr_to_vec<RL>(acc);
+    }
+    stamp_rows<RL>(nz, active, (size_t)rb * RB + loff, stamp);
+}
+
+// Group sums written out: column dst[16 g + o] of the full layout is group g's, for every output o of the group.
+template <int RL>
+__global__ __launch_bounds__(256) void sums_expand_kernel(Feat sums, Feat full, const int32_t* __restrict__ dst, int N,
+                                                          int ngroups, int gpw) {
+    using V = typename VecOf<RL>::type;
+    constexpr int RB = 64 * RL;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int rb = blockIdx.x, loff = (threadIdx.x & 63) * RL;
+    const float* __restrict__ in = block_base(sums, rb, (size_t)ngroups * RB) + loff;
+    float* __restrict__ out = block_base(full, rb, (size_t)N * RB) + loff;
+    const int g0 = (blockIdx.y * 4 + wave) * gpw;
+    const int g1 = min(ngroups, g0 + gpw);
+    for (int g = g0; g < g1; ++g) {
+        const V v = *reinterpret_cast<const V*>(in + (size_t)g * RB);
+#pragma unroll
+        for (int o = 0; o < 16; ++o) {
+            const int d = dst[(size_t)g * 16 + o];
+            if (d >= 0) *reinterpret_cast<V*>(out + (size_t)d * RB) = v;
+        }
+    }
+}
+
+// Further layers of the run, R rows (4, 2 or 1) of a workgroup in LDS from the first to the last: two buffers of
+// ngroups + 1 places of R rows (the last one a zero, which the lists of groups with fewer than 32 inputs are padded
+// with).  Thread t takes groups t, t + blockDim, ...: its list is 32 16-bit byte offsets (four 16-byte loads, requested
+// one group ahead across the layers), an input is one LDS read of R rows.  Bound by those reads: the places of a
+// wave's 64 lanes are as random as the layer's relabelling, and a read of 64 x 16 bytes takes 20 cycles instead of 8.
+// Per layer, against the launches that carry full columns: 65536 neurons, 60160 rows 1.57 ms against 5.25, 2304 rows
+// 67 us against 180; 16384 neurons, 512 rows 2.6 us against 15.7; 1024 neurons, 2304 rows 1.1 us against 1.8.
+// Accumulation as in block_body: ascending input index,
+// multiply-add by the one exact weight, bias last.  One barrier per layer; rows are stamped with the last layer that
+// left them nonzero, a workgroup whose rows are all zero stops.
+struct SumsArgs {
+    const LayerDesc* table;
+    int nlayers;
+    Feat yin, yout;
+    int32_t* active;
+    int ngroups, rl;
+    int stamp0, prev_stamp, check_dead;
+    float bias, clampv;
+    Publish pub;
+};
+
+template <int R>
+__global__ __launch_bounds__(1024) void sums_resident_kernel(SumsArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int sh_alive[3];
+    constexpr int SHIFT = R == 4 ? 0 : R == 2 ? 1 : 2;   // the lists hold places of 16 bytes
+    using V = typename VecOf<R>::type;
+    using GQ = const __attribute__((address_space(1))) u32x4_t*;
+    publish_counts(a.pub);
+    const int t = (int)threadIdx.x, lane = t & 63, nthr = (int)blockDim.x;
+    const int RB = 64 * a.rl, G = a.ngroups;
+    // (every XCD takes a contiguous eighth of the rows: the workgroups that share a line of a column find it in one L2)
+    const unsigned nwg = gridDim.x;
+    const unsigned wg = (nwg % 8u) == 0u ? (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u : blockIdx.x;
+    const size_t row0 = (size_t)wg * R;
+    const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
+    bool all_dead = false;
+    if (a.check_dead && a.prev_stamp != 0) {
+        int alive = 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        if (__syncthreads_or(alive) == 0) return;   // a row block without an active row is skipped, as by the per-layer kernels
+        int own = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) own |= (a.active[row0 + r] == a.prev_stamp) ? 1 : 0;
+        all_dead = __builtin_amdgcn_readfirstlane(own) == 0;   // (the same four words for every thread)
+    }
+    const uint32_t buf_bytes = (uint32_t)(G + 1) * R * 4;
+    const size_t blkf = (size_t)G * RB;
+    float* __restrict__ gout = block_base(a.yout, rb, blkf) + rin;
+    if (all_dead) {   // zero rows of a row block that goes on
+        for (int g = t; g < G; g += nthr) *reinterpret_cast<V*>(gout + (size_t)g * RB) = V{};
+        return;
+    }
+    const float* __restrict__ gin = block_base(a.yin, rb, blkf) + rin;
+    for (int g = t; g < G; g += nthr) *reinterpret_cast<V*>(smem + (uint32_t)g * (R * 4)) = *reinterpret_cast<const V*>(gin + (size_t)g * RB);
+    if (t < 2) *reinterpret_cast<V*>(smem + (uint32_t)t * buf_bytes + (uint32_t)G * (R * 4)) = V{};
+    if (t < 3) sh_alive[t] = 0;
+    const int trips = (G + nthr - 1) / nthr;
+    u32x4_t next[4];
+    // (a layer's entry of the table is read a layer before it is needed: a scalar load at the top of a layer, and the
+    // loads that need its pointer, would be waited for by all waves at once)
+    GQ cols_here = (GQ)load_layer_desc(a.table, 0).sum_cols, cols_next = (GQ)load_layer_desc(a.table, min(1, a.nlayers - 1)).sum_cols;
+    float wu = load_layer_desc(a.table, 0).wu, wu_next = load_layer_desc(a.table, min(1, a.nlayers - 1)).wu;
+    auto request = [&](GQ cols, int trip) {
+        const int g = min(t + trip * nthr, G - 1);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) next[c] = cols[(size_t)c * G + g];
+    };
+    request(cols_here, 0);
+    int last_alive = -1, done_layers = 0;
+    ring_barrier<1>();
+    for (int j = 0; j < a.nlayers; ++j) {
+        const unsigned char* const in = smem + ((j & 1) ? buf_bytes : 0u);
+        unsigned char* const out = smem + ((j & 1) ? 0u : buf_bytes);
+        const int ahead = min(j + 2, a.nlayers - 1);
+        const GQ cols_ahead = (GQ)load_layer_desc(a.table, ahead).sum_cols;
+        const float wu_ahead = load_layer_desc(a.table, ahead).wu;
+        float nz[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) nz[q] = 0.0f;
+        for (int trip = 0; trip < trips; ++trip) {
+            u32x4_t cur[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) cur[c] = next[c];
+            if (trip + 1 < trips) request(cols_here, trip + 1);
+            else if (j + 1 < a.nlayers) request(cols_next, 0);
+            float acc[R];
+#pragma unroll
+            for (int q = 0; q < R; ++q) acc[q] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                V x[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const uint32_t d = cur[c][k >> 1];
+                    const uint32_t off = ((k & 1) ? (d >> 16) : (d & 0xffffu)) >> SHIFT;
+                    x[k] = *reinterpret_cast<const V*>(in + off);
+                }
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    float xa[R];
+                    vec_to_arr<R>(x[k], xa);
+#pragma unroll
+                    for (int q = 0; q < R; ++q) acc[q] = mac<0>(acc[q], xa[q], wu);
+                }
+            }
+            const int g = t + trip * nthr;
+#pragma unroll
+            for (int q = 0; q < R; ++q) acc[q] = relu_clamp(acc[q] + a.bias, a.clampv);
+            if (g < G) {
+#pragma unroll
+                for (int q = 0; q < R; ++q) nz[q] = nz_merge(nz[q], acc[q]);
+                *reinterpret_cast<V*>(out + (uint32_t)g * (R * 4)) = arr_to_vec<R>(acc);
+            }
+        }
+        int bits = 0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) bits |= __ballot(nz[q] > 0.0f ? 1 : 0) != 0ull ? 1 << q : 0;
+        if (lane == 0 && bits != 0) atomicOr(&sh_alive[j % 3], bits);
+        ring_barrier<1>();
+        const int mask = sh_alive[j % 3];
+        if (t == 0) sh_alive[(j + 2) % 3] = 0;
+        if (t < R && ((mask >> t) & 1)) last_alive = j;
+        done_layers = j + 1;
+        cols_here = cols_next; cols_next = cols_ahead;
+        wu = wu_next; wu_next = wu_ahead;
+        if (mask == 0 && a.bias <= 0.0f) { all_dead = true; break; }   // zero rows stay zero
+    }
+    const unsigned char* const fin = smem + ((done_layers & 1) ? buf_bytes : 0u);
+    for (int g = t; g < G; g += nthr) {
+        V v{};
+        if (!all_dead) v = *reinterpret_cast<const V*>(fin + (uint32_t)g * (R * 4));
+        *reinterpret_cast<V*>(gout + (size_t)g * RB) = v;
+    }
+    if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
+}
+
 // The resident launch of TILED layers: block_resident_kernel's frame (R rows of a workgroup in LDS through all layers
 // of the launch, two buffers, one barrier per layer, rows stamped with the last layer that left them nonzero, a
 // workgroup whose rows are all zero stops) around rowtile_kernel's arithmetic (thread t computes whole outputs - slots
@@ -3272,6 +3492,72 @@ hipError_t launch_block(const BlockLaunch& a, hipStream_t s) {
 #undef SPDNN_BLOCK_WM
 #undef SPDNN_BLOCK
     return hipGetLastError();
+}
+
+hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s) {
+    if (a.N <= 0 || a.ngroups <= 0 || a.nblk <= 0 || !a.yin || !a.yout || a.yin == a.yout || !a.cols || !a.cnt || !a.active ||
+        a.wmode != 0 || a.ngroups > a.N)
+        return hipErrorInvalidValue;
+    int gpw = 8;   // groups per wave, as in launch_block
+    while (gpw > 1 && (long long)a.nblk * ((a.ngroups + 4 * gpw - 1) / (4 * gpw)) < 2048) gpw >>= 1;
+    dim3 grid(a.nblk, (a.ngroups + 4 * gpw - 1) / (4 * gpw)), block(256);
+    if (grid.y > 65535) return hipErrorInvalidValue;
+#define SPDNN_HEAD(RLv, FL)                                                                                            \
+    hipLaunchKernelGGL((sums_head_kernel<RLv, FL>), grid, block, 0, s, a.yin, a.yout, a.cols, a.cnt, a.active,         \
+                       a.count_prev, a.N, a.ngroups, gpw, a.stamp, a.prev_stamp, a.check_dead, a.wu, a.bias, a.clampv, \
+                       a.publish)
+    switch (a.rl) {
+        case 4: if (a.full) SPDNN_HEAD(4, true); else SPDNN_HEAD(4, false); break;
+        case 2: if (a.full) SPDNN_HEAD(2, true); else SPDNN_HEAD(2, false); break;
+        case 1: if (a.full) SPDNN_HEAD(1, true); else SPDNN_HEAD(1, false); break;
+        default: return hipErrorInvalidValue;
+    }
+#undef SPDNN_HEAD
+    return hipGetLastError();
+}
+
+hipError_t launch_sums_expand(const Feat& sums, const Feat& full, const int32_t* dst, int N, int ngroups, int nblk, int rl,
+                              hipStream_t s) {
+    if (N <= 0 || ngroups <= 0 || ngroups > N || nblk <= 0 || !sums || !full || sums == full || !dst) return hipErrorInvalidValue;
+    int gpw = 8;
+    while (gpw > 1 && (long long)nblk * ((ngroups + 4 * gpw - 1) / (4 * gpw)) < 2048) gpw >>= 1;
+    dim3 grid(nblk, (ngroups + 4 * gpw - 1) / (4 * gpw)), block(256);
+    if (grid.y > 65535) return hipErrorInvalidValue;
+    switch (rl) {
+        case 4: hipLaunchKernelGGL(sums_expand_kernel<4>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
+        case 2: hipLaunchKernelGGL(sums_expand_kernel<2>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
+        case 1: hipLaunchKernelGGL(sums_expand_kernel<1>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <int R>
+static hipError_t launch_sums_resident_r(const SumsLaunch& a, int nthr, hipStream_t s) {
+    SumsArgs k{};
+    k.table = a.table; k.nlayers = a.nlayers; k.yin = a.yin; k.yout = a.yout; k.active = a.active; k.ngroups = a.ngroups; k.rl = a.rl;
+    k.stamp0 = a.stamp0; k.prev_stamp = a.prev_stamp; k.check_dead = a.check_dead; k.bias = a.bias; k.clampv = a.clampv;
+    k.pub = a.publish;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(sums_resident_kernel<R>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(sums_resident_kernel<R>, dim3((unsigned)(a.rows / R)), dim3((unsigned)nthr),
+                       (size_t)(a.ngroups + 1) * R * 8, s, k);
+    return hipGetLastError();
+}
+
+hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s) {
+    // host-side shape checks: what the 16-bit lists and the two LDS buffers assume
+    if (a.nlayers < 1 || !a.table || !a.yin || !a.yout || a.yin == a.yout || !a.active || a.ngroups <= 0 || a.ngroups > 4096 ||
+        a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0)
+        return hipErrorInvalidValue;
+    const int nthr = std::min(1024, (a.ngroups + 63) / 64 * 64);
+    // fewer rows per workgroup where four would leave CUs without one
+    const long long threads = (long long)a.n_cu * 1024;
+    int R = 4;
+    while (R > 1 && (long long)(a.rows / R) * nthr < threads) R /= 2;
+    return R == 4 ? launch_sums_resident_r<4>(a, nthr, s) : R == 2 ? launch_sums_resident_r<2>(a, nthr, s)
+                                                                   : launch_sums_resident_r<1>(a, nthr, s);
 }
 
 hipError_t launch_scan_active(const int32_t* active, const int32_t* gid, int rows, int stamp, int32_t* count,

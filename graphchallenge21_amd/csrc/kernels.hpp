@@ -152,6 +152,31 @@ struct BlockLaunch {
 };
 hipError_t launch_block(const BlockLaunch& a, hipStream_t s);
 
+// Group sums.  In a layer whose groups of (up to 16) outputs share their inputs and the one exact weight, all outputs
+// of a group are equal: its result is one column per GROUP.  Where the next layer has such groups too its inputs can
+// be named by the group that computes them (LayerPlan::sum_cols), and everything between the two layers - memory,
+// LDS, compactions - carries ngroups columns instead of N.
+//   launch_sums_head: the first such layer, from the full columns (cols / cnt of its BLOCK form) to group sums
+//   launch_sums_resident: `nlayers` further ones from group sums to group sums, R rows of a workgroup in LDS throughout
+//   launch_sums_expand: group sums written out as the full columns that any kernel may read
+// Buffers of group sums have the row-block layout with ngroups columns.
+hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s);
+struct LayerDesc;   // (a.wmode 0; a.dst is not used)
+struct SumsLaunch {
+    const LayerDesc* table;       // device pointer to the entry of the launch's first layer
+    int nlayers;
+    Feat yin, yout;               // group sums in, group sums out (another buffer)
+    int32_t* active;
+    int ngroups, rows, rl;        // rows: carried rows (whole row blocks)
+    int stamp0, prev_stamp, check_dead;
+    int n_cu;
+    float bias, clampv;
+    Publish publish;
+};
+hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s);
+hipError_t launch_sums_expand(const Feat& sums, const Feat& full, const int32_t* dst, int N, int ngroups, int nblk, int rl,
+                              hipStream_t s);
+
 // ------------------------------------------------------------------------------------------
 // Several layers per launch ("persistent" launches): the per-layer decomposition - many segments
 // per row block - kept, with a dependency per ROW BLOCK where the per-layer launches have a launch
@@ -193,6 +218,8 @@ struct LayerDesc {           // one entry of the device-side layer table
     int quad_groups;
     const uint32_t* quad_col;
     const float* quad_w;
+    // group sums of the layer before (layers of equal groups behind one another)
+    const uint16_t* sum_cols;
 };
 
 struct PersistCtl {          // device words of one persistent launch (zero before the launch)

@@ -185,12 +185,13 @@ struct DevLayer {
     uint32_t* rt_ent = nullptr;    // (with alt_cnt / alt_dst: its ROWTILE form)
     uint32_t* quad_col = nullptr;  // the QUAD form of a BAND layer (with dst)
     float* quad_w = nullptr;
+    uint16_t* sum_cols = nullptr;  // inputs named by the groups of the layer before
 };
 
 // Where the arrays of one layer's plan lie inside its block of device memory (and inside the
 // pinned host copy of that block when plans are streamed): pairs, ell, rowlen, wv, dst, blk_cols,
-// blk_cnt, alt_cols, alt_cnt, alt_dst, alt_wv, rt_ent, quad_col, quad_w, each aligned to 256 bytes.
-constexpr int kPlanArrays = 14;
+// blk_cnt, alt_cols, alt_cnt, alt_dst, alt_wv, rt_ent, quad_col, quad_w, sum_cols, each aligned to 256 bytes.
+constexpr int kPlanArrays = 15;
 struct PlanLayout {
     size_t off[kPlanArrays] = {};
     size_t len[kPlanArrays] = {};
@@ -303,6 +304,7 @@ struct spdnn_net {
     int64_t tiled_min_rows = 8192;                    // see use_gather_form (SPDNN_TILED_MIN_ROWS)
     bool tiled_min_rows_given = false;                // ... set in the environment: also layers with a ROWTILE form follow it
     int rowtile_mode = 1;                             // TILED layers up to 8192 neurons wide run their ROWTILE form (SPDNN_ROWTILE=0: the tiles)
+    int sums_mode = 1;                                // layers of equal groups behind one another carry group sums (SPDNN_GROUP_SUMS=0: never)
     int band_resident_mode = 1;                       // BAND layers up to 1024 neurons wide join resident launches (SPDNN_BAND_RESIDENT=0: never)
     int band_resident_min_layers = 0;                 // ... of at least this many layers (SPDNN_BAND_RESIDENT_MIN_LAYERS; 0: 6, from 16384 rows up 16)
     long long stream_min_bytes = 96ll << 20;          // see BandLaunch (SPDNN_STREAM_MIN_BYTES, read at creation)
@@ -585,7 +587,7 @@ PlanLayout plan_layout(const LayerPlan& p) {
     const size_t len[kPlanArrays] = {p.pairs.size() * 4,    p.ell_col.size() * 4,  p.rowlen.size() * 4,   p.wv.size() * 4,
                                      p.dst.size() * 4,      p.blk_cols.size() * 4, p.blk_cnt.size() * 4,  p.alt_cols.size() * 4,
                                      p.alt_cnt.size() * 4,  p.alt_dst.size() * 4,  p.alt_wv.size() * 4,
-                                     p.rt_ent.size() * 4,   p.quad_col.size() * 4, p.quad_w.size() * 4};
+                                     p.rt_ent.size() * 4,   p.quad_col.size() * 4, p.quad_w.size() * 4,   p.sum_cols.size() * 2};
     for (int k = 0; k < kPlanArrays; ++k) {
         y.off[k] = y.bytes;
         y.len[k] = len[k];
@@ -597,7 +599,7 @@ PlanLayout plan_layout(const LayerPlan& p) {
 void pack_plan(const LayerPlan& p, const PlanLayout& y, char* dst) {
     const void* src[kPlanArrays] = {p.pairs.data(),   p.ell_col.data(),  p.rowlen.data(),  p.wv.data(),      p.dst.data(),
                                     p.blk_cols.data(), p.blk_cnt.data(), p.alt_cols.data(), p.alt_cnt.data(), p.alt_dst.data(),
-                                    p.alt_wv.data(),   p.rt_ent.data(),   p.quad_col.data(), p.quad_w.data()};
+                                    p.alt_wv.data(),   p.rt_ent.data(),   p.quad_col.data(), p.quad_w.data(),   p.sum_cols.data()};
     for (int k = 0; k < kPlanArrays; ++k)
         if (y.len[k]) memcpy(dst + y.off[k], src[k], y.len[k]);
 }
@@ -619,6 +621,7 @@ DevLayer plan_at(const PlanLayout& y, char* base) {
     d.rt_ent = (uint32_t*)at(11);
     d.quad_col = (uint32_t*)at(12);
     d.quad_w = (float*)at(13);
+    d.sum_cols = (uint16_t*)at(14);
     return d;
 }
 
@@ -650,6 +653,7 @@ int upload_plans(spdnn_net* n) {
             LayerDesc& t = table[l];
             t = LayerDesc{};
             t.wu = p.info.value;
+            t.sum_cols = n->dl[l].sum_cols;
             if (p.kernel == SPDNN_KERNEL_BAND) {
                 t.pairs = n->dl[l].pairs;
                 t.pw = n->dl[l].wv;
@@ -920,6 +924,7 @@ static int spdnn_create_impl(int neuron, int max_batch, int layers, float bias, 
     if (const char* e = getenv("SPDNN_PERSIST_LIGHT_SYNC")) n->persist_light = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_SEGLEN")) n->persist_seglen = std::max(0, atoi(e));
     if (const char* e = getenv("SPDNN_RESIDENT")) n->resident_mode = atoi(e) != 0 ? 1 : 0;
+    if (const char* e = getenv("SPDNN_GROUP_SUMS")) n->sums_mode = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_WAIT_US")) n->persist_wait_us = std::max(0ll, atoll(e));
     if (const char* e = getenv("SPDNN_BAND_SEGLEN")) n->band_seglen = std::max(0, atoi(e));
     if (const char* e = getenv("SPDNN_BAND_DIRECT_LDS")) n->band_direct_lds = atoi(e) != 0 ? 1 : 0;
@@ -1172,6 +1177,17 @@ static int spdnn_inspect_impl(spdnn_net* n) {
         LayerPlan* cur = &n->layers[(size_t)l];
         const std::vector<int32_t>* nxt = l + 1 < n->L ? &n->layers[(size_t)l + 1].in_pos : nullptr;
         n->pool->submit([=] { link_layers(*cur, nxt); });
+    }
+    n->pool->wait_all();
+    // (streamed plans run layer by layer: no launch there reads this form)
+    const bool streamed = n->plan_window >= 2 && n->plan_window < n->L;
+    n->layers[0].sum_cols.clear();
+    for (int l = 1; l < n->L; ++l) {
+        LayerPlan *prev = &n->layers[(size_t)l - 1], *cur = &n->layers[(size_t)l];
+        cur->sum_cols.clear();
+        const int N = n->N;
+        if (!streamed && n->sums_mode && sum_groups(*cur) > 0)
+            n->pool->submit([=] { link_sums(*prev, *cur, N); });
     }
     n->pool->wait_all();
     for (int l = 0; l < n->L; ++l) {
@@ -1783,10 +1799,22 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
         Feat cur; int cur_layer, carried, stamp, last_stamp; bool blocks_skipped;
         int l; bool dead, count_pending; int last_launched; int64_t newest_count; int c_prune;
         Publish pub; size_t nrecs, processed, ntimed; spdnn_run_result r;
+        int sums;   // columns of n->cur where it holds group sums (see launch_sums_head), 0: the full layout
     };
     State st{};
     st.l = first; st.dead = n->carried == 0; st.count_pending = false; st.last_launched = -1; st.newest_count = -1;
-    st.c_prune = 1; st.pub = Publish{}; st.processed = 0; st.r = spdnn_run_result{};
+    st.c_prune = 1; st.pub = Publish{}; st.processed = 0; st.r = spdnn_run_result{}; st.sums = 0;
+    // group sums of layer l - 1 written out for whatever reads the full columns next
+    auto expand_sums = [&](int l) -> hipError_t {
+        const LayerPlan& p = n->layers[(size_t)l - 1];
+        const DevLayer& d = n->dl[(size_t)l - 1];
+        const Feat full = (n->cur == n->A) ? n->C : n->A;
+        const hipError_t e = launch_sums_expand(n->cur, full, p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst, n->N, st.sums,
+                                                n->carried / n->RB, n->rl, n->stream);
+        n->cur = full;
+        st.sums = 0;
+        return e;
+    };
     auto save = [&]() {
         State s = st;
         s.cur = n->cur; s.cur_layer = n->cur_layer; s.carried = n->carried; s.stamp = n->stamp; s.last_stamp = n->last_stamp;
@@ -1912,7 +1940,24 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             // (with at most 16 rows known alive - the rows of one workgroup of a resident launch - the run is about to end:
             // layer by layer, so that the host sees the end when it comes instead of queueing launches of many layers)
             if (opt.prune && !persist_asked && st.newest_count >= 0 && st.newest_count <= 16) cmax = 1;
-            if (!fb && persist_on && n->resident_mode && n->d_table && (rsig = resident_sig(n, l)).ok) {
+            // Layers of equal groups carry group sums (see launch_sums_head) from the second one on: the first by the head
+            // launch, which reads the full columns, the others by resident launches on a sixteenth of the columns; three
+            // layers at least, or the head and the expansion behind it cost more than they save.
+            const bool sums_on = !fb && persist_on && !persist_asked && n->resident_mode && n->sums_mode && n->d_table;
+            auto takes_sums = [&](int k) { return k <= last && !n->layers[(size_t)k].sum_cols.empty(); };
+            if (st.sums && !(sums_on && takes_sums(l))) HIPCHK(expand_sums(l));
+            const bool chain = st.sums != 0;
+            const bool head = sums_on && !chain && takes_sums(l + 1) && takes_sums(l + 2);
+            if (chain) {
+                // While the counts still move a launch holds the layers that take about as long as the host's look at
+                // them (an estimate: a read of four rows takes a CU's LDS 20 cycles for 64 groups).
+                const double us = 1.0 + (double)n->carried * st.sums * 32.0 * 0.08 / ((double)n->n_cu * 2400.0);
+                int kmax = n->persist_layers;
+                if (opt.prune) kmax = std::min(kmax, std::max(st.c_prune, (int)(25.0 / us)));
+                kmax = std::max(1, std::min(kmax, last - l + 1));
+                while (c < kmax && takes_sums(l + c)) ++c;
+            }
+            if (!fb && !chain && !head && persist_on && n->resident_mode && n->d_table && (rsig = resident_sig(n, l)).ok) {
                 // Bringing the rows in and out costs such a launch as much as two layers save it with 16 rows per workgroup
                 // (64-byte pieces of a column) and as much as eight save it with 4 rows (16-byte pieces): measured
                 // at 2048 and at 60000 rows.  So left to the library: from 2 layers (even while the counts still move -
@@ -1932,13 +1977,13 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 const bool too_large = !persist_asked && rsig.ok == 2 && !wide_rows && n->carried >= n->tiled_min_rows;
                 if (k >= rmin && !too_large) { c = k; resident = true; }
             }
-            const bool pair = !fb && !resident && is_pair(l);
+            const bool pair = !fb && !resident && !chain && !head && is_pair(l);
             if (pair) c = 2;
             // a persistent launch: consecutive layers of one kernel form and variant
             LayerSig sig;
             if (fb) {
                 c = fb_c;
-            } else if (!pair && !resident && persist_on) {
+            } else if (!pair && !resident && !chain && !head && persist_on) {
                 sig = layer_sig(n, l, nblk);
                 const long long layer_bytes = 8ll * (long long)n->carried * (long long)n->N;
                 const bool small = layer_bytes >= n->persist_min_bytes && layer_bytes <= n->persist_max_bytes && nblk >= n->persist_min_blocks;
@@ -1965,7 +2010,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             State at_start{};
             if (persist) at_start = save();
             if (check_dead && (prev_stamp != 0 || c > 1)) n->blocks_skipped = true;
-            const bool group = persist || fb || resident;   // c layers whose rows are counted behind them, from the stamps
+            const bool group = persist || fb || resident || chain || head;   // c layers whose rows are counted behind them, from the stamps
             int32_t* const count_prev = (fused_count && st.count_pending && prev_stamp != 0 && !group) ? n->d_counts + (l - 1) : nullptr;
             const Feat in = n->cur;
             Feat out = (n->cur == n->A) ? n->C : n->A;
@@ -1974,7 +2019,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             int shape = -1, seglen = 0;
             bool trial = false;
             spdnn_net::Trial tr{};
-            if (c == 1 && p.kernel == SPDNN_KERNEL_BAND && !use_block_form(n, p, nblk)) {
+            if (c == 1 && !chain && !head && p.kernel == SPDNN_KERNEL_BAND && !use_block_form(n, p, nblk)) {
                 if (const spdnn_net::Tuned* t = find_tuned(n, nblk, p.kmax)) {
                     shape = t->shape;
                     seglen = t->seglen;
@@ -2030,6 +2075,25 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                             pl.xcd_queues, pl.light_sync);
                 for (int j = 1; j < c; ++j) out = (out == n->A) ? n->C : n->A;  // where the last layer wrote
                 st.r.persistent_launches += 1;
+            } else if (head) {
+                const DevLayer& d = n->dl[(size_t)l];
+                const bool alt = p.kernel == SPDNN_KERNEL_BAND;
+                BlockLaunch b{};
+                b.yin = in; b.yout = out; b.cols = alt ? d.alt_cols : d.blk_cols; b.cnt = alt ? d.alt_cnt : d.blk_cnt;
+                b.active = n->d_active; b.check_dead = check_dead; b.N = n->N; b.ngroups = sum_groups(p); b.nblk = nblk;
+                b.stamp = stamp0; b.prev_stamp = prev_stamp; b.rl = n->rl; b.wmode = 0; b.full = (alt ? p.alt_full : p.blk_full) ? 1 : 0;
+                b.wu = p.info.value; b.bias = n->bias; b.clampv = n->clampv; b.publish = st.pub;
+                HIPCHK(launch_sums_head(b, n->stream));
+                st.sums = b.ngroups;
+            } else if (chain) {
+                SumsLaunch sl{};
+                sl.table = n->d_table + l; sl.nlayers = c; sl.yin = in; sl.yout = out; sl.active = n->d_active; sl.ngroups = st.sums;
+                sl.rows = n->carried; sl.rl = n->rl; sl.stamp0 = stamp0; sl.prev_stamp = prev_stamp; sl.check_dead = check_dead;
+                sl.n_cu = n->n_cu; sl.bias = n->bias; sl.clampv = n->clampv; sl.publish = st.pub;
+                HIPCHK(launch_sums_resident(sl, n->stream));
+                if (n->run_verbose)
+                    fprintf(stderr, "spdnn: resident launch (group sums): layers %d..%d, %d rows, %d groups\n", l, l + c - 1, n->carried, st.sums);
+                st.r.resident_launches += 1;
             } else if (resident) {
                 ResidentLaunch rl{};
                 rl.table = n->d_table + l; rl.nlayers = c; rl.first_in = in; rl.buf_a = n->A; rl.buf_c = n->C; rl.active = n->d_active;
@@ -2176,7 +2240,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                         st.count_pending = false;
                     }
                     HIPCHK(launch_repack(n->cur, dstbuf, n->d_count, n->d_alive_src, n->d_alive_gid, n->d_gid_tmp,
-                                         n->N, n->rl, nb, n->stream));
+                                         st.sums ? st.sums : n->N, n->rl, nb, n->stream));
                     std::swap(n->d_gid, n->d_gid_tmp);
                     n->gid_dirty = true;
                     n->cur = dstbuf;
@@ -2187,6 +2251,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 }
             }
         }
+        if (failed < 0 && st.sums && !st.dead) HIPCHK(expand_sums(st.l));
         if (failed < 0) {
             // categories of the last layer: survivor list by the scan.  After a final repack the list
             // produced for the repack is that list already.

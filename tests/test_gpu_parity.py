@@ -1788,3 +1788,60 @@ def test_reference_side_binding(gc, orc, tmp_path):
         assert "layer %d, batch = %d" % (l, len(ref["active_ids"][l])) in r.stdout
     got = np.array([int(x.split()[1]) for x in r.stdout.splitlines() if x.startswith("category ")], dtype=np.int64)
     assert np.array_equal(got, ref["categories"])
+
+
+@pytest.mark.parametrize("N,B,kind,rl", [
+    (512, 300, "radix", 4),      # 32 groups: half a wave's lanes without one
+    (1008, 777, "radix", 2),     # 63 groups, rows one at a time
+    (1024, 17000, "radix", 4),   # four rows per workgroup
+    (1024, 9000, "hub", 4),      # two rows per workgroup; lists of fewer than 32 inputs
+    (4096, 700, "common", 4),    # one neuron order for all layers
+    (16400, 90, "radix", 1),     # 1025 groups: a second trip for one of them
+    (65520, 40, "hub", 4),       # 4095 groups and the zero behind them: the last 16-bit offset
+    (65536, 70, "radix", 4),     # 4096 groups
+])
+def test_group_sums(gc, orc, monkeypatch, N, B, kind, rl):
+    """Layers of equal groups behind one another carry one column per group between a head launch and an expansion:
+    counts, categories and activations against the oracle bit for bit, pruned and unpruned, whole and cut into calls, and
+    the same with the launches that carry full columns."""
+    print("group sums N=%d B=%d %s rl=%d" % (N, B, kind, rl), flush=True)
+    monkeypatch.setenv("SPDNN_ROWS_PER_LANE", str(rl))
+    rng = np.random.default_rng(N + B)
+    if kind == "hub":
+        base = [hub_block_csr(rng, N) for _ in range(2)]
+    else:
+        perm = rng.permutation(N) if kind == "common" else None
+        base = [radix_like_csr(rng, N, 16 << k, perm=perm) for k in range(2 if N > 20000 else 4)]
+    L = 7
+    layers = [base[l % len(base)] for l in range(L)]
+    dens = np.where(rng.random(B) < 0.3, 0.7, 0.08).astype(np.float32)
+    feats = (rng.random((B, N), dtype=np.float32) < dens[:, None]).astype(np.float32)
+    bias = -0.3 if N <= 1024 else -0.35 if N <= 4096 else -0.4
+    ref = orc.infer(feats, layers, bias, prune=True, keep=set(range(L)))
+    want = [len(a) for a in ref["active_ids"]]
+    assert 0 < want[-1] < B
+    cats = ref["categories"]
+    for mode in ("1", "0"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", mode)
+        with gc.Network(N, B, L, bias=bias) as net:
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            net.inspect()
+            net.set_features_dense(feats)
+            for prune in (True, False):
+                r = net.run(prune=prune, collect_counts=True)
+                if mode == "1":
+                    assert r.resident_launches >= 1 and r.persistent_launches == 0 and r.fused_pairs == 0
+                assert [net.active_count(l) for l in range(L)] == want
+                assert np.array_equal(net.categories(), cats)
+                assert same_floats(net.activations(cats), ref["y"])
+                dead = np.setdiff1d(np.arange(B), cats)[:64].astype(np.int32)
+                assert not net.activations(dead).any()
+            for cut in (3, 4):      # a call that ends in the middle leaves full columns behind, which the next one reads
+                net.run(prune=True, n_layers=cut)
+                gid, y = ref["kept"][cut - 1]
+                assert np.array_equal(net.categories(), gid)
+                assert same_floats(net.activations(gid), y)
+                net.run(prune=False, first_layer=cut)
+                assert np.array_equal(net.categories(), cats)
+                assert same_floats(net.activations(cats), ref["y"])
