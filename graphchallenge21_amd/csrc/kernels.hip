@@ -2813,11 +2813,12 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(
 }
 
 __global__ void unpack_rows_kernel(Feat y, const int32_t* __restrict__ phys_of_col,
-                                   const int32_t* __restrict__ phys_rows, int N, int RB,
+                                   const int32_t* __restrict__ row_ids, const int32_t* __restrict__ where, int N, int RB,
                                    const int32_t* __restrict__ active, int stamp, float* __restrict__ rowmajor) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    const int pr = phys_rows[blockIdx.y];
+    const int id = row_ids[blockIdx.y];
+    const int pr = where ? where[id] : id;
     float x = 0.0f;
     // a row that the last layer did not stamp is all zero by definition (its block may have been
     // skipped, leaving stale data in the buffer)
@@ -3626,12 +3627,18 @@ hipError_t launch_pack_rows(const float* rowmajor, const Feat& y, const int32_t*
     return hipGetLastError();
 }
 
-hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* phys_rows, int nreq,
+hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* row_ids, const int32_t* where, int nreq,
                               int N, int rl, const int32_t* active, int stamp, float* rowmajor, hipStream_t s) {
     if (nreq <= 0 || nreq > 65535 || N <= 0) return hipErrorInvalidValue;
     dim3 grid((N + 255) / 256, nreq);
-    hipLaunchKernelGGL(unpack_rows_kernel, grid, dim3(256), 0, s, y, phys_of_col, phys_rows, N, 64 * rl, active,
+    hipLaunchKernelGGL(unpack_rows_kernel, grid, dim3(256), 0, s, y, phys_of_col, row_ids, where, N, 64 * rl, active,
                        stamp, rowmajor);
+    return hipGetLastError();
+}
+
+hipError_t launch_fill_i32(int32_t* p, int n, int32_t v, hipStream_t s) {
+    if (n <= 0 || !p) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(fill_i32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
     return hipGetLastError();
 }
 

@@ -127,6 +127,7 @@ class JobPool {
         ++pending_;
         cv_job_.notify_one();
     }
+    int size() const { return (int)workers_.size(); }
     void wait_all() {
         std::unique_lock<std::mutex> lk(m_);
         cv_done_.wait(lk, [this] { return pending_ == 0; });
@@ -157,6 +158,70 @@ class JobPool {
     std::condition_variable cv_job_, cv_room_, cv_done_;
     size_t pending_ = 0;
     bool stop_ = false;
+};
+
+// Copies between a caller's memory and the pinned slots of a transfer that is cut into pieces: piece k in kParts parts,
+// the parts handed out in order (a ticket) to a few workers of the pool and to the calling thread while it waits.  The
+// caller opens the pieces one after the other (their slot may be read or written) and waits for piece k's copies.
+// One thread moves 21 GB/s between touched buffers and 5 GB/s into pages that do not exist yet - what a read-back
+// into a fresh array meets - against the 57 GB/s of the link.
+class CopyCrew {
+  public:
+    static constexpr int kParts = 8;
+    CopyCrew(JobPool* pool, int pieces, std::function<void(int, int)> copy)
+        : pieces_(pieces), copy_(std::move(copy)), done_(new std::atomic<int>[(size_t)pieces]) {
+        for (int k = 0; k < pieces; ++k) done_[(size_t)k].store(0, std::memory_order_relaxed);
+        if (pool) {
+            const int workers = std::min(kParts - 1, pool->size());
+            for (int w = 0; w < workers; ++w) {
+                { std::lock_guard<std::mutex> lk(m_); ++running_; }
+                pool->submit([this] {
+                    while (step(true)) {}
+                    std::lock_guard<std::mutex> lk(m_);
+                    if (--running_ == 0) cv_.notify_all();
+                });
+            }
+        }
+    }
+    // (every return path ends the workers before the buffers they copy go away)
+    ~CopyCrew() {
+        stop_.store(true, std::memory_order_release);
+        std::unique_lock<std::mutex> lk(m_);
+        cv_.wait(lk, [this] { return running_ == 0; });
+    }
+    CopyCrew(const CopyCrew&) = delete;
+    CopyCrew& operator=(const CopyCrew&) = delete;
+    void open(int k) { open_.store(k + 1, std::memory_order_release); }
+    void wait(int k) {
+        while (done_[(size_t)k].load(std::memory_order_acquire) < kParts)
+            if (!step(false)) std::this_thread::yield();
+    }
+
+  private:
+    // takes the next part and copies it.  block: waits for its piece to be opened; false: nothing (more) to take
+    bool step(bool block) {
+        for (unsigned spins = 0;; ++spins) {
+            if (stop_.load(std::memory_order_acquire)) return false;
+            int t = next_.load(std::memory_order_relaxed);
+            if (t >= pieces_ * kParts) return false;
+            if (t / kParts < open_.load(std::memory_order_acquire)) {
+                if (!next_.compare_exchange_weak(t, t + 1, std::memory_order_relaxed)) continue;
+                copy_(t / kParts, t % kParts);
+                done_[(size_t)(t / kParts)].fetch_add(1, std::memory_order_release);
+                return true;
+            }
+            if (!block) return false;
+            if ((spins & 63) == 63) std::this_thread::yield();
+        }
+    }
+    const int pieces_;
+    const std::function<void(int, int)> copy_;
+    std::unique_ptr<std::atomic<int>[]> done_;
+    std::atomic<int> next_{0}, open_{0};
+    std::atomic<bool> stop_{false};
+    std::mutex m_;
+    std::condition_variable cv_;
+    int running_ = 0;
 };
 
 int host_threads() {
@@ -248,6 +313,13 @@ struct spdnn_net {
     int32_t* d_counts = nullptr; // per-layer active-row counters (device)
     int32_t* h_counts = nullptr; // pinned mirror
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
+    // Transfers from and to a caller's memory (see ensure_staging): pinned slots, an event per slot, and the device copy of
+    // the rows that are packed at a time
+    unsigned char* h_stage = nullptr;
+    size_t stage_slot = 0;
+    hipEvent_t ev_stage[4] = {};
+    float* d_stage = nullptr;
+    size_t d_stage_bytes = 0;
     std::vector<hipEvent_t> ev_layer;
 
     // state
@@ -351,6 +423,16 @@ void release_device_base(spdnn_net* n) {
     n->ev_free.clear();
     n->exploring.clear();
     n->ev_layer.clear();
+    if (n->h_stage) hipHostFree(n->h_stage);
+    n->h_stage = nullptr;
+    n->stage_slot = 0;
+    hipFree(n->d_stage);
+    n->d_stage = nullptr;
+    n->d_stage_bytes = 0;
+    for (hipEvent_t& e : n->ev_stage) {
+        if (e) hipEventDestroy(e);
+        e = nullptr;
+    }
     if (n->ev_start) hipEventDestroy(n->ev_start);
     if (n->ev_stop) hipEventDestroy(n->ev_stop);
     if (n->stream) hipStreamDestroy(n->stream);
@@ -409,6 +491,31 @@ int ensure_device(spdnn_net* n) {
     if (rc != SPDNN_OK) release_device_base(n);  // nothing half-built stays behind (g_err is kept)
     return rc;
 }
+
+// Pinned slots for a transfer of `bytes` in units of `unit`: four of 8 MiB at most (or of one unit, where that is more),
+// kept with the network and grown when a larger transfer comes.  At 8 MiB a slot takes the link 0.15 ms, against which
+// the launch and the wait around it are small; small transfers keep small slots, because pinning costs 0.2 ms per MiB.
+constexpr int kStageSlots = 4;
+int ensure_staging(spdnn_net* n, size_t bytes, size_t unit) {
+    size_t slot = std::min<size_t>((size_t)8 << 20, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
+    slot = (std::max(slot, unit) + 4095) & ~(size_t)4095;
+    for (hipEvent_t& e : n->ev_stage)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (n->stage_slot >= slot) return SPDNN_OK;
+    if (n->h_stage) hipHostFree(n->h_stage);
+    n->h_stage = nullptr;
+    n->stage_slot = 0;
+    HIPCHK(hipHostMalloc((void**)&n->h_stage, slot * kStageSlots));
+    n->stage_slot = slot;
+    return SPDNN_OK;
+}
+// Part `part` of CopyCrew::kParts of a piece of `bytes`
+void copy_part(void* dst, const void* src, size_t bytes, int part) {
+    const size_t per = ((bytes + CopyCrew::kParts - 1) / CopyCrew::kParts + 4095) & ~(size_t)4095;
+    const size_t lo = std::min(bytes, per * (size_t)part), hi = std::min(bytes, lo + per);
+    if (hi > lo) memcpy((char*)dst + lo, (const char*)src + lo, hi - lo);
+}
+constexpr size_t kCrewMinBytes = (size_t)2 << 20;   // transfers below this are copied by the calling thread
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -1348,31 +1455,61 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
     int rc = begin_features(n, batch);
     if (rc) return rc;
     const int RB = n->RB, N = n->N;
-    // staging chunk: a whole number of row blocks, about 256 MiB
-    int64_t chunk_rows = std::max<int64_t>(RB, ((int64_t)(256 << 20) / ((int64_t)N * 4)) / RB * RB);
-    chunk_rows = std::min<int64_t>(chunk_rows, n->rows_cap);
-    DevTmp stage_buf;
-    HIPCHK(stage_buf.alloc((size_t)chunk_rows * N * 4));
-    float* stage = stage_buf.as<float>();
-    HIPCHK(hipMemsetAsync(n->d_nonfinite, 0, 8, n->stream));
+    // Rows are packed in chunks of whole row blocks, about 32 MiB, from a device copy of the chunk's rows; that copy is
+    // filled in pieces, each through a pinned slot.
+    const size_t row_bytes = (size_t)N * 4;
+    int64_t chunk_rows = std::max<int64_t>(RB, ((int64_t)(32 << 20) / (int64_t)row_bytes) / RB * RB);
     const int padded = ((batch + RB - 1) / RB) * RB;
-    for (int64_t r0 = 0; r0 < padded; r0 += chunk_rows) {
-        const int64_t rows_here = std::min<int64_t>(chunk_rows, padded - r0);
-        const int64_t real = std::max<int64_t>(0, std::min<int64_t>(rows_here, batch - r0));
-        if (real > 0)
-            HIPCHK(hipMemcpyAsync(stage, rowmajor + (size_t)r0 * N, (size_t)real * N * 4, hipMemcpyHostToDevice,
-                                  n->stream));
-        // rows >= real inside the chunk are written as zero by the kernel (nrows = real)
-        HIPCHK(launch_pack_rows(stage, n->F, n->d_lab, N, r0, (int)std::max<int64_t>(real, 1), n->rl,
-                                n->d_nonfinite, n->stream));
-        HIPCHK(hipStreamSynchronize(n->stream));  // the staging buffer is reused by the next chunk
+    chunk_rows = std::min<int64_t>(chunk_rows, padded);
+    const size_t chunk_bytes = (size_t)chunk_rows * row_bytes, total = (size_t)batch * row_bytes;
+    if (n->d_stage_bytes < chunk_bytes) {
+        hipFree(n->d_stage);
+        n->d_stage = nullptr;
+        n->d_stage_bytes = 0;
+        HIPCHK(dev_malloc(&n->d_stage, chunk_bytes));
+        n->d_stage_bytes = chunk_bytes;
+    }
+    rc = ensure_staging(n, total, 4096);
+    if (rc) return rc;
+    HIPCHK(launch_fill_i32(n->d_nonfinite, 2, 0, n->stream));
+    struct Piece { size_t at, bytes; bool last; };   // last: of its chunk
+    std::vector<Piece> pieces;
+    for (size_t c = 0; c < total; c += chunk_bytes) {
+        const size_t end = std::min(total, c + chunk_bytes);
+        for (size_t p = c; p < end; p += n->stage_slot) pieces.push_back({p, std::min(n->stage_slot, end - p), p + n->stage_slot >= end});
+    }
+    {
+        auto slot_at = [&](int k) { return n->h_stage + (size_t)(k % kStageSlots) * n->stage_slot; };
+        CopyCrew crew(total >= kCrewMinBytes ? n->pool.get() : nullptr, (int)pieces.size(), [&](int k, int part) {
+            copy_part(slot_at(k), (const char*)rowmajor + pieces[(size_t)k].at, pieces[(size_t)k].bytes, part);
+        });
+        const int K = (int)pieces.size();
+        for (int k = 0; k < std::min(K, kStageSlots); ++k) crew.open(k);
+        for (int k = 0; k < K; ++k) {
+            const Piece& p = pieces[(size_t)k];
+            crew.wait(k);
+            HIPCHK(hipMemcpyAsync((char*)n->d_stage + p.at % chunk_bytes, slot_at(k), p.bytes, hipMemcpyHostToDevice, n->stream));
+            HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
+            if (p.last) {
+                // rows behind the batch's last inside the chunk are written as zero by the kernel
+                const int64_t r0 = (int64_t)(p.at / chunk_bytes) * chunk_rows;
+                HIPCHK(launch_pack_rows(n->d_stage, n->F, n->d_lab, N, r0, (int)std::min<int64_t>(chunk_rows, batch - r0), n->rl,
+                                        n->d_nonfinite, n->stream));
+            }
+            // the slot after the newest one: free once its transfer has ended
+            if (k >= 1 && k - 1 + kStageSlots < K) {
+                HIPCHK(hipEventSynchronize(n->ev_stage[(k - 1) % kStageSlots]));
+                crew.open(k - 1 + kStageSlots);
+            }
+        }
     }
     int32_t bad[2] = {0, 0};
-    HIPCHK(hipMemcpy(bad, n->d_nonfinite, 8, hipMemcpyDeviceToHost));
-    if (bad[0]) return fail(SPDNN_E_ARG, "features contain NaN, infinity or values above 2^100 in magnitude");
-    if (bad[1]) return fail(SPDNN_E_ARG, "features contain nonzero values below 2^-100 in magnitude");
+    HIPCHK(hipMemcpyAsync(n->h_stage, n->d_nonfinite, 8, hipMemcpyDeviceToHost, n->stream));
     HIPCHK(launch_iota_gid(n->d_gid, n->rows_cap, batch, n->stream));
     HIPCHK(hipStreamSynchronize(n->stream));
+    memcpy(bad, n->h_stage, 8);
+    if (bad[0]) return fail(SPDNN_E_ARG, "features contain NaN, infinity or values above 2^100 in magnitude");
+    if (bad[1]) return fail(SPDNN_E_ARG, "features contain nonzero values below 2^-100 in magnitude");
     n->have_features = true;
     reset_state(n);
     return SPDNN_OK;
@@ -2351,32 +2488,52 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     if (!n->have_features) return fail(SPDNN_E_STATE, "no features set");
     if (nrows < 0) return fail(SPDNN_E_ARG, "nrows negative");
     if (nrows == 0) return SPDNN_OK;
-    // global id -> physical row of the current buffer
-    std::vector<int32_t> gid((size_t)std::max(n->carried, 1));
-    if (n->carried > 0) HIPCHK(hipMemcpy(gid.data(), n->d_gid, (size_t)n->carried * 4, hipMemcpyDeviceToHost));
-    std::vector<int32_t> where((size_t)n->batch, -1);
-    for (int r = 0; r < n->carried; ++r)
-        if (gid[(size_t)r] >= 0 && gid[(size_t)r] < n->batch) where[(size_t)gid[(size_t)r]] = r;
-    std::vector<int32_t> phys((size_t)nrows);
-    for (int i = 0; i < nrows; ++i) {
+    for (int i = 0; i < nrows; ++i)
         if (rows[i] < 0 || rows[i] >= n->batch) return fail(SPDNN_E_ARG, "row id out of range");
-        phys[(size_t)i] = where[(size_t)rows[i]];
+    // The rows go through pinned slots: a kernel finds a slot's rows and writes them into it (over the link: as fast as a
+    // copy command, and no copy in device memory in between), the host copies them out while the next slots are filled.
+    const size_t row_bytes = (size_t)n->N * 4, id_bytes = (size_t)nrows * 4;
+    int rc = ensure_staging(n, (size_t)nrows * row_bytes, row_bytes);
+    if (rc) return rc;
+    const int per = (int)std::min<size_t>(65535, n->stage_slot / row_bytes);   // rows per slot
+    DevTmp table;   // global id -> physical row of the current buffer, and the ids asked for
+    HIPCHK(table.alloc((size_t)n->batch * 4 + id_bytes));
+    int32_t* const d_where = table.as<int32_t>();
+    int32_t* const d_ids = d_where + n->batch;
+    HIPCHK(launch_row_table(n->d_gid, n->carried, n->batch, d_where, n->stream));
+    const void* ids_from = rows;
+    if (id_bytes <= n->stage_slot) {   // (from pinned memory where they fit the last slot, whose rows come behind this copy)
+        unsigned char* const last_slot = n->h_stage + (size_t)(kStageSlots - 1) * n->stage_slot;
+        memcpy(last_slot, rows, id_bytes);
+        ids_from = last_slot;
     }
-    const int chunk = 4096;
-    DevTmp phys_buf, out_buf;
-    HIPCHK(phys_buf.alloc((size_t)chunk * 4));
-    if (out_buf.alloc((size_t)chunk * (size_t)n->N * 4) != hipSuccess) return fail(SPDNN_E_NOMEM, "out of device memory");
-    int32_t* d_phys = phys_buf.as<int32_t>();
-    float* d_out = out_buf.as<float>();
+    HIPCHK(hipMemcpyAsync(d_ids, ids_from, id_bytes, hipMemcpyHostToDevice, n->stream));
     const int32_t* lab = nullptr;
     HIPCHK(labelling_dev(n, n->cur_layer, &lab));
-    for (int i0 = 0; i0 < nrows; i0 += chunk) {
-        const int m = std::min(chunk, nrows - i0);
-        HIPCHK(hipMemcpyAsync(d_phys, phys.data() + i0, (size_t)m * 4, hipMemcpyHostToDevice, n->stream));
-        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys, m, n->N, n->rl, n->d_active, n->last_stamp, d_out, n->stream));
-        HIPCHK(hipMemcpyAsync(rowmajor + (size_t)i0 * n->N, d_out, (size_t)m * n->N * 4, hipMemcpyDeviceToHost, n->stream));
-        HIPCHK(hipStreamSynchronize(n->stream));
+    const int K = (nrows + per - 1) / per;
+    auto slot_at = [&](int k) { return n->h_stage + (size_t)(k % kStageSlots) * n->stage_slot; };
+    auto rows_in = [&](int k) { return std::min(per, nrows - k * per); };
+    CopyCrew crew((size_t)nrows * row_bytes >= kCrewMinBytes ? n->pool.get() : nullptr, K, [&](int k, int part) {
+        copy_part(rowmajor + (size_t)k * per * n->N, slot_at(k), (size_t)rows_in(k) * row_bytes, part);
+    });
+    auto ready = [&](int k) -> hipError_t {   // slot k's rows have arrived: handed to the crew
+        const hipError_t e = hipEventSynchronize(n->ev_stage[k % kStageSlots]);
+        if (e == hipSuccess) crew.open(k);
+        return e;
+    };
+    int arrived = 0;
+    for (int k = 0; k < K; ++k) {
+        if (k >= kStageSlots) {
+            HIPCHK(ready(arrived++));
+            crew.wait(k - kStageSlots);
+        }
+        HIPCHK(launch_unpack_rows(n->cur, lab, d_ids + (size_t)k * per, d_where, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+                                  (float*)slot_at(k), n->stream));
+        HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
     }
+    while (arrived < K) HIPCHK(ready(arrived++));
+    crew.wait(K - 1);
+    for (int k = std::max(0, K - kStageSlots); k < K; ++k) crew.wait(k);
     return SPDNN_OK;
 }
 
@@ -2411,7 +2568,7 @@ static int spdnn_get_activations_noalloc_impl(spdnn_net* n, const int32_t* rows,
         const int m = std::min(chunk, nrows - i0);
         HIPCHK(hipMemcpyAsync(d_ids, rows + i0, (size_t)m * 4, hipMemcpyHostToDevice, n->stream));
         HIPCHK(launch_lookup_rows(d_ids, m, d_where, d_phys, n->stream));
-        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys, m, n->N, n->rl, n->d_active, n->last_stamp, d_out, n->stream));
+        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys, nullptr, m, n->N, n->rl, n->d_active, n->last_stamp, d_out, n->stream));
         HIPCHK(hipMemcpyAsync(rowmajor + (size_t)i0 * n->N, d_out, (size_t)m * row_bytes, hipMemcpyDeviceToHost, n->stream));
         HIPCHK(hipStreamSynchronize(n->stream));  // the staging rows are reused by the next pass
     }

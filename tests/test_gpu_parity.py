@@ -1845,3 +1845,31 @@ def test_group_sums(gc, orc, monkeypatch, N, B, kind, rl):
                 net.run(prune=False, first_layer=cut)
                 assert np.array_equal(net.categories(), cats)
                 assert same_floats(net.activations(cats), ref["y"])
+
+
+@pytest.mark.parametrize("N,B,asked", [
+    (1000, 3, 3),          # one small slot, copied by the calling thread
+    (1024, 700, 1300),     # past the size from which the copies are shared out
+    (3001, 4999, 4000),    # 60 MB: more pieces than slots, none of them whole rows on the way in
+    (65536, 300, 40),      # rows of 256 KiB: 32 to a slot
+])
+def test_transfers(gc, N, B, asked):
+    """Features handed over and rows read back through the pinned slots come out as they went in, in any order of rows and
+    asked for more than once; a row number out of range is refused."""
+    print("transfers N=%d B=%d" % (N, B), flush=True)
+    rng = np.random.default_rng(N + B)
+    rowptr, col = np.arange(N + 1, dtype=np.int32), rng.permutation(N).astype(np.int32)
+    with gc.Network(N, B, 1, bias=-0.3) as net:
+        net.set_layer_csr(0, rowptr, col, np.ones(N, np.float32))
+        net.inspect()
+        for _ in range(2):     # the second time through slots that are there
+            feats = rng.random((B, N), dtype=np.float32)
+            net.set_features_dense(feats)
+            rows = rng.integers(0, B, size=asked).astype(np.int32)
+            assert same_floats(net.activations(rows), feats[rows])
+        assert same_floats(net.activations(rows[:1]), feats[rows[:1]])
+        with pytest.raises(gc.SpdnnError):
+            net.activations(np.array([0, B], np.int32))
+        feats[B - 1, N - 1] = np.nan
+        with pytest.raises(gc.SpdnnError):
+            net.set_features_dense(feats)
