@@ -167,7 +167,7 @@ class JobPool {
 // into a fresh array meets - against the 57 GB/s of the link.
 class CopyCrew {
   public:
-    static constexpr int kParts = 8;
+    static constexpr int kParts = 16;
     CopyCrew(JobPool* pool, int pieces, std::function<void(int, int)> copy)
         : pieces_(pieces), copy_(std::move(copy)), done_(new std::atomic<int>[(size_t)pieces]) {
         for (int k = 0; k < pieces; ++k) done_[(size_t)k].store(0, std::memory_order_relaxed);
@@ -320,6 +320,8 @@ struct spdnn_net {
     hipEvent_t ev_stage[4] = {};
     float* d_stage = nullptr;
     size_t d_stage_bytes = 0;
+    int32_t* d_rowtab = nullptr;      // see spdnn_get_activations
+    size_t rowtab_bytes = 0;
     std::vector<hipEvent_t> ev_layer;
 
     // state
@@ -429,6 +431,9 @@ void release_device_base(spdnn_net* n) {
     hipFree(n->d_stage);
     n->d_stage = nullptr;
     n->d_stage_bytes = 0;
+    hipFree(n->d_rowtab);
+    n->d_rowtab = nullptr;
+    n->rowtab_bytes = 0;
     for (hipEvent_t& e : n->ev_stage) {
         if (e) hipEventDestroy(e);
         e = nullptr;
@@ -492,12 +497,13 @@ int ensure_device(spdnn_net* n) {
     return rc;
 }
 
-// Pinned slots for a transfer of `bytes` in units of `unit`: four of 8 MiB at most (or of one unit, where that is more),
-// kept with the network and grown when a larger transfer comes.  At 8 MiB a slot takes the link 0.15 ms, against which
-// the launch and the wait around it are small; small transfers keep small slots, because pinning costs 0.2 ms per MiB.
+// Pinned slots for a transfer of `bytes` in units of `unit`: four of 16 MiB at most (or of one unit, where that is more),
+// kept with the network and grown when a larger transfer comes.  At 16 MiB a slot takes the link 0.3 ms, against which
+// the launch and the waits around it are small (590 MB read back in 12.2 ms; with slots of 8 MiB 13.6); small transfers
+// keep small slots, because pinning costs 0.2 ms per MiB.
 constexpr int kStageSlots = 4;
 int ensure_staging(spdnn_net* n, size_t bytes, size_t unit) {
-    size_t slot = std::min<size_t>((size_t)8 << 20, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
+    size_t slot = std::min<size_t>((size_t)16 << 20, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
     slot = (std::max(slot, unit) + 4095) & ~(size_t)4095;
     for (hipEvent_t& e : n->ev_stage)
         if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1445,6 +1451,11 @@ static int begin_features(spdnn_net* n, int batch) {
     if (!n->inspected) return fail(SPDNN_E_STATE, "spdnn_inspect has not been called (or a layer changed since)");
     int rc = ensure_uploaded(n);
     if (rc) return rc;
+    if (n->batch != batch) {
+        hipFree(n->d_rowtab);
+        n->d_rowtab = nullptr;
+        n->rowtab_bytes = 0;
+    }
     n->batch = batch;
     n->have_features = false;
     return SPDNN_OK;
@@ -2496,9 +2507,17 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     int rc = ensure_staging(n, (size_t)nrows * row_bytes, row_bytes);
     if (rc) return rc;
     const int per = (int)std::min<size_t>(65535, n->stage_slot / row_bytes);   // rows per slot
-    DevTmp table;   // global id -> physical row of the current buffer, and the ids asked for
-    HIPCHK(table.alloc((size_t)n->batch * 4 + id_bytes));
-    int32_t* const d_where = table.as<int32_t>();
+    // global id -> physical row of the current buffer, and the ids asked for: kept until another batch size comes (an
+    // allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
+    const size_t table_bytes = (size_t)n->batch * 4 + id_bytes;
+    if (n->rowtab_bytes < table_bytes) {
+        hipFree(n->d_rowtab);
+        n->d_rowtab = nullptr;
+        n->rowtab_bytes = 0;
+        HIPCHK(dev_malloc(&n->d_rowtab, table_bytes));
+        n->rowtab_bytes = table_bytes;
+    }
+    int32_t* const d_where = n->d_rowtab;
     int32_t* const d_ids = d_where + n->batch;
     HIPCHK(launch_row_table(n->d_gid, n->carried, n->batch, d_where, n->stream));
     const void* ids_from = rows;
