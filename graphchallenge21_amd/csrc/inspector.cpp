@@ -676,6 +676,52 @@ static void build_quad_form(int N, const std::vector<int32_t>& rowptr, const std
     }
 }
 
+// The TILE form of a BAND layer under one exact weight (see LayerPlan::tile_rec).  Left empty when some sixteen outputs
+// merge to more than 48 steps.
+static void build_tile_form(int N, const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col, float value,
+                            LayerPlan& plan) {
+    static_assert(kQuadMaxNeurons <= 1024, "a tile's inputs are a set of 1024 bits");
+    const int nt = N / 16;
+    uint32_t wbits;
+    memcpy(&wbits, &value, 4);
+    std::vector<uint32_t> recs((size_t)nt * 96, 0u);
+    int steps = 0;
+    for (int c = 0; c < nt; ++c) {
+        uint64_t set[16] = {};      // the inputs of the tile's outputs; an input's step is its rank in the set
+        int before[16];
+        for (int j = 0; j < 16; ++j) {
+            const int row = plan.out_at[(size_t)16 * c + j];
+            for (int e = rowptr[row]; e < rowptr[row + 1]; ++e) set[col[e] >> 6] |= 1ull << (col[e] & 63);
+        }
+        int m = 0;
+        for (int w = 0; w < 16; ++w) {
+            before[w] = m;
+            m += __builtin_popcountll(set[w]);
+        }
+        if (m < 1 || m > 48) return;
+        steps = std::max(steps, m);
+        uint32_t* rec = &recs[(size_t)c * 96];
+        int s = 0;
+        for (int w = 0; w < 16; ++w)
+            for (uint64_t left = set[w]; left; left &= left - 1)
+                rec[s++] = (uint32_t)plan.in_pos[(size_t)(w * 64 + __builtin_ctzll(left))] * (uint32_t)kQuadColumnBytes;
+        for (; s < 48; ++s) rec[s] = rec[m - 1];
+        for (int j = 0; j < 16; ++j) {
+            const int row = plan.out_at[(size_t)16 * c + j];
+            uint64_t use = 0;
+            for (int e = rowptr[row]; e < rowptr[row + 1]; ++e) {
+                const int w = col[e] >> 6;
+                use |= 1ull << (before[w] + __builtin_popcountll(set[w] & ((1ull << (col[e] & 63)) - 1)));
+            }
+            rec[48 + j] = (uint32_t)use;
+            rec[64 + j] = (uint32_t)(use >> 32);
+            rec[80 + j] = wbits;
+        }
+    }
+    plan.tile_steps = (steps + 3) / 4 * 4;
+    plan.tile_rec.swap(recs);
+}
+
 void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col,
                    const std::vector<float>& val, int force_kernel, bool fma_ok, LayerPlan& plan,
                    const std::vector<int32_t>* common_pos) {
@@ -774,6 +820,8 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
     plan.quad_col.clear();
     plan.quad_w.clear();
     plan.quad_groups = 0;
+    plan.tile_rec.clear();
+    plan.tile_steps = 0;
     if (band && halo == 32 && uniform && exact) {
         // the BLOCK form of a run-chain layer, its columns in the band's input labelling
         plan.alt_ngroups = (int)groups.size();
@@ -871,6 +919,7 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
         plan.ell_col.clear();
         plan.rowlen.clear();
         if (N <= kQuadMaxNeurons) build_quad_form(N, rowptr, col, val, plan);
+        if (N <= kQuadMaxNeurons && (N % 64) == 0 && plan.wmode == 0) build_tile_form(N, rowptr, col, plan.info.value, plan);
     } else if (force_kernel != SPDNN_KERNEL_GATHER && !(getenv("SPDNN_TILED") && atoi(getenv("SPDNN_TILED")) == 0) &&
                build_tiled_plan(N, rowptr, col, val, plan)) {
         plan.kernel = SPDNN_KERNEL_TILED;
@@ -935,7 +984,7 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
     plan.info.block_form = plan.alt_ngroups > 0 ? 1 : (plan.alt_kmax > 0 ? 2 : 0);
     plan.info.plan_bytes = (int64_t)(4 * (plan.ell_col.size() + plan.rowlen.size() + plan.wv.size() +
                                                               plan.blk_cols.size() + plan.blk_cnt.size() + plan.pairs.size() +
-                                                              plan.alt_cols.size() + plan.alt_cnt.size() + plan.alt_out_at.size() + plan.alt_wv.size() + plan.rt_ent.size() + plan.quad_col.size() + plan.quad_w.size() +
+                                                              plan.alt_cols.size() + plan.alt_cnt.size() + plan.alt_out_at.size() + plan.alt_wv.size() + plan.rt_ent.size() + plan.quad_col.size() + plan.quad_w.size() + plan.tile_rec.size() +
                                                               plan.out_at.size() + (size_t)N));
     plan.dst.clear();
     plan.failed = false;

@@ -1872,6 +1872,7 @@ struct ResidentArgs {
     const float* quad_w;
     const int32_t* quad_dst;
     long long quad_stride;
+    const uint32_t* tile_rec;   // TILE form, at the same distances (ngroups: its steps)
 };
 
 // the value register k / R of the lane with row index k % R of this lane's group holds (k a constant after unrolling)
@@ -2617,6 +2618,144 @@ __global__ __launch_bounds__(1024) void band_resident_kernel(ResidentArgs a) {
     if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
 }
 
+// The resident launch of BAND layers under one exact weight, on the matrix cores.  A wave owns 64 neighbouring band
+// positions as four tiles of sixteen; v_mfma_f32_16x16x1_4b adds one step of all four tiles' merged lists to sixteen
+// rows: D[row][output] += x[row] * w[output], one rounding per product as in the multiply-add of the other kernels, and
+// a step an output does not use enters it with weight 0.  So the order of every sum stays ascending input index, and
+// the bits stay those of the oracle - which a form that adds several products in one instruction would not promise.
+// The lanes of tile b = lane / 16 read the step's column from LDS (sixteen rows, 64 bytes) and hold output lane % 16's
+// use mask; the steps' columns lie in three registers across the tile's lanes and enter the address add by DPP.
+// The rows stay in place: a wave's 64 x 16 results wait in its registers until every wave has read the layer's inputs,
+// so the buffer is N x 16 floats and two workgroups of 1024 threads share a CU (which is what limits a thread to 64
+// registers).  1024 neurons, 32 entries, 39700 rows: 62 us a layer against 68 of the QUAD form; the matrix cores are
+// busy 48 % of the cycles (48 instructions a tile and layer, a third of them on zeros), the LDS 38 %, over half of that
+// in bank conflicts of the steps' columns, the vector ALUs 35 %.  The frame around it - rows in and out, stamps, early
+// exit - is band_resident_kernel's.
+template <int NS>   // steps (a multiple of 4), 0: as the launch says
+__global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int sh_alive[3];
+    __shared__ int sh_last[16];
+    typedef float f32x16_t __attribute__((ext_vector_type(16)));
+    constexpr int R = 16, PARTS = 4;
+    using GU = const __attribute__((address_space(1))) uint32_t*;
+    using GB = const __attribute__((address_space(1))) unsigned char*;
+    publish_counts(a.pub);
+    const int t = (int)threadIdx.x, lane = t & 63, nthr = a.N;   // (launched with N threads)
+    const int RB = 64 * a.rl;
+    const unsigned nwg = gridDim.x;
+    const unsigned wg = (nwg % 8u) == 0u ? (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u : blockIdx.x;
+    const size_t row0 = (size_t)wg * R;
+    const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
+    if (a.check_dead && a.prev_stamp != 0) {   // a row block without an active row is skipped, as by the per-layer kernels
+        int alive = 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        if (__syncthreads_or(alive) == 0) return;
+    }
+    const size_t blkf = (size_t)a.N * RB;
+    {
+        const float* __restrict__ gin = block_base(a.first_in, rb, blkf) + rin;
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int idx = t + u * nthr;
+            v[u] = *reinterpret_cast<const float4*>(gin + (size_t)(idx / PARTS) * RB + (idx % PARTS) * 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<float4*>(smem + (size_t)(t + u * nthr) * 16) = v[u];
+    }
+    if (t < 3) sh_alive[t] = 0;
+    if (t < R) sh_last[t] = -1;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // this lane's words of its tile's record (requested a layer ahead), and the columns its four tiles' outputs go to
+    // (requested as their layer begins)
+    const uint32_t rec_off = ((uint32_t)(t >> 4) * 96u + (uint32_t)(lane & 15)) * 4u;
+    const uint32_t dst_off = ((uint32_t)wave * 64u + (uint32_t)(lane & 15)) * 4u;
+    uint32_t rec_next[6];
+    auto request = [&](int j) {
+        const GB rec = (GB)a.tile_rec + (long long)j * a.quad_stride;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) rec_next[i] = *(GU)(rec + i * 64 + rec_off);
+    };
+    request(0);
+    const int steps = NS ? NS : a.ngroups;
+    uint32_t last_nz = 0;   // per row of this lane, a byte: the last layer that left it nonzero, from 1 (64 layers at most)
+    bool all_dead = false;
+    ring_barrier<1>();
+    for (int j = 0; j < a.nlayers; ++j) {
+        const unsigned char* const in = smem + (lane & 15) * 4;
+        unsigned char* const out = smem + (lane >> 4) * 16;
+        uint32_t rec[5], dst[4];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) rec[i] = rec_next[i];
+        const uint32_t wbits = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec_next[5]);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) dst[b] = *(GU)((GB)a.quad_dst + (long long)j * a.quad_stride + b * 64 + dst_off);
+        if (j + 1 < a.nlayers) request(j + 1);   // in flight under this layer's arithmetic
+        f32x16_t acc = {};
+#pragma unroll
+        for (int s0 = 0; s0 < 48; s0 += 4) {
+            if (s0 < steps) {
+#pragma unroll
+                for (int s = s0; s < s0 + 4; ++s) {
+                    const float x = *reinterpret_cast<const float*>(in + row_lane(rec[s >> 4], s & 15));
+                    const uint32_t use = (uint32_t)((int32_t)(rec[3 + (s >> 5)] << (31 - (s & 31))) >> 31);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(x, __uint_as_float(use & wbits), acc, 0, 0, 0);
+                }
+            }
+        }
+        // register 4 b + q: row 4 (lane / 16) + q of output lane % 16 of tile b
+        float top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                acc[4 * b + q] = relu_clamp(acc[4 * b + q] + a.bias, a.clampv);
+                top[q] = nz_merge(top[q], acc[4 * b + q]);
+            }
+        }
+        float any = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (top[q] > 0.0f) last_nz = (last_nz & ~(255u << (8 * q))) | ((uint32_t)(j + 1) << (8 * q));
+            any = nz_merge(any, top[q]);
+        }
+        if (__ballot(any > 0.0f ? 1 : 0) != 0ull && lane == 0) sh_alive[j % 3] = 1;
+        ring_barrier<1>();   // all of the layer's inputs have been read
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            *reinterpret_cast<float4*>(out + dst[b] * (uint32_t)(R * 4)) = float4{acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]};
+        ring_barrier<1>();
+        const int some = sh_alive[j % 3];
+        if (t == 0) sh_alive[(j + 2) % 3] = 0;
+        if (some == 0 && a.bias <= 0.0f) { all_dead = true; break; }   // zero rows stay zero
+    }
+    // the last layer that left each of the 16 rows nonzero: the largest over the lanes that hold the row's outputs
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        int v = (int)((last_nz >> (8 * q)) & 255u) - 1;
+#pragma unroll
+        for (int sft = 1; sft < 16; sft <<= 1) v = max(v, __shfl_xor(v, sft, 64));
+        if ((lane & 15) == 0 && v >= 0) atomicMax(&sh_last[(lane >> 4) * 4 + q], v);
+    }
+    __syncthreads();
+    const int last_alive = t < R ? sh_last[t] : -1;
+    // the launch's last layer writes the work buffer the layer before it did not (layer 0: the one it did not read)
+    const bool in_a = a.first_in.half[0] == a.buf_a.half[0];
+    const bool to_c = in_a == ((a.nlayers & 1) != 0);
+    float* const o_h0 = to_c ? a.buf_c.half[0] : a.buf_a.half[0];
+    float* const o_h1 = to_c ? a.buf_c.half[1] : a.buf_a.half[1];
+    float* __restrict__ gout = ((rb & 1) ? o_h1 : o_h0) + (size_t)(rb >> 1) * blkf + rin;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int idx = t + u * nthr;
+        float4 v{};
+        if (!all_dead) v = *reinterpret_cast<const float4*>(smem + (size_t)idx * 16);
+        *reinterpret_cast<float4*>(gout + (size_t)(idx / PARTS) * RB + (idx % PARTS) * 4) = v;
+    }
+    if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
+}
+
 // counts[i] = rows whose stamp is at least stamp_lo + i (see launch_count_stamp_range).  Every workgroup takes a
 // share of the rows: a histogram in LDS (per wave one atomic per distinct value), sums from the top, and - where the
 // launch has several workgroups - the sums added to `partial` (n words, zero when the launch starts).  The workgroup
@@ -3303,6 +3442,30 @@ hipError_t launch_band_resident(const ResidentLaunch& a, int wmode, hipStream_t 
         if (a.ngroups == 9) SPDNN_BAND_RESIDENT(9, 2); else SPDNN_BAND_RESIDENT(0, 2);
     }
 #undef SPDNN_BAND_RESIDENT
+    return hipGetLastError();
+}
+
+hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s) {
+    // host-side shape checks: as launch_band_resident, and the waves' 64 band positions
+    if (a.nlayers < 1 || a.nlayers > 254 || !a.tile_rec || !a.quad_dst || (a.quad_stride % 4) != 0 || !a.first_in || !a.buf_a || !a.buf_c ||
+        a.buf_a == a.buf_c || !a.active || a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0 ||
+        band_resident_rows(a.N) != 16 || (a.N % 64) != 0 || a.ngroups < 4 || a.ngroups > 48 || (a.ngroups % 4) != 0)
+        return hipErrorInvalidValue;
+    ResidentArgs k{};
+    k.nlayers = a.nlayers; k.first_in = a.first_in; k.buf_a = a.buf_a; k.buf_c = a.buf_c; k.active = a.active;
+    k.N = a.N; k.ngroups = a.ngroups; k.rl = a.rl; k.stamp0 = a.stamp0; k.prev_stamp = a.prev_stamp; k.check_dead = a.check_dead;
+    k.bias = a.bias; k.clampv = a.clampv; k.pub = a.publish;
+    k.quad_dst = a.quad_dst; k.quad_stride = a.quad_stride; k.tile_rec = a.tile_rec;
+    dim3 grid((unsigned)(a.rows / 16)), block((unsigned)a.N);
+#define SPDNN_TILE_RESIDENT(NS)                                                                                            \
+    do {                                                                                                                   \
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(band_tile_resident_kernel<NS>),   \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);        \
+        if (attr != hipSuccess) return attr;                                                                               \
+        hipLaunchKernelGGL(band_tile_resident_kernel<NS>, grid, block, (size_t)a.N * 16 * 4, s, k);                        \
+    } while (0)
+    if (a.ngroups == 48) SPDNN_TILE_RESIDENT(48); else SPDNN_TILE_RESIDENT(0);
+#undef SPDNN_TILE_RESIDENT
     return hipGetLastError();
 }
 

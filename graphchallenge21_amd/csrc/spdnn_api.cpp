@@ -250,13 +250,14 @@ struct DevLayer {
     uint32_t* rt_ent = nullptr;    // (with alt_cnt / alt_dst: its ROWTILE form)
     uint32_t* quad_col = nullptr;  // the QUAD form of a BAND layer (with dst)
     float* quad_w = nullptr;
+    uint32_t* tile_rec = nullptr;  // the TILE form of a BAND layer (with dst)
     uint16_t* sum_cols = nullptr;  // inputs named by the groups of the layer before
 };
 
 // Where the arrays of one layer's plan lie inside its block of device memory (and inside the
 // pinned host copy of that block when plans are streamed): pairs, ell, rowlen, wv, dst, blk_cols,
-// blk_cnt, alt_cols, alt_cnt, alt_dst, alt_wv, rt_ent, quad_col, quad_w, sum_cols, each aligned to 256 bytes.
-constexpr int kPlanArrays = 15;
+// blk_cnt, alt_cols, alt_cnt, alt_dst, alt_wv, rt_ent, quad_col, quad_w, sum_cols, tile_rec, each aligned to 256 bytes.
+constexpr int kPlanArrays = 16;
 struct PlanLayout {
     size_t off[kPlanArrays] = {};
     size_t len[kPlanArrays] = {};
@@ -378,6 +379,7 @@ struct spdnn_net {
     int64_t tiled_min_rows = 8192;                    // see use_gather_form (SPDNN_TILED_MIN_ROWS)
     bool tiled_min_rows_given = false;                // ... set in the environment: also layers with a ROWTILE form follow it
     int rowtile_mode = 1;                             // TILED layers up to 8192 neurons wide run their ROWTILE form (SPDNN_ROWTILE=0: the tiles)
+    int tile_mode = 1;                                // BAND layers of one exact weight join resident launches in their TILE form (SPDNN_BAND_TILES=0: QUAD, 2: whatever the size)
     int sums_mode = 1;                                // layers of equal groups behind one another carry group sums (SPDNN_GROUP_SUMS=0: never)
     int band_resident_mode = 1;                       // BAND layers up to 1024 neurons wide join resident launches (SPDNN_BAND_RESIDENT=0: never)
     int band_resident_min_layers = 0;                 // ... of at least this many layers (SPDNN_BAND_RESIDENT_MIN_LAYERS; 0: 6, from 16384 rows up 16)
@@ -700,7 +702,8 @@ PlanLayout plan_layout(const LayerPlan& p) {
     const size_t len[kPlanArrays] = {p.pairs.size() * 4,    p.ell_col.size() * 4,  p.rowlen.size() * 4,   p.wv.size() * 4,
                                      p.dst.size() * 4,      p.blk_cols.size() * 4, p.blk_cnt.size() * 4,  p.alt_cols.size() * 4,
                                      p.alt_cnt.size() * 4,  p.alt_dst.size() * 4,  p.alt_wv.size() * 4,
-                                     p.rt_ent.size() * 4,   p.quad_col.size() * 4, p.quad_w.size() * 4,   p.sum_cols.size() * 2};
+                                     p.rt_ent.size() * 4,   p.quad_col.size() * 4, p.quad_w.size() * 4,   p.sum_cols.size() * 2,
+                                     p.tile_rec.size() * 4};
     for (int k = 0; k < kPlanArrays; ++k) {
         y.off[k] = y.bytes;
         y.len[k] = len[k];
@@ -712,7 +715,8 @@ PlanLayout plan_layout(const LayerPlan& p) {
 void pack_plan(const LayerPlan& p, const PlanLayout& y, char* dst) {
     const void* src[kPlanArrays] = {p.pairs.data(),   p.ell_col.data(),  p.rowlen.data(),  p.wv.data(),      p.dst.data(),
                                     p.blk_cols.data(), p.blk_cnt.data(), p.alt_cols.data(), p.alt_cnt.data(), p.alt_dst.data(),
-                                    p.alt_wv.data(),   p.rt_ent.data(),   p.quad_col.data(), p.quad_w.data(),   p.sum_cols.data()};
+                                    p.alt_wv.data(),   p.rt_ent.data(),   p.quad_col.data(), p.quad_w.data(),   p.sum_cols.data(),
+                                    p.tile_rec.data()};
     for (int k = 0; k < kPlanArrays; ++k)
         if (y.len[k]) memcpy(dst + y.off[k], src[k], y.len[k]);
 }
@@ -735,6 +739,7 @@ DevLayer plan_at(const PlanLayout& y, char* base) {
     d.quad_col = (uint32_t*)at(12);
     d.quad_w = (float*)at(13);
     d.sum_cols = (uint16_t*)at(14);
+    d.tile_rec = (uint32_t*)at(15);
     return d;
 }
 
@@ -1037,6 +1042,7 @@ static int spdnn_create_impl(int neuron, int max_batch, int layers, float bias, 
     if (const char* e = getenv("SPDNN_PERSIST_LIGHT_SYNC")) n->persist_light = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_SEGLEN")) n->persist_seglen = std::max(0, atoi(e));
     if (const char* e = getenv("SPDNN_RESIDENT")) n->resident_mode = atoi(e) != 0 ? 1 : 0;
+    if (const char* e = getenv("SPDNN_BAND_TILES")) n->tile_mode = std::min(2, std::max(0, atoi(e)));
     if (const char* e = getenv("SPDNN_GROUP_SUMS")) n->sums_mode = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_WAIT_US")) n->persist_wait_us = std::max(0ll, atoll(e));
     if (const char* e = getenv("SPDNN_BAND_SEGLEN")) n->band_seglen = std::max(0, atoi(e));
@@ -1834,7 +1840,7 @@ static LayerSig layer_sig(const spdnn_net* n, int l, int nblk) {
 // BLOCK form with one exact weight - a BLOCK layer of weight mode 0, or a run-chain BAND layer that carries its
 // BLOCK form - or the ROWTILE form of a TILED layer; and a shape the kernel's LDS buffers and numbering hold.
 struct ResidentSig {
-    int ok = 0;      // 0 no resident form; 1 BLOCK form of one exact weight; 2 ROWTILE form (TILED layers); 3 QUAD form (BAND layers)
+    int ok = 0;      // 0 no resident form; 1 BLOCK form of one exact weight; 2 ROWTILE form (TILED layers); 3 QUAD form (BAND layers), 4 TILE form (BAND layers of one exact weight)
     int full = 0, ngroups = 0, wmode = 0;
     int rows = 0;    // rows a workgroup keeps
     bool operator==(const ResidentSig& o) const { return ok == o.ok && full == o.full && ngroups == o.ngroups && wmode == o.wmode; }
@@ -1845,6 +1851,12 @@ static ResidentSig resident_sig(const spdnn_net* n, int l) {
     if (p.kernel == SPDNN_KERNEL_BAND && p.alt_ngroups > 0) { g.ok = 1; g.full = p.alt_full ? 1 : 0; g.ngroups = p.alt_ngroups; }
     else if (p.kernel == SPDNN_KERNEL_BLOCK && p.wmode == 0) { g.ok = 1; g.full = p.blk_full ? 1 : 0; g.ngroups = p.ngroups; }
     else if (p.kernel == SPDNN_KERNEL_TILED && !p.rt_ent.empty() && n->rowtile_mode) { g.ok = 2; g.wmode = p.wmode; }
+    // Band tiles need two workgroups on a CU to hide a layer's latency, and waves enough in each: 60 layers of 8, 20 and 32
+    // entries against QUAD, times faster: 1024 neurons, 60000 rows 1.05, 1.25, 1.05, 6000 rows 0.99, 1.19, 1.01, 700 rows
+    // 0.89, 1.11, 0.95; 768 neurons 1.18, 1.41, 1.08 and 1.09, 1.31, 1.01 and 0.90, 1.14, 0.92; 512 neurons 0.97, 1.14, 0.96
+    // and 0.86, 1.02, 0.80 and 1.05, 1.25, 0.84.  So: from 768 neurons and a workgroup of 16 rows for every CU.
+    else if (p.kernel == SPDNN_KERNEL_BAND && p.tile_steps > 0 && n->band_resident_mode &&
+             (n->tile_mode == 2 || (n->tile_mode == 1 && n->N >= 768 && n->carried >= 16 * n->n_cu))) { g.ok = 4; g.ngroups = p.tile_steps; }
     else if (p.kernel == SPDNN_KERNEL_BAND && p.quad_groups > 0 && n->band_resident_mode) { g.ok = 3; g.ngroups = p.quad_groups; g.wmode = p.wmode == 2 ? 2 : 1; }
     if (g.ok) {
         g.rows = g.ok == 1 ? resident_rows_per_workgroup(n->N, g.ngroups) : g.ok == 2 ? rowtile_resident_rows(n->N) : band_resident_rows(n->N);
@@ -1853,17 +1865,18 @@ static ResidentSig resident_sig(const spdnn_net* n, int l) {
     return g;
 }
 
-// The band resident kernel finds the QUAD form of its j-th layer j strides behind that of its first: whether layer k's
-// arrays lie where that rule, set by layers l0 and l0 + 1, puts them.
-static bool quad_plans_equidistant(const spdnn_net* n, int l0, int k) {
+// The band resident kernels find the QUAD or TILE form of their j-th layer j strides behind that of their first: whether
+// layer k's arrays lie where that rule, set by layers l0 and l0 + 1, puts them.
+static bool band_plans_equidistant(const spdnn_net* n, int l0, int k, bool tiles) {
     const DevLayer& a = n->dl[(size_t)l0];
     const DevLayer& b = n->dl[(size_t)l0 + 1];
     const DevLayer& c = n->dl[(size_t)k];
-    const long long stride = (const char*)b.quad_col - (const char*)a.quad_col;
+    const long long stride = (const char*)b.dst - (const char*)a.dst;
     const long long j = k - l0;
-    return (stride % 16) == 0 && (const char*)b.quad_w - (const char*)a.quad_w == stride && (const char*)b.dst - (const char*)a.dst == stride &&
-           (const char*)c.quad_col - (const char*)a.quad_col == j * stride && (const char*)c.quad_w - (const char*)a.quad_w == j * stride &&
-           (const char*)c.dst - (const char*)a.dst == j * stride;
+    if ((stride % 16) != 0 || (const char*)c.dst - (const char*)a.dst != j * stride) return false;
+    if (tiles) return (const char*)b.tile_rec - (const char*)a.tile_rec == stride && (const char*)c.tile_rec - (const char*)a.tile_rec == j * stride;
+    return (const char*)b.quad_col - (const char*)a.quad_col == stride && (const char*)b.quad_w - (const char*)a.quad_w == stride &&
+           (const char*)c.quad_col - (const char*)a.quad_col == j * stride && (const char*)c.quad_w - (const char*)a.quad_w == j * stride;
 }
 
 static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_run_result* res) {
@@ -2111,14 +2124,15 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // at 2048 and at 60000 rows.  So left to the library: from 2 layers (even while the counts still move -
                 // workgroups whose rows have all died leave early) and from 8; a caller that asks for launches of a
                 // given length gets them.
-                const bool wide_rows = rsig.rows >= 16 && rsig.ok != 3;
+                const bool wide_rows = rsig.rows >= 16 && rsig.ok < 3;
                 // (band quads: a layer inside the launch takes 0.88 of its time alone at 60000 rows, 0.76 at 6000, and rows in
                 // and out cost the launch what 1.5 layers take at either size: worth it from 16 and from 6 layers)
-                const int band_rmin = n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : (n->carried >= 16384 ? 16 : 6);
-                const int rmin = (persist_asked || wide_rows) ? 2 : rsig.ok == 3 ? band_rmin : 8;
+                // (band tiles: from 4; 120 layers that keep 40000 of 60000 rows take 8.4 ms with 3 or 4, 8.6 with 8, 8.7 with 16)
+                const int band_rmin = n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : rsig.ok == 4 ? 4 : (n->carried >= 16384 ? 16 : 6);
+                const int rmin = (persist_asked || wide_rows) ? 2 : rsig.ok >= 3 ? band_rmin : 8;
                 const int rmax = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
                 int k = 1;
-                while (k < rmax && resident_sig(n, l + k) == rsig && (rsig.ok != 3 || quad_plans_equidistant(n, l, l + k))) ++k;
+                while (k < rmax && resident_sig(n, l + k) == rsig && (rsig.ok < 3 || band_plans_equidistant(n, l, l + k, rsig.ok == 4))) ++k;
                 // (entry lists for 8 or 4 rows at a time: on large launches the per-layer kernel, which reads them for 16, is the
                 // faster one - measured per layer at batch 60000: N=2048 376 against 337 us, N=4096 1232 against 948; at 2048
                 // rows 13 against 38 and 42 against 57)
@@ -2248,16 +2262,18 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 rl.N = n->N; rl.ngroups = rsig.ngroups; rl.rows = n->carried; rl.rl = n->rl; rl.full = rsig.full;
                 rl.stamp0 = stamp0; rl.prev_stamp = prev_stamp; rl.check_dead = check_dead; rl.bias = n->bias; rl.clampv = n->clampv;
                 rl.publish = st.pub;
-                if (rsig.ok == 3) {
+                if (rsig.ok >= 3) {
                     const DevLayer& d0 = n->dl[(size_t)l];
+                    rl.tile_rec = d0.tile_rec;
                     rl.quad_col = d0.quad_col; rl.quad_w = d0.quad_w; rl.quad_dst = d0.dst;
-                    rl.quad_stride = c > 1 ? (long long)((const char*)n->dl[(size_t)l + 1].quad_col - (const char*)d0.quad_col) : 0;
+                    rl.quad_stride = c > 1 ? (long long)((const char*)n->dl[(size_t)l + 1].dst - (const char*)d0.dst) : 0;
                 }
                 HIPCHK(rsig.ok == 1 ? launch_block_resident(rl, n->stream)
-                       : rsig.ok == 2 ? launch_rowtile_resident(rl, rsig.wmode, n->stream) : launch_band_resident(rl, rsig.wmode, n->stream));
+                       : rsig.ok == 2 ? launch_rowtile_resident(rl, rsig.wmode, n->stream)
+                       : rsig.ok == 3 ? launch_band_resident(rl, rsig.wmode, n->stream) : launch_band_tile_resident(rl, n->stream));
                 if (n->run_verbose)
                     fprintf(stderr, "spdnn: resident launch (%s): layers %d..%d, %d rows, %d rows per workgroup\n",
-                            rsig.ok == 1 ? "groups" : rsig.ok == 2 ? "entry lists" : "band quads", l, l + c - 1, n->carried, rsig.rows);
+                            rsig.ok == 1 ? "groups" : rsig.ok == 2 ? "entry lists" : rsig.ok == 3 ? "band quads" : "band tiles", l, l + c - 1, n->carried, rsig.rows);
                 for (int j = 1; j < c; ++j) out = (out == n->A) ? n->C : n->A;  // where the last layer wrote
                 st.r.resident_launches += 1;
             } else if (fb) {

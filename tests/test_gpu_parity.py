@@ -1873,3 +1873,11 @@ def test_transfers(gc, N, B, asked):
         feats[B - 1, N - 1] = np.nan
         with pytest.raises(gc.SpdnnError):
             net.set_features_dense(feats)
+
+
+@pytest.mark.parametrize("N,B,K,rl", [(1024, 1500, 32, 4), (512, 900, 16, 2), (256, 300, 8, 1), (768, 400, 12, 4), (1024, 700, 20, 4)])
+def test_resident_launches_in_tiles(gc, orc, monkeypatch, N, B, K, rl):
+    """Bands under one power-of-two weight run their resident launches on the matrix cores (lists of 48 steps and of fewer):
+    the same checks as for bands of any weights."""
+    monkeypatch.setenv("SPDNN_BAND_TILES", "2")
+    test_resident_launches_of_band_layers(gc, orc, monkeypatch, N, B, K, "uniform", rl)
