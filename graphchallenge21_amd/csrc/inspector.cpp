@@ -810,6 +810,7 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
     plan.blk_cnt.clear();
     plan.alt_ngroups = 0;
     plan.alt_full = false;
+    plan.alt_walk = false;
     plan.alt_cols.clear();
     plan.alt_cnt.clear();
     plan.alt_out_at.clear();
@@ -824,6 +825,27 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
     plan.tile_steps = 0;
     if (band && halo == 32 && uniform && exact) {
         // the BLOCK form of a run-chain layer, its columns in the band's input labelling
+        // in the order of the band where every group is one of its tiles
+        const int nt = N / 16;
+        std::vector<int32_t> pos((size_t)N);
+        for (int v = 0; v < N; ++v) pos[(size_t)plan.out_at[(size_t)v]] = v;
+        std::vector<int> at((size_t)nt, -1);
+        bool walk = (N % 64) == 0 && (int)groups.size() == nt;
+        for (int g = 0; walk && g < nt; ++g) {
+            const std::vector<int32_t>& outs = groups[(size_t)g];
+            const int t = pos[(size_t)outs[0]] / 16;
+            walk = outs.size() == 16 && at[(size_t)t] < 0 && rowptr[outs[0] + 1] - rowptr[outs[0]] == 32;
+            for (size_t o = 0; walk && o < outs.size(); ++o) walk = pos[(size_t)outs[o]] / 16 == t;
+            for (int e = rowptr[outs[0]]; walk && e < rowptr[outs[0] + 1]; ++e)
+                walk = (plan.in_pos[(size_t)col[e]] - 16 * t + 32 + N) % N < 48;
+            at[(size_t)t] = g;
+        }
+        if (walk) {
+            std::vector<std::vector<int32_t>> ordered((size_t)nt);
+            for (int t = 0; t < nt; ++t) ordered[(size_t)t].swap(groups[(size_t)at[(size_t)t]]);
+            groups.swap(ordered);
+        }
+        plan.alt_walk = walk;
         plan.alt_ngroups = (int)groups.size();
         plan.alt_full = true;
         plan.alt_cols.assign((size_t)plan.alt_ngroups * 32, 0);

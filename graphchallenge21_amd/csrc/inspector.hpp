@@ -53,6 +53,9 @@ struct LayerPlan {
     // caches the BLOCK kernel is the faster of the two.
     int alt_ngroups = 0;
     bool alt_full = false;
+    // ... group g's outputs lie at band positions 16 g .. 16 g + 15 and its inputs in the 48 up to there (mod N), all lists 32
+    // long and N a multiple of 64: the groups can be walked with each input column read once (see launch_sums_head)
+    bool alt_walk = false;
     std::vector<int32_t> alt_cols;   // [alt_ngroups][32] physical input columns, accumulation order
     std::vector<int32_t> alt_cnt;    // [alt_ngroups]
     std::vector<int32_t> alt_out_at; // [alt_ngroups*16] output neuron of the slot, -1 = unused

@@ -145,6 +145,7 @@ struct BlockLaunch {
     int32_t* count_prev;     // as in BandLaunch
     int N, ngroups, nblk, stamp, prev_stamp, check_dead, rl, wmode;
     int full;                // 1: every group has exactly 32 shared inputs
+    int walk = 0;            // launch_sums_head: the groups are the tiles of a run-chain band (LayerPlan::alt_walk)
     float wu, bias, clampv;
     const int32_t* frontier = nullptr;   // as in BandLaunch
     int frontier_layer = 0;

@@ -2244,6 +2244,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 b.yin = in; b.yout = out; b.cols = alt ? d.alt_cols : d.blk_cols; b.cnt = alt ? d.alt_cnt : d.blk_cnt;
                 b.active = n->d_active; b.check_dead = check_dead; b.N = n->N; b.ngroups = sum_groups(p); b.nblk = nblk;
                 b.stamp = stamp0; b.prev_stamp = prev_stamp; b.rl = n->rl; b.wmode = 0; b.full = (alt ? p.alt_full : p.blk_full) ? 1 : 0;
+                b.walk = alt && p.alt_walk ? 1 : 0;
                 b.wu = p.info.value; b.bias = n->bias; b.clampv = n->clampv; b.publish = st.pub;
                 HIPCHK(launch_sums_head(b, n->stream));
                 st.sums = b.ngroups;

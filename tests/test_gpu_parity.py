@@ -1796,6 +1796,8 @@ def test_reference_side_binding(gc, orc, tmp_path):
     (1024, 17000, "radix", 4),   # four rows per workgroup
     (1024, 9000, "hub", 4),      # two rows per workgroup; lists of fewer than 32 inputs
     (4096, 700, "common", 4),    # one neuron order for all layers
+    (4160, 130, "radix", 1),     # 260 groups, walked in segments of which the last is short
+    (8192, 300, "radix", 2),
     (16400, 90, "radix", 1),     # 1025 groups: a second trip for one of them
     (65520, 40, "hub", 4),       # 4095 groups and the zero behind them: the last 16-bit offset
     (65536, 70, "radix", 4),     # 4096 groups
