@@ -2507,7 +2507,15 @@ static int spdnn_get_categories_impl(spdnn_net* n, int32_t* ids, int64_t cap, in
     if (!ids || n->alive == 0) return SPDNN_OK;
     if (cap < n->alive) return fail(SPDNN_E_ARG, "ids buffer too small");
     if (!n->alive_list_valid) return fail(SPDNN_E_STATE, "no active list available");
-    HIPCHK(hipMemcpy(ids, n->d_alive_gid, (size_t)n->alive * 4, hipMemcpyDeviceToHost));
+    const size_t bytes = (size_t)n->alive * 4;
+    if (int rc = ensure_staging(n, bytes, 4096)) return rc;
+    if (bytes > n->stage_slot * kStageSlots) {
+        HIPCHK(hipMemcpy(ids, n->d_alive_gid, bytes, hipMemcpyDeviceToHost));
+        return SPDNN_OK;
+    }
+    HIPCHK(hipMemcpyAsync(n->h_stage, n->d_alive_gid, bytes, hipMemcpyDeviceToHost, n->stream));
+    HIPCHK(hipStreamSynchronize(n->stream));
+    memcpy(ids, n->h_stage, bytes);
     return SPDNN_OK;
 }
 
