@@ -1857,6 +1857,11 @@ __global__ __launch_bounds__(256) void block_persist_kernel(PersistArgs a) {
 // weight, bias last.  One barrier per layer.  Rows are stamped with the last layer that left them
 // nonzero (the per-layer counts are taken from the stamps behind the launch); once all R rows are
 // zero and the bias is not positive the workgroup stops and stores zeros.
+//
+// A row block is skipped where no row carries the previous launch's stamp or a later one: a workgroup of the same
+// block may have finished before this one starts, and its rows then carry this launch's stamps.  (Looked at for the
+// previous stamp alone, the block seems dead to the late workgroup, which leaves its rows' older values in a buffer
+// that the block's next launch reads.)
 // ------------------------------------------------------------------------------------------
 struct ResidentArgs {
     const LayerDesc* table;
@@ -1913,7 +1918,7 @@ __global__ __launch_bounds__(1024) void block_resident_kernel(ResidentArgs a) {
     const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
     if (a.check_dead && a.prev_stamp != 0) {   // a row block without an active row is skipped, as by the per-layer kernels
         int alive = 0;
-        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] >= a.prev_stamp) ? 1 : 0;
         if (__syncthreads_or(alive) == 0) return;
     }
     const size_t blkf = (size_t)a.N * RB;
@@ -2203,11 +2208,11 @@ __global__ __launch_bounds__(1024) void sums_resident_kernel(SumsArgs a) {
     bool all_dead = false;
     if (a.check_dead && a.prev_stamp != 0) {
         int alive = 0;
-        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] >= a.prev_stamp) ? 1 : 0;
         if (__syncthreads_or(alive) == 0) return;   // a row block without an active row is skipped, as by the per-layer kernels
         int own = 0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) own |= (a.active[row0 + r] == a.prev_stamp) ? 1 : 0;
+        for (int r = 0; r < R; ++r) own |= (a.active[row0 + r] >= a.prev_stamp) ? 1 : 0;
         all_dead = __builtin_amdgcn_readfirstlane(own) == 0;   // (the same four words for every thread)
     }
     const uint32_t buf_bytes = (uint32_t)(G + 1) * R * 4;
@@ -2324,7 +2329,7 @@ __global__ __launch_bounds__(1024) void rowtile_resident_kernel(ResidentArgs a) 
     const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
     if (a.check_dead && a.prev_stamp != 0) {   // a row block without an active row is skipped, as by the per-layer kernels
         int alive = 0;
-        for (int i = t; i < RB; i += 1024) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        for (int i = t; i < RB; i += 1024) alive |= (a.active[(size_t)rb * RB + i] >= a.prev_stamp) ? 1 : 0;
         if (__syncthreads_or(alive) == 0) return;
     }
     const size_t blkf = (size_t)a.N * RB;
@@ -2535,7 +2540,7 @@ __global__ __launch_bounds__(1024) void band_resident_kernel(ResidentArgs a) {
     const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
     if (a.check_dead && a.prev_stamp != 0) {   // a row block without an active row is skipped, as by the per-layer kernels
         int alive = 0;
-        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] >= a.prev_stamp) ? 1 : 0;
         if (__syncthreads_or(alive) == 0) return;
     }
     const size_t blkf = (size_t)a.N * RB;
@@ -2715,7 +2720,7 @@ __global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArg
     const int rb = (int)(row0 / (size_t)RB), rin = (int)(row0 - (size_t)rb * RB);
     if (a.check_dead && a.prev_stamp != 0) {   // a row block without an active row is skipped, as by the per-layer kernels
         int alive = 0;
-        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] == a.prev_stamp) ? 1 : 0;
+        for (int i = t; i < RB; i += nthr) alive |= (a.active[(size_t)rb * RB + i] >= a.prev_stamp) ? 1 : 0;
         if (__syncthreads_or(alive) == 0) return;
     }
     const size_t blkf = (size_t)a.N * RB;

@@ -1883,3 +1883,35 @@ def test_resident_launches_in_tiles(gc, orc, monkeypatch, N, B, K, rl):
     the same checks as for bands of any weights."""
     monkeypatch.setenv("SPDNN_BAND_TILES", "2")
     test_resident_launches_of_band_layers(gc, orc, monkeypatch, N, B, K, "uniform", rl)
+
+
+@pytest.mark.parametrize("N,B,kind", [(1024, 60000, "radix"), (16384, 6000, "radix"), (1024, 60000, "band")])
+def test_resident_launches_with_one_survivor_per_row_block(gc, orc, monkeypatch, N, B, kind):
+    """One row of every 256 lives on, the others die layer by layer, and nothing is compacted: workgroups of a row block
+    whose survivor's workgroup has finished already still write their dead rows as zeros.  Against one launch per layer."""
+    print("one survivor per row block N=%d B=%d %s" % (N, B, kind), flush=True)
+    rng = np.random.default_rng(N)
+    L = 24
+    base = [radix_like_csr(rng, N, 16 << k) for k in range(3)] if kind == "radix" else [orc.gen_layer_csr(5, l, N) for l in range(3)]
+    lo, hi = (0.10, 0.27) if N <= 1024 else (0.20, 0.38)
+    dens = np.where(np.arange(B) % 256 == 0, 0.8, rng.uniform(lo, hi, size=B)).astype(np.float32)
+    feats = (rng.random((B, N), dtype=np.float32) < dens[:, None]).astype(np.float32)
+    for sums in ("1", "0"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", sums)
+        monkeypatch.setenv("SPDNN_BAND_TILES", "2" if sums == "1" else "0")
+        with gc.Network(N, B, L, bias=-0.3 if N <= 1024 else -0.4) as net:
+            for l in range(L):
+                net.set_layer_csr(l, *base[l % 3])
+            net.inspect()
+            net.set_features_dense(feats)
+            net.run(prune=True, collect_counts=True, fuse_layers=1, compact_threshold=1e-6)
+            want = [net.active_count(l) for l in range(L)]
+            cats = net.categories()
+            y = net.activations(cats)
+            assert (B + 255) // 256 <= want[-1] < B // 100 and len(set(want)) > 3
+            for fuse in (0, 2, 5):
+                r = net.run(prune=True, collect_counts=True, fuse_layers=fuse, compact_threshold=1e-6)
+                assert r.compactions == 0 and (r.resident_launches > 0 or N > 4096 or fuse < 5)
+                assert [net.active_count(l) for l in range(L)] == want
+                assert np.array_equal(net.categories(), cats)
+                assert same_floats(net.activations(cats), y)
