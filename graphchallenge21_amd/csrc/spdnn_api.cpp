@@ -175,11 +175,17 @@ class CopyCrew {
             const int workers = std::min(kParts - 1, pool->size());
             for (int w = 0; w < workers; ++w) {
                 { std::lock_guard<std::mutex> lk(m_); ++running_; }
-                pool->submit([this] {
-                    while (step(true)) {}
+                try {
+                    pool->submit([this] {
+                        while (step(true)) {}
+                        std::lock_guard<std::mutex> lk(m_);
+                        if (--running_ == 0) cv_.notify_all();
+                    });
+                } catch (...) {   // no memory for the job: the workers there are and the caller do it
                     std::lock_guard<std::mutex> lk(m_);
-                    if (--running_ == 0) cv_.notify_all();
-                });
+                    --running_;
+                    break;
+                }
             }
         }
     }
@@ -2110,11 +2116,13 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             const bool chain = st.sums != 0;
             const bool head = sums_on && !chain && takes_sums(l + 1) && takes_sums(l + 2);
             if (chain) {
-                // While the counts still move a launch holds the layers that take about as long as the host's look at
-                // them (an estimate: a read of four rows takes a CU's LDS 20 cycles for 64 groups).
+                // While the counts still move a launch holds about 120 us of layers (an estimate: a read of four rows takes
+                // a CU's LDS 20 cycles for 64 groups): counting, the host's look, scan and repack behind a launch take 50 to
+                // 70 us, and workgroups whose rows have died leave by themselves.  Layers of 60000 x 1024, 30000 x 4096 and
+                // 12000 x 16384 with 25 us of layers at first: 422, 730 and 864 us; with 60 410, 730, 870; with 120 347, 617, 800.
                 const double us = 1.0 + (double)n->carried * st.sums * 32.0 * 0.08 / ((double)n->n_cu * 2400.0);
                 int kmax = n->persist_layers;
-                if (opt.prune) kmax = std::min(kmax, std::max(st.c_prune, (int)(25.0 / us)));
+                if (opt.prune) kmax = std::min(kmax, std::max(st.c_prune, (int)(120.0 / us)));
                 kmax = std::max(1, std::min(kmax, last - l + 1));
                 while (c < kmax && takes_sums(l + c)) ++c;
             }
