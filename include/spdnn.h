@@ -98,6 +98,9 @@ typedef struct spdnn_run_options {
                                     at most 1024 neurons wide (from 6 layers on, from 16 at 16384 rows and more): a workgroup
                                     keeps 16, 8 or 4 rows in LDS through up to 64 layers (SPDNN_RESIDENT=0: never;
                                     SPDNN_BAND_RESIDENT=0: not the BAND layers);
+                                    three or more consecutive layers with such a BLOCK form, of any width up to 65536, carry
+                                    one column per group of equal outputs between a first launch that reads all columns and
+                                    an expansion at the end (SPDNN_GROUP_SUMS=0: not these);
                                   - pairs of layers the inspector marked fuse_next as one launch with the intermediate tile
                                     in LDS, on launches of 2^23 rows x neurons and more (SPDNN_PAIR_MIN_ELEMS);
                                   - persistent launches (up to 64 layers of one kernel form, a dependency per row block
