@@ -1971,17 +1971,27 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     State st{};
     st.l = first; st.dead = n->carried == 0; st.count_pending = false; st.last_launched = -1; st.newest_count = -1;
     st.c_prune = 1; st.pub = Publish{}; st.processed = 0; st.r = spdnn_run_result{}; st.sums = 0;
-    // group sums of layer l - 1 written out for whatever reads the full columns next
-    auto expand_sums = [&](int l) -> hipError_t {
-        const LayerPlan& p = n->layers[(size_t)l - 1];
-        const DevLayer& d = n->dl[(size_t)l - 1];
+    // the group sums that n->cur holds, written out for whatever reads the full columns next
+    auto expand_sums = [&]() -> hipError_t {
+        const LayerPlan& p = n->layers[(size_t)n->cur_layer - 1];
+        const DevLayer& d = n->dl[(size_t)n->cur_layer - 1];
         const Feat full = (n->cur == n->A) ? n->C : n->A;
         const hipError_t e = launch_sums_expand(n->cur, full, p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst, n->N, st.sums,
                                                 n->carried / n->RB, n->rl, n->stream);
-        n->cur = full;
-        st.sums = 0;
+        if (e == hipSuccess) {
+            n->cur = full;
+            st.sums = 0;
+        }
         return e;
     };
+    // A run that ends in an error behind such a launch leaves full columns behind, as one that ends elsewhere does: the
+    // state may be read, and a later run may continue it.  Where even that launch fails there is no state to speak of.
+    struct AtEnd {
+        std::function<void()> f;
+        ~AtEnd() { f(); }
+    } at_end{[&] {
+        if (st.sums != 0 && n->carried > 0 && expand_sums() != hipSuccess) n->have_features = false;
+    }};
     auto save = [&]() {
         State s = st;
         s.cur = n->cur; s.cur_layer = n->cur_layer; s.carried = n->carried; s.stamp = n->stamp; s.last_stamp = n->last_stamp;
@@ -2112,7 +2122,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             // layers at least, or the head and the expansion behind it cost more than they save.
             const bool sums_on = !fb && persist_on && !persist_asked && n->resident_mode && n->sums_mode && n->d_table;
             auto takes_sums = [&](int k) { return k <= last && !n->layers[(size_t)k].sum_cols.empty(); };
-            if (st.sums && !(sums_on && takes_sums(l))) HIPCHK(expand_sums(l));
+            if (st.sums && !(sums_on && takes_sums(l))) HIPCHK(expand_sums());
             const bool chain = st.sums != 0;
             const bool head = sums_on && !chain && takes_sums(l + 1) && takes_sums(l + 2);
             if (chain) {
@@ -2255,7 +2265,6 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 b.walk = alt && p.alt_walk ? 1 : 0;
                 b.wu = p.info.value; b.bias = n->bias; b.clampv = n->clampv; b.publish = st.pub;
                 HIPCHK(launch_sums_head(b, n->stream));
-                st.sums = b.ngroups;
             } else if (chain) {
                 SumsLaunch sl{};
                 sl.table = n->d_table + l; sl.nlayers = c; sl.yin = in; sl.yout = out; sl.active = n->d_active; sl.ngroups = st.sums;
@@ -2333,6 +2342,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             n->last_stamp = stamp0 + c - 1;
             n->cur = out;
             n->cur_layer = l + c;
+            if (head) st.sums = sum_groups(p);
             if (scan_count) {
                 HIPCHK(launch_scan_active(n->d_active, n->d_gid, n->carried, n->last_stamp, n->d_count, n->d_alive_src,
                                           n->d_alive_gid, n->stream));
@@ -2424,7 +2434,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 }
             }
         }
-        if (failed < 0 && st.sums && !st.dead) HIPCHK(expand_sums(st.l));
+        if (failed < 0 && st.sums && !st.dead) HIPCHK(expand_sums());
         if (failed < 0) {
             // categories of the last layer: survivor list by the scan.  After a final repack the list
             // produced for the repack is that list already.

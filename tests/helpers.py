@@ -110,3 +110,13 @@ def common_band_csr(rng, n, perm, values="uniform", k=32):
     else:
         val = rng.uniform(-0.05, 0.15, size=m).astype(np.float32)
     return rowptr, col, val
+
+
+def hold_device(seconds):
+    """Keeps what is queued from now on, on the null stream and on every stream that waits for it, from starting for that
+    long: a host function (libc's usleep) on the null stream.  The library's HIP runtime has to be loaded already."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipLaunchHostFunc.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    sleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p)
+    assert hip.hipLaunchHostFunc(None, sleep, ctypes.c_void_p(int(seconds * 1e6))) == 0

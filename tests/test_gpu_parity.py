@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from helpers import random_csr, same_floats, sort_rows
-from helpers import common_band_csr, hub_block_csr, radix_like_csr
+from helpers import common_band_csr, hold_device, hub_block_csr, radix_like_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -1915,3 +1915,39 @@ def test_resident_launches_with_one_survivor_per_row_block(gc, orc, monkeypatch,
                 assert [net.active_count(l) for l in range(L)] == want
                 assert np.array_equal(net.categories(), cats)
                 assert same_floats(net.activations(cats), y)
+
+
+@pytest.mark.parametrize("calls", [1, 2])
+def test_run_that_ends_in_an_error_inside_group_sums(gc, orc, monkeypatch, calls):
+    """The host gives up waiting for a layer's counts (the device is held back for longer than it waits) while the network
+    carries group sums.  What is read back and what is continued afterwards are full columns, as without group sums."""
+    print("error inside group sums, %d calls" % calls, flush=True)
+    N, B, L = 1024, 300, 8
+    rng = np.random.default_rng(5)
+    base = [radix_like_csr(rng, N, 16 << k) for k in range(3)]
+    layers = [base[l % 3] for l in range(L)]
+    dens = np.where(rng.random(B) < 0.4, 0.7, 0.1).astype(np.float32)
+    feats = (rng.random((B, N), dtype=np.float32) < dens[:, None]).astype(np.float32)
+    ref = orc.infer(feats, layers, -0.3, prune=True, keep=set(range(L)))
+    monkeypatch.setenv("SPDNN_COUNT_TIMEOUT_MS", "1")
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        done = 0
+        if calls == 2:      # the second call starts its own run of group sums
+            net.run(prune=True, n_layers=2)
+            done = 2
+        hold_device(0.5)
+        with pytest.raises(gc.SpdnnError) as e:
+            net.run(prune=True, first_layer=done)
+        assert "timed out" in e.value.message
+        done += 1           # the launch that the host gave up on was the first layer's
+        gid, y = ref["kept"][done - 1]
+        assert same_floats(net.activations(gid), y)
+        dead = np.setdiff1d(np.arange(B), gid).astype(np.int32)
+        assert not net.activations(dead).any()
+        net.run(prune=True, first_layer=done)
+        assert np.array_equal(net.categories(), ref["categories"])
+        assert same_floats(net.activations(ref["categories"]), ref["y"])
