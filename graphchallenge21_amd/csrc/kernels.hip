@@ -2750,7 +2750,7 @@ __global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArg
     };
     request(0);
     const int steps = NS ? NS : a.ngroups;
-    uint32_t last_nz = 0;   // per row of this lane, a byte: the last layer that left it nonzero, from 1 (64 layers at most)
+    uint32_t last_nz = 0;   // per row of this lane, a byte: the last layer that left it nonzero, from 1 (kTileMaxLayers at most)
     bool all_dead = false;
     ring_barrier<1>();
     for (int j = 0; j < a.nlayers; ++j) {
@@ -3518,7 +3518,7 @@ hipError_t launch_band_resident(const ResidentLaunch& a, int wmode, hipStream_t 
 
 hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s) {
     // host-side shape checks: as launch_band_resident, and the waves' 64 band positions
-    if (a.nlayers < 1 || a.nlayers > 254 || !a.tile_rec || !a.quad_dst || (a.quad_stride % 4) != 0 || !a.first_in || !a.buf_a || !a.buf_c ||
+    if (a.nlayers < 1 || a.nlayers > kTileMaxLayers || !a.tile_rec || !a.quad_dst || (a.quad_stride % 4) != 0 || !a.first_in || !a.buf_a || !a.buf_c ||
         a.buf_a == a.buf_c || !a.active || a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0 ||
         band_resident_rows(a.N) != 16 || (a.N % 64) != 0 || a.ngroups < 4 || a.ngroups > 48 || (a.ngroups % 4) != 0)
         return hipErrorInvalidValue;

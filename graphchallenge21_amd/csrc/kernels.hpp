@@ -302,7 +302,9 @@ int band_resident_rows(int N);
 // rows a workgroup keeps (16 or 4), 0 if the shape does not fit: two buffers of (N + 1) x R floats in LDS
 // (N <= 1024: 16 rows, N <= 4096: 4) and one (group, row) item per thread of 1024
 int resident_rows_per_workgroup(int N, int ngroups);
-// Their TILE form (one exact weight): sixteen outputs by sixteen rows on the matrix cores.
+// Their TILE form (one exact weight): sixteen outputs by sixteen rows on the matrix cores.  kTileMaxLayers layers per
+// launch at most: a byte per row holds the last layer that left it nonzero.
+constexpr int kTileMaxLayers = 254;
 hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s);
 hipError_t launch_block_resident(const ResidentLaunch& a, hipStream_t s);
 

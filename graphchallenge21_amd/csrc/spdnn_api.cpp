@@ -2148,7 +2148,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // (band tiles: from 4; 120 layers that keep 40000 of 60000 rows take 8.4 ms with 3 or 4, 8.6 with 8, 8.7 with 16)
                 const int band_rmin = n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : rsig.ok == 4 ? 4 : (n->carried >= 16384 ? 16 : 6);
                 const int rmin = (persist_asked || wide_rows) ? 2 : rsig.ok >= 3 ? band_rmin : 8;
-                const int rmax = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
+                int rmax = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
+                if (rsig.ok == 4) rmax = std::min(rmax, kTileMaxLayers);
                 int k = 1;
                 while (k < rmax && resident_sig(n, l + k) == rsig && (rsig.ok < 3 || band_plans_equidistant(n, l, l + k, rsig.ok == 4))) ++k;
                 // (entry lists for 8 or 4 rows at a time: on large launches the per-layer kernel, which reads them for 16, is the

@@ -1951,3 +1951,26 @@ def test_run_that_ends_in_an_error_inside_group_sums(gc, orc, monkeypatch, calls
         net.run(prune=True, first_layer=done)
         assert np.array_equal(net.categories(), ref["categories"])
         assert same_floats(net.activations(ref["categories"]), ref["y"])
+
+
+@pytest.mark.parametrize("L,asked", [(300, 300), (255, 1000), (256, 255)])
+def test_more_layers_than_one_launch_in_tiles_holds(gc, L, asked):
+    """A caller may ask for launches of any number of layers: those in tiles, which hold 254, are cut.  Against one launch
+    per layer."""
+    print("tiles, %d layers in launches of up to %d" % (L, asked), flush=True)
+    N, B = 1024, 4200
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        net.synth_layers(3, nnz_per_row=32, value=0.0625)
+        net.inspect()
+        net.synth_features(3, B, 0.1, 0.6)
+        net.run(prune=True, collect_counts=True, fuse_layers=1)
+        want = [net.active_count(l) for l in range(L)]
+        cats = net.categories()
+        y = net.activations(cats)
+        assert 0 < want[-1] < B
+        for prune in (True, False):
+            r = net.run(prune=prune, collect_counts=True, fuse_layers=asked)
+            assert r.layers_run == L and r.resident_launches >= 1
+            assert [net.active_count(l) for l in range(L)] == want
+            assert np.array_equal(net.categories(), cats)
+            assert same_floats(net.activations(cats), y)
