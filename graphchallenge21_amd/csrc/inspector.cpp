@@ -676,14 +676,15 @@ static void build_quad_form(int N, const std::vector<int32_t>& rowptr, const std
     }
 }
 
-// The TILE form of a BAND layer under one exact weight (see LayerPlan::tile_rec).  Left empty when some sixteen outputs
-// merge to more than 48 steps.
+// The TILE form of a BAND layer under one exact weight (see LayerPlan::tile_rec).  Without steps where some sixteen
+// outputs merge to more than 48 of them.
 static void build_tile_form(int N, const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col, float value,
                             LayerPlan& plan) {
     static_assert(kQuadMaxNeurons <= 1024, "a tile's inputs are a set of 1024 bits");
     const int nt = N / 16;
     uint32_t wbits;
     memcpy(&wbits, &value, 4);
+    plan.tile_rec.assign((size_t)nt * 96, 0u);
     std::vector<uint32_t> recs((size_t)nt * 96, 0u);
     int steps = 0;
     for (int c = 0; c < nt; ++c) {
@@ -941,7 +942,10 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
         plan.ell_col.clear();
         plan.rowlen.clear();
         if (N <= kQuadMaxNeurons) build_quad_form(N, rowptr, col, val, plan);
+        // (bands of other exact weights share resident launches with these in their QUAD form, which asks for plans at equal
+        // distances: they keep the room)
         if (N <= kQuadMaxNeurons && (N % 64) == 0 && plan.wmode == 0) build_tile_form(N, rowptr, col, plan.info.value, plan);
+        else if (N <= kQuadMaxNeurons && (N % 64) == 0 && plan.wmode == 1) plan.tile_rec.assign((size_t)N / 16 * 96, 0u);
     } else if (force_kernel != SPDNN_KERNEL_GATHER && !(getenv("SPDNN_TILED") && atoi(getenv("SPDNN_TILED")) == 0) &&
                build_tiled_plan(N, rowptr, col, val, plan)) {
         plan.kernel = SPDNN_KERNEL_TILED;

@@ -82,7 +82,7 @@ struct LayerPlan {
     // ... and, under one exact weight, its TILE form, for the matrix cores: the sixteen outputs at band positions 16 c ..
     // 16 c + 15 merge into one list of steps (K + 15 for a circulant band, 48 at most).  tile_rec [N/16][6][16]: the steps'
     // input columns as byte offsets (three sixteens; behind the list the last one again), the steps each output uses as
-    // a 48-bit mask (low words, high words), the weight's bits sixteen times.
+    // a 48-bit mask (low words, high words), the weight's bits sixteen times.  tile_steps 0: no such form, tile_rec is room.
     std::vector<uint32_t> tile_rec;
     int tile_steps = 0;
     // BAND: neuron j sits at the same band position as an input and as an output (see

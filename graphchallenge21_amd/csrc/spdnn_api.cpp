@@ -1851,7 +1851,7 @@ struct ResidentSig {
     int rows = 0;    // rows a workgroup keeps
     bool operator==(const ResidentSig& o) const { return ok == o.ok && full == o.full && ngroups == o.ngroups && wmode == o.wmode; }
 };
-static ResidentSig resident_sig(const spdnn_net* n, int l) {
+static ResidentSig resident_sig(const spdnn_net* n, int l, bool tiles = true) {   // tiles = false: not the TILE form
     const LayerPlan& p = n->layers[(size_t)l];
     ResidentSig g;
     if (p.kernel == SPDNN_KERNEL_BAND && p.alt_ngroups > 0) { g.ok = 1; g.full = p.alt_full ? 1 : 0; g.ngroups = p.alt_ngroups; }
@@ -1861,7 +1861,7 @@ static ResidentSig resident_sig(const spdnn_net* n, int l) {
     // entries against QUAD, times faster: 1024 neurons, 60000 rows 1.05, 1.25, 1.05, 6000 rows 0.99, 1.19, 1.01, 700 rows
     // 0.89, 1.11, 0.95; 768 neurons 1.18, 1.41, 1.08 and 1.09, 1.31, 1.01 and 0.90, 1.14, 0.92; 512 neurons 0.97, 1.14, 0.96
     // and 0.86, 1.02, 0.80 and 1.05, 1.25, 0.84.  So: from 768 neurons and a workgroup of 16 rows for every CU.
-    else if (p.kernel == SPDNN_KERNEL_BAND && p.tile_steps > 0 && n->band_resident_mode &&
+    else if (tiles && p.kernel == SPDNN_KERNEL_BAND && p.tile_steps > 0 && n->band_resident_mode &&
              (n->tile_mode == 2 || (n->tile_mode == 1 && n->N >= 768 && n->carried >= 16 * n->n_cu))) { g.ok = 4; g.ngroups = p.tile_steps; }
     else if (p.kernel == SPDNN_KERNEL_BAND && p.quad_groups > 0 && n->band_resident_mode) { g.ok = 3; g.ngroups = p.quad_groups; g.wmode = p.wmode == 2 ? 2 : 1; }
     if (g.ok) {
@@ -2146,12 +2146,37 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // (band quads: a layer inside the launch takes 0.88 of its time alone at 60000 rows, 0.76 at 6000, and rows in
                 // and out cost the launch what 1.5 layers take at either size: worth it from 16 and from 6 layers)
                 // (band tiles: from 4; 120 layers that keep 40000 of 60000 rows take 8.4 ms with 3 or 4, 8.6 with 8, 8.7 with 16)
-                const int band_rmin = n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : rsig.ok == 4 ? 4 : (n->carried >= 16384 ? 16 : 6);
-                const int rmin = (persist_asked || wide_rows) ? 2 : rsig.ok >= 3 ? band_rmin : 8;
-                int rmax = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
-                if (rsig.ok == 4) rmax = std::min(rmax, kTileMaxLayers);
-                int k = 1;
-                while (k < rmax && resident_sig(n, l + k) == rsig && (rsig.ok < 3 || band_plans_equidistant(n, l, l + k, rsig.ok == 4))) ++k;
+                auto shortest = [&](const ResidentSig& g) {
+                    if (persist_asked || wide_rows) return 2;
+                    if (g.ok < 3) return 8;
+                    return n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : g.ok == 4 ? 4 : (n->carried >= 16384 ? 16 : 6);
+                };
+                const int room = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
+                // layers from l0 on that one launch takes in the form g, of `most`
+                auto run_of = [&](int l0, const ResidentSig& g, int most, bool tiles) {
+                    if (g.ok == 4) most = std::min(most, kTileMaxLayers);
+                    int k = 1;
+                    while (k < most && resident_sig(n, l0 + k, tiles) == g && (g.ok < 3 || band_plans_equidistant(n, l0, l0 + k, g.ok == 4))) ++k;
+                    return k;
+                };
+                int k = run_of(l, rsig, room, true);
+                // Bands under one weight have both forms, other bands the QUAD form alone.  Where a run of layers is a mixture of
+                // the two, tiles would cut it into pieces: taken as QUAD throughout if that costs less, counted in layers of a
+                // QUAD launch - alone a layer takes 1.45 of them, in tiles 0.95, rows in and out 1.25 (6000 x 1024, five
+                // layers of several weights behind one of one weight, ten times over: 0.82 ms in ten launches, 1.08 layer by
+                // layer; the other way round 0.82 in ten launches, 0.90 as one layer and five in tiles).
+                const ResidentSig quad = rsig.ok >= 3 ? resident_sig(n, l, false) : ResidentSig{};
+                const int kq = quad.ok == 3 ? run_of(l, quad, room, false) : 0;
+                if (kq > k && kq >= shortest(quad)) {
+                    double pieces = 0.0;
+                    for (int i = 0, m; i < kq; i += m) {
+                        const ResidentSig g = resident_sig(n, l + i);
+                        m = run_of(l + i, g, kq - i, true);
+                        pieces += m < shortest(g) ? 1.45 * m : g.ok == 4 ? 1.25 + 0.95 * m : 1.25 + m;
+                    }
+                    if (1.25 + kq <= pieces) { rsig = quad; k = kq; }
+                }
+                const int rmin = shortest(rsig);
                 // (entry lists for 8 or 4 rows at a time: on large launches the per-layer kernel, which reads them for 16, is the
                 // faster one - measured per layer at batch 60000: N=2048 376 against 337 us, N=4096 1232 against 948; at 2048
                 // rows 13 against 38 and 42 against 57)

@@ -1974,3 +1974,43 @@ def test_more_layers_than_one_launch_in_tiles_holds(gc, L, asked):
             assert [net.active_count(l) for l in range(L)] == want
             assert np.array_equal(net.categories(), cats)
             assert same_floats(net.activations(cats), y)
+
+
+@pytest.mark.parametrize("N,B,pattern,resident,launches", [
+    (1024, 4200, "011111" * 3, 3, 3),     # behind one layer of one weight those of several, too few for a launch of their own
+    (768, 4200, "100000" * 3, 3, 3),      # the other way round: alone the first layer would be left over
+    (1024, 4200, "1" + "0" * 17, 1, 2),   # long enough in tiles: the first layer alone
+    (512, 900, "011111" * 2, 2, 2),       # narrower layers keep the QUAD form anyway
+])
+def test_resident_launches_of_bands_of_one_weight_among_others(gc, orc, N, B, pattern, resident, launches):
+    """Band layers of one power-of-two weight (which have a TILE form) among band layers of several (which do not): one
+    resident launch holds both, in the QUAD form, where tiles would leave pieces too short for a launch."""
+    print("bands of one weight among others N=%d %s" % (N, pattern), flush=True)
+    rng = np.random.default_rng(N)
+    layers = []
+    for l, kind in enumerate(pattern):
+        rp, c, v = orc.gen_layer_csr(11, l % 6, N)
+        if kind == "1":
+            v = np.ldexp(1.0, rng.choice([-5, -4, -3], size=len(v), p=[0.4, 0.4, 0.2])).astype(np.float32)
+        layers.append((rp, c, v))
+    L = len(layers)
+    dens = np.where(rng.random(B) < 0.4, 0.8, 0.05).astype(np.float32)
+    feats = (rng.random((B, N), dtype=np.float32) < dens[:, None]).astype(np.float32)
+    ref = orc.infer(feats[:200], layers, -0.3, prune=True)
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        net.run(prune=True, collect_counts=True, fuse_layers=1)
+        want = [net.active_count(l) for l in range(L)]
+        cats = net.categories()
+        y = net.activations(cats)
+        assert np.array_equal(cats[cats < 200], ref["categories"]) and same_floats(y[cats < 200], ref["y"])
+        for prune in (False, True):
+            r = net.run(prune=prune, collect_counts=True)
+            if not prune:
+                assert (r.resident_launches, r.launches) == (resident, launches)
+            assert [net.active_count(l) for l in range(L)] == want
+            assert np.array_equal(net.categories(), cats)
+            assert same_floats(net.activations(cats), y)
