@@ -230,6 +230,96 @@ class CopyCrew {
     int running_ = 0;
 };
 
+// Pinned memory for transfers from and to a caller's memory: sets of four slots, lent to the network that transfers and
+// shared by all networks of the process.  What a new set costs is not the allocation (0.05 - 0.4 ms) but the host's
+// first touch of its pages, 0.4 ms per MiB: held by each network, a network's first read-back of 9 MB took 2.1 - 2.3 ms,
+// more than through pageable memory (0.76); out of a set that is there it takes 0.6.
+// At most two sets stay here idle (two threads that transfer in turn find theirs), none with slots above kStageMaxSlot;
+// without a network in the process one is left, of kStageMaxRest bytes at most, for the next one.
+constexpr int kStageSlots = 4;
+constexpr size_t kStageMaxSlot = (size_t)16 << 20;
+constexpr size_t kStageMaxRest = (size_t)16 << 20;
+class StagePool {
+  public:
+    struct Set { unsigned char* p = nullptr; size_t slot = 0; };
+    static StagePool& get() {
+        static StagePool* const pool = new StagePool;   // (never destroyed: the runtime may be gone before it at the end)
+        return *pool;
+    }
+    void network_created() { std::lock_guard<std::mutex> lk(m_); ++networks_; }
+    void network_destroyed() {
+        std::lock_guard<std::mutex> lk(m_);
+        --networks_;
+        trim();
+    }
+    // a set with slots of `slot` bytes at least: an idle one, or a new one in the place of the largest idle one
+    hipError_t lend(size_t slot, Set* out) {
+        std::lock_guard<std::mutex> lk(m_);
+        if (take(slot, out)) return hipSuccess;
+        if (!idle_.empty()) drop(idle_.size() - 1);
+        Set s;
+        const hipError_t e = hipHostMalloc((void**)&s.p, slot * kStageSlots);
+        if (e != hipSuccess) return e;
+        s.slot = slot;
+        *out = s;
+        return hipSuccess;
+    }
+    // ... an idle one only
+    bool lend_idle(size_t slot, Set* out) {
+        std::lock_guard<std::mutex> lk(m_);
+        return take(slot, out);
+    }
+    void give_back(const Set& s) {
+        std::lock_guard<std::mutex> lk(m_);
+        size_t at = 0;   // (ordered by size)
+        while (at < idle_.size() && idle_[at].slot < s.slot) ++at;
+        idle_.insert(idle_.begin() + (long)at, s);
+        trim();
+    }
+
+  private:
+    StagePool() { idle_.reserve(4); }   // (give_back, in a destructor, allocates nothing)
+    bool take(size_t slot, Set* out) {
+        for (size_t i = 0; i < idle_.size(); ++i)
+            if (idle_[i].slot >= slot) {
+                *out = idle_[i];
+                idle_.erase(idle_.begin() + (long)i);
+                return true;
+            }
+        return false;
+    }
+    void drop(size_t i) {
+        hipHostFree(idle_[i].p);
+        idle_.erase(idle_.begin() + (long)i);
+    }
+    void trim() {
+        const size_t most = networks_ > 0 ? kStageMaxSlot : kStageMaxRest / kStageSlots;
+        while (!idle_.empty() && idle_.back().slot > most) drop(idle_.size() - 1);
+        while (idle_.size() > (networks_ > 0 ? 2u : 1u)) drop(0);
+    }
+    std::mutex m_;
+    std::vector<Set> idle_;
+    int networks_ = 0;
+};
+
+// A set for the length of one transfer.  Left early, the transfer may still be under way: the stream is waited for
+// before the set goes back.
+struct StageLease {
+    StagePool::Set set;
+    hipStream_t stream;
+    size_t slot = 0;      // bytes of a slot as this transfer uses them
+    bool done = false;    // nothing queued touches the set any more
+    explicit StageLease(hipStream_t s) : stream(s) {}
+    ~StageLease() {
+        if (!set.p) return;
+        if (!done) hipStreamSynchronize(stream);
+        StagePool::get().give_back(set);
+    }
+    StageLease(const StageLease&) = delete;
+    StageLease& operator=(const StageLease&) = delete;
+    unsigned char* at(int k) const { return set.p + (size_t)(k % kStageSlots) * slot; }
+};
+
 int host_threads() {
     const char* e = getenv("SPDNN_HOST_THREADS");
     int n = e ? atoi(e) : 0;
@@ -320,11 +410,9 @@ struct spdnn_net {
     int32_t* d_counts = nullptr; // per-layer active-row counters (device)
     int32_t* h_counts = nullptr; // pinned mirror
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-    // Transfers from and to a caller's memory (see ensure_staging): pinned slots, an event per slot, and the device copy of
-    // the rows that are packed at a time
-    unsigned char* h_stage = nullptr;
-    size_t stage_slot = 0;
-    hipEvent_t ev_stage[4] = {};
+    // Transfers from and to a caller's memory (see StagePool): an event per slot, and the device copy of the rows that are
+    // packed at a time
+    hipEvent_t ev_stage[kStageSlots] = {};
     float* d_stage = nullptr;
     size_t d_stage_bytes = 0;
     int32_t* d_rowtab = nullptr;      // see spdnn_get_activations
@@ -433,9 +521,6 @@ void release_device_base(spdnn_net* n) {
     n->ev_free.clear();
     n->exploring.clear();
     n->ev_layer.clear();
-    if (n->h_stage) hipHostFree(n->h_stage);
-    n->h_stage = nullptr;
-    n->stage_slot = 0;
     hipFree(n->d_stage);
     n->d_stage = nullptr;
     n->d_stage_bytes = 0;
@@ -505,22 +590,16 @@ int ensure_device(spdnn_net* n) {
     return rc;
 }
 
-// Pinned slots for a transfer of `bytes` in units of `unit`: four of 16 MiB at most (or of one unit, where that is more),
-// kept with the network and grown when a larger transfer comes.  At 16 MiB a slot takes the link 0.3 ms, against which
-// the launch and the waits around it are small (590 MB read back in 12.2 ms; with slots of 8 MiB 13.6); small transfers
-// keep small slots, because pinning costs 0.2 ms per MiB.
-constexpr int kStageSlots = 4;
-int ensure_staging(spdnn_net* n, size_t bytes, size_t unit) {
-    size_t slot = std::min<size_t>((size_t)16 << 20, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
+// Pinned slots for a transfer of `bytes` in units of `unit`: a quarter of it each, 16 MiB at most (or one unit, where that
+// is more).  At 16 MiB a slot takes the link 0.3 ms, against which the launch and the waits around it are small (590 MB
+// read back in 12.2 ms; with slots of 8 MiB 13.6).
+int lend_staging(spdnn_net* n, size_t bytes, size_t unit, StageLease* lease) {
+    size_t slot = std::min<size_t>(kStageMaxSlot, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
     slot = (std::max(slot, unit) + 4095) & ~(size_t)4095;
     for (hipEvent_t& e : n->ev_stage)
         if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (n->stage_slot >= slot) return SPDNN_OK;
-    if (n->h_stage) hipHostFree(n->h_stage);
-    n->h_stage = nullptr;
-    n->stage_slot = 0;
-    HIPCHK(hipHostMalloc((void**)&n->h_stage, slot * kStageSlots));
-    n->stage_slot = slot;
+    HIPCHK(StagePool::get().lend(slot, &lease->set));
+    lease->slot = slot;
     return SPDNN_OK;
 }
 // Part `part` of CopyCrew::kParts of a piece of `bytes`
@@ -1068,6 +1147,7 @@ static int spdnn_create_impl(int neuron, int max_batch, int layers, float bias, 
         const int w = atoi(e);
         if (w == 0 || (w >= 2 && w <= 64)) n->plan_window = w;
     }
+    StagePool::get().network_created();
     *out = n;
     return SPDNN_OK;
 }
@@ -1082,6 +1162,7 @@ static int spdnn_destroy_impl(spdnn_net* n) {
         release_device_base(n);
     }
     delete n;
+    StagePool::get().network_destroyed();
     return SPDNN_OK;
 }
 
@@ -1492,26 +1573,26 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
         HIPCHK(dev_malloc(&n->d_stage, chunk_bytes));
         n->d_stage_bytes = chunk_bytes;
     }
-    rc = ensure_staging(n, total, 4096);
+    StageLease lease(n->stream);
+    rc = lend_staging(n, total, 4096, &lease);
     if (rc) return rc;
     HIPCHK(launch_fill_i32(n->d_nonfinite, 2, 0, n->stream));
     struct Piece { size_t at, bytes; bool last; };   // last: of its chunk
     std::vector<Piece> pieces;
     for (size_t c = 0; c < total; c += chunk_bytes) {
         const size_t end = std::min(total, c + chunk_bytes);
-        for (size_t p = c; p < end; p += n->stage_slot) pieces.push_back({p, std::min(n->stage_slot, end - p), p + n->stage_slot >= end});
+        for (size_t p = c; p < end; p += lease.slot) pieces.push_back({p, std::min(lease.slot, end - p), p + lease.slot >= end});
     }
     {
-        auto slot_at = [&](int k) { return n->h_stage + (size_t)(k % kStageSlots) * n->stage_slot; };
         CopyCrew crew(total >= kCrewMinBytes ? n->pool.get() : nullptr, (int)pieces.size(), [&](int k, int part) {
-            copy_part(slot_at(k), (const char*)rowmajor + pieces[(size_t)k].at, pieces[(size_t)k].bytes, part);
+            copy_part(lease.at(k), (const char*)rowmajor + pieces[(size_t)k].at, pieces[(size_t)k].bytes, part);
         });
         const int K = (int)pieces.size();
         for (int k = 0; k < std::min(K, kStageSlots); ++k) crew.open(k);
         for (int k = 0; k < K; ++k) {
             const Piece& p = pieces[(size_t)k];
             crew.wait(k);
-            HIPCHK(hipMemcpyAsync((char*)n->d_stage + p.at % chunk_bytes, slot_at(k), p.bytes, hipMemcpyHostToDevice, n->stream));
+            HIPCHK(hipMemcpyAsync((char*)n->d_stage + p.at % chunk_bytes, lease.at(k), p.bytes, hipMemcpyHostToDevice, n->stream));
             HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
             if (p.last) {
                 // rows behind the batch's last inside the chunk are written as zero by the kernel
@@ -1527,10 +1608,11 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
         }
     }
     int32_t bad[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(n->h_stage, n->d_nonfinite, 8, hipMemcpyDeviceToHost, n->stream));
+    HIPCHK(hipMemcpyAsync(lease.at(0), n->d_nonfinite, 8, hipMemcpyDeviceToHost, n->stream));
     HIPCHK(launch_iota_gid(n->d_gid, n->rows_cap, batch, n->stream));
     HIPCHK(hipStreamSynchronize(n->stream));
-    memcpy(bad, n->h_stage, 8);
+    lease.done = true;
+    memcpy(bad, lease.at(0), 8);
     if (bad[0]) return fail(SPDNN_E_ARG, "features contain NaN, infinity or values above 2^100 in magnitude");
     if (bad[1]) return fail(SPDNN_E_ARG, "features contain nonzero values below 2^-100 in magnitude");
     n->have_features = true;
@@ -2552,14 +2634,16 @@ static int spdnn_get_categories_impl(spdnn_net* n, int32_t* ids, int64_t cap, in
     if (cap < n->alive) return fail(SPDNN_E_ARG, "ids buffer too small");
     if (!n->alive_list_valid) return fail(SPDNN_E_STATE, "no active list available");
     const size_t bytes = (size_t)n->alive * 4;
-    if (int rc = ensure_staging(n, bytes, 4096)) return rc;
-    if (bytes > n->stage_slot * kStageSlots) {
+    // (2000 ids: 20 us through pinned memory, 27 - 36 through pageable; a new set for them alone would cost more)
+    StageLease lease(n->stream);
+    if (!StagePool::get().lend_idle((bytes + kStageSlots - 1) / kStageSlots, &lease.set)) {
         HIPCHK(hipMemcpy(ids, n->d_alive_gid, bytes, hipMemcpyDeviceToHost));
         return SPDNN_OK;
     }
-    HIPCHK(hipMemcpyAsync(n->h_stage, n->d_alive_gid, bytes, hipMemcpyDeviceToHost, n->stream));
+    HIPCHK(hipMemcpyAsync(lease.at(0), n->d_alive_gid, bytes, hipMemcpyDeviceToHost, n->stream));
     HIPCHK(hipStreamSynchronize(n->stream));
-    memcpy(ids, n->h_stage, bytes);
+    lease.done = true;
+    memcpy(ids, lease.at(0), bytes);
     return SPDNN_OK;
 }
 
@@ -2573,9 +2657,10 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     // The rows go through pinned slots: a kernel finds a slot's rows and writes them into it (over the link: as fast as a
     // copy command, and no copy in device memory in between), the host copies them out while the next slots are filled.
     const size_t row_bytes = (size_t)n->N * 4, id_bytes = (size_t)nrows * 4;
-    int rc = ensure_staging(n, (size_t)nrows * row_bytes, row_bytes);
+    StageLease lease(n->stream);
+    int rc = lend_staging(n, (size_t)nrows * row_bytes, row_bytes, &lease);
     if (rc) return rc;
-    const int per = (int)std::min<size_t>(65535, n->stage_slot / row_bytes);   // rows per slot
+    const int per = (int)std::min<size_t>(65535, lease.slot / row_bytes);   // rows per slot
     // global id -> physical row of the current buffer, and the ids asked for: kept until another batch size comes (an
     // allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
     const size_t table_bytes = (size_t)n->batch * 4 + id_bytes;
@@ -2590,19 +2675,17 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     int32_t* const d_ids = d_where + n->batch;
     HIPCHK(launch_row_table(n->d_gid, n->carried, n->batch, d_where, n->stream));
     const void* ids_from = rows;
-    if (id_bytes <= n->stage_slot) {   // (from pinned memory where they fit the last slot, whose rows come behind this copy)
-        unsigned char* const last_slot = n->h_stage + (size_t)(kStageSlots - 1) * n->stage_slot;
-        memcpy(last_slot, rows, id_bytes);
-        ids_from = last_slot;
+    if (id_bytes <= lease.slot) {   // (from pinned memory where they fit the last slot, whose rows come behind this copy)
+        memcpy(lease.at(kStageSlots - 1), rows, id_bytes);
+        ids_from = lease.at(kStageSlots - 1);
     }
     HIPCHK(hipMemcpyAsync(d_ids, ids_from, id_bytes, hipMemcpyHostToDevice, n->stream));
     const int32_t* lab = nullptr;
     HIPCHK(labelling_dev(n, n->cur_layer, &lab));
     const int K = (nrows + per - 1) / per;
-    auto slot_at = [&](int k) { return n->h_stage + (size_t)(k % kStageSlots) * n->stage_slot; };
     auto rows_in = [&](int k) { return std::min(per, nrows - k * per); };
     CopyCrew crew((size_t)nrows * row_bytes >= kCrewMinBytes ? n->pool.get() : nullptr, K, [&](int k, int part) {
-        copy_part(rowmajor + (size_t)k * per * n->N, slot_at(k), (size_t)rows_in(k) * row_bytes, part);
+        copy_part(rowmajor + (size_t)k * per * n->N, lease.at(k), (size_t)rows_in(k) * row_bytes, part);
     });
     auto ready = [&](int k) -> hipError_t {   // slot k's rows have arrived: handed to the crew
         const hipError_t e = hipEventSynchronize(n->ev_stage[k % kStageSlots]);
@@ -2616,11 +2699,11 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
             crew.wait(k - kStageSlots);
         }
         HIPCHK(launch_unpack_rows(n->cur, lab, d_ids + (size_t)k * per, d_where, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
-                                  (float*)slot_at(k), n->stream));
+                                  (float*)lease.at(k), n->stream));
         HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
     }
     while (arrived < K) HIPCHK(ready(arrived++));
-    crew.wait(K - 1);
+    lease.done = true;
     for (int k = std::max(0, K - kStageSlots); k < K; ++k) crew.wait(k);
     return SPDNN_OK;
 }

@@ -2014,3 +2014,77 @@ def test_resident_launches_of_bands_of_one_weight_among_others(gc, orc, N, B, pa
             assert [net.active_count(l) for l in range(L)] == want
             assert np.array_equal(net.categories(), cats)
             assert same_floats(net.activations(cats), y)
+
+
+def _device_file_bytes():
+    """Address space of this process that maps the GPU's device file: its pinned host memory, among others."""
+    total = 0
+    for line in open("/proc/self/maps"):
+        if "/dev/dri/renderD" in line:
+            a, b = line.split(None, 1)[0].split("-")
+            total += int(b, 16) - int(a, 16)
+    return total
+
+
+def test_pinned_slots_are_shared_by_the_networks_of_a_process(gc):
+    """The pinned memory of transfers belongs to the process: a network's first read-back finds what an earlier one (alive
+    or closed) has used, threads that transfer at a time have a set each, and the last network's end leaves little."""
+    print("pinned slots", flush=True)
+    import threading
+    N, B, rows = 1024, 9000, np.arange(2500, dtype=np.int32)
+    MiB = 1 << 20
+    host = gc.synth_features_host(3, N, 0, B, 0.4, 0.6)
+
+    def network(batch=B):
+        net = gc.Network(N, batch, 2, bias=-0.3)
+        net.synth_layers(3, nnz_per_row=32, value=0.0625)
+        net.inspect()
+        net.synth_features(3, batch, 0.4, 0.6)
+        return net
+
+    a = network()
+    assert same_floats(a.activations(rows), host[rows])
+    a.run(prune=True, n_layers=1)
+    a.categories()          # (a process's first copies of a kind map room of the runtime's own)
+    b = network()
+    b.run(prune=True, n_layers=1)
+    before = _device_file_bytes()
+    assert before > 0
+    ids = b.categories()
+    assert len(ids) > 2500 and b.activations(ids[:2500]).any(axis=1).all()
+    assert _device_file_bytes() - before < 4 * MiB
+
+    # two networks, a thread each, several transfers of different sizes in both directions
+    wrong = []
+
+    def work(net, shift):
+        for i in range(6):
+            n = 300 + 1700 * ((i + shift) % 3)
+            mine = np.roll(host, shift + i, axis=0)
+            net.set_features_dense(mine)
+            ask = (np.arange(n) * 7 + i) % B
+            if not same_floats(net.activations(ask.astype(np.int32)), mine[ask]):
+                wrong.append((shift, i))
+    threads = [threading.Thread(target=work, args=(net, shift)) for shift, net in enumerate((a, b))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    a.close()
+    b.close()
+
+    # sequential networks: the slots of a small transfer stay for the next one
+    with network() as net:
+        net.activations(rows)
+    with network() as net:
+        before = _device_file_bytes()
+        assert same_floats(net.activations(rows), host[rows])
+        assert _device_file_bytes() - before < 4 * MiB
+    # ... those of a large one are given back
+    with network(20000) as net:
+        before = _device_file_bytes()
+        net.activations(np.arange(20000, dtype=np.int32))
+        held = _device_file_bytes()
+        assert 50 * MiB < held - before < 70 * MiB       # (in the place of the smaller one)
+    assert held - _device_file_bytes() > 50 * MiB
