@@ -473,6 +473,7 @@ struct spdnn_net {
     int64_t tiled_min_rows = 8192;                    // see use_gather_form (SPDNN_TILED_MIN_ROWS)
     bool tiled_min_rows_given = false;                // ... set in the environment: also layers with a ROWTILE form follow it
     int rowtile_mode = 1;                             // TILED layers up to 8192 neurons wide run their ROWTILE form (SPDNN_ROWTILE=0: the tiles)
+    int pinned_staging = 1;                           // transfers go through pinned slots (SPDNN_PINNED_STAGING=0: never)
     int tile_mode = 1;                                // BAND layers of one exact weight join resident launches in their TILE form (SPDNN_BAND_TILES=0: QUAD, 2: whatever the size)
     int sums_mode = 1;                                // layers of equal groups behind one another carry group sums (SPDNN_GROUP_SUMS=0: never)
     int band_resident_mode = 1;                       // BAND layers up to 1024 neurons wide join resident launches (SPDNN_BAND_RESIDENT=0: never)
@@ -593,13 +594,29 @@ int ensure_device(spdnn_net* n) {
 // Pinned slots for a transfer of `bytes` in units of `unit`: a quarter of it each, 16 MiB at most (or one unit, where that
 // is more).  At 16 MiB a slot takes the link 0.3 ms, against which the launch and the waits around it are small (590 MB
 // read back in 12.2 ms; with slots of 8 MiB 13.6).
+// Where pinned memory is refused (or not wanted, SPDNN_PINNED_STAGING=0) the lease stays empty: such a transfer goes
+// between the caller's pageable memory and the device as the runtime does it.
 int lend_staging(spdnn_net* n, size_t bytes, size_t unit, StageLease* lease) {
+    if (!n->pinned_staging) return SPDNN_OK;
     size_t slot = std::min<size_t>(kStageMaxSlot, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
     slot = (std::max(slot, unit) + 4095) & ~(size_t)4095;
     for (hipEvent_t& e : n->ev_stage)
         if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    HIPCHK(StagePool::get().lend(slot, &lease->set));
+    if (StagePool::get().lend(slot, &lease->set) != hipSuccess) {
+        (void)hipGetLastError();
+        return SPDNN_OK;
+    }
     lease->slot = slot;
+    return SPDNN_OK;
+}
+// n->d_stage with at least `bytes`
+int ensure_d_stage(spdnn_net* n, size_t bytes) {
+    if (n->d_stage_bytes >= bytes) return SPDNN_OK;
+    hipFree(n->d_stage);
+    n->d_stage = nullptr;
+    n->d_stage_bytes = 0;
+    HIPCHK(dev_malloc(&n->d_stage, bytes));
+    n->d_stage_bytes = bytes;
     return SPDNN_OK;
 }
 // Part `part` of CopyCrew::kParts of a piece of `bytes`
@@ -1127,6 +1144,7 @@ static int spdnn_create_impl(int neuron, int max_batch, int layers, float bias, 
     if (const char* e = getenv("SPDNN_PERSIST_LIGHT_SYNC")) n->persist_light = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_SEGLEN")) n->persist_seglen = std::max(0, atoi(e));
     if (const char* e = getenv("SPDNN_RESIDENT")) n->resident_mode = atoi(e) != 0 ? 1 : 0;
+    if (const char* e = getenv("SPDNN_PINNED_STAGING")) n->pinned_staging = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_BAND_TILES")) n->tile_mode = std::min(2, std::max(0, atoi(e)));
     if (const char* e = getenv("SPDNN_GROUP_SUMS")) n->sums_mode = atoi(e) != 0 ? 1 : 0;
     if (const char* e = getenv("SPDNN_PERSIST_WAIT_US")) n->persist_wait_us = std::max(0ll, atoll(e));
@@ -1566,21 +1584,26 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
     const int padded = ((batch + RB - 1) / RB) * RB;
     chunk_rows = std::min<int64_t>(chunk_rows, padded);
     const size_t chunk_bytes = (size_t)chunk_rows * row_bytes, total = (size_t)batch * row_bytes;
-    if (n->d_stage_bytes < chunk_bytes) {
-        hipFree(n->d_stage);
-        n->d_stage = nullptr;
-        n->d_stage_bytes = 0;
-        HIPCHK(dev_malloc(&n->d_stage, chunk_bytes));
-        n->d_stage_bytes = chunk_bytes;
-    }
+    rc = ensure_d_stage(n, chunk_bytes);
+    if (rc) return rc;
     StageLease lease(n->stream);
     rc = lend_staging(n, total, 4096, &lease);
     if (rc) return rc;
     HIPCHK(launch_fill_i32(n->d_nonfinite, 2, 0, n->stream));
+    // rows r0 .. of a chunk that is in d_stage, packed; rows behind the batch's last inside the chunk are written as zero
+    auto pack = [&](int64_t r0) {
+        return launch_pack_rows(n->d_stage, n->F, n->d_lab, N, r0, (int)std::min<int64_t>(chunk_rows, batch - r0), n->rl,
+                                n->d_nonfinite, n->stream);
+    };
     struct Piece { size_t at, bytes; bool last; };   // last: of its chunk
     std::vector<Piece> pieces;
     for (size_t c = 0; c < total; c += chunk_bytes) {
         const size_t end = std::min(total, c + chunk_bytes);
+        if (!lease.set.p) {
+            HIPCHK(hipMemcpyAsync(n->d_stage, (const char*)rowmajor + c, end - c, hipMemcpyHostToDevice, n->stream));
+            HIPCHK(pack((int64_t)(c / chunk_bytes) * chunk_rows));
+            continue;
+        }
         for (size_t p = c; p < end; p += lease.slot) pieces.push_back({p, std::min(lease.slot, end - p), p + lease.slot >= end});
     }
     {
@@ -1594,12 +1617,7 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
             crew.wait(k);
             HIPCHK(hipMemcpyAsync((char*)n->d_stage + p.at % chunk_bytes, lease.at(k), p.bytes, hipMemcpyHostToDevice, n->stream));
             HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
-            if (p.last) {
-                // rows behind the batch's last inside the chunk are written as zero by the kernel
-                const int64_t r0 = (int64_t)(p.at / chunk_bytes) * chunk_rows;
-                HIPCHK(launch_pack_rows(n->d_stage, n->F, n->d_lab, N, r0, (int)std::min<int64_t>(chunk_rows, batch - r0), n->rl,
-                                        n->d_nonfinite, n->stream));
-            }
+            if (p.last) HIPCHK(pack((int64_t)(p.at / chunk_bytes) * chunk_rows));
             // the slot after the newest one: free once its transfer has ended
             if (k >= 1 && k - 1 + kStageSlots < K) {
                 HIPCHK(hipEventSynchronize(n->ev_stage[(k - 1) % kStageSlots]));
@@ -1608,11 +1626,11 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
         }
     }
     int32_t bad[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(lease.at(0), n->d_nonfinite, 8, hipMemcpyDeviceToHost, n->stream));
     HIPCHK(launch_iota_gid(n->d_gid, n->rows_cap, batch, n->stream));
+    HIPCHK(hipMemcpyAsync(lease.set.p ? (void*)lease.at(0) : bad, n->d_nonfinite, 8, hipMemcpyDeviceToHost, n->stream));
     HIPCHK(hipStreamSynchronize(n->stream));
     lease.done = true;
-    memcpy(bad, lease.at(0), 8);
+    if (lease.set.p) memcpy(bad, lease.at(0), 8);
     if (bad[0]) return fail(SPDNN_E_ARG, "features contain NaN, infinity or values above 2^100 in magnitude");
     if (bad[1]) return fail(SPDNN_E_ARG, "features contain nonzero values below 2^-100 in magnitude");
     n->have_features = true;
@@ -2636,7 +2654,7 @@ static int spdnn_get_categories_impl(spdnn_net* n, int32_t* ids, int64_t cap, in
     const size_t bytes = (size_t)n->alive * 4;
     // (2000 ids: 20 us through pinned memory, 27 - 36 through pageable; a new set for them alone would cost more)
     StageLease lease(n->stream);
-    if (!StagePool::get().lend_idle((bytes + kStageSlots - 1) / kStageSlots, &lease.set)) {
+    if (!n->pinned_staging || !StagePool::get().lend_idle((bytes + kStageSlots - 1) / kStageSlots, &lease.set)) {
         HIPCHK(hipMemcpy(ids, n->d_alive_gid, bytes, hipMemcpyDeviceToHost));
         return SPDNN_OK;
     }
@@ -2660,7 +2678,12 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     StageLease lease(n->stream);
     int rc = lend_staging(n, (size_t)nrows * row_bytes, row_bytes, &lease);
     if (rc) return rc;
-    const int per = (int)std::min<size_t>(65535, lease.slot / row_bytes);   // rows per slot
+    const bool pinned = lease.set.p != nullptr;
+    if (!pinned) {   // through device memory then, 32 MiB of rows at a time
+        rc = ensure_d_stage(n, std::max(row_bytes, std::min((size_t)nrows * row_bytes, (size_t)32 << 20)));
+        if (rc) return rc;
+    }
+    const int per = (int)std::min<size_t>(65535, (pinned ? lease.slot : n->d_stage_bytes) / row_bytes);   // rows per slot
     // global id -> physical row of the current buffer, and the ids asked for: kept until another batch size comes (an
     // allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
     const size_t table_bytes = (size_t)n->batch * 4 + id_bytes;
@@ -2684,6 +2707,15 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     HIPCHK(labelling_dev(n, n->cur_layer, &lab));
     const int K = (nrows + per - 1) / per;
     auto rows_in = [&](int k) { return std::min(per, nrows - k * per); };
+    if (!pinned) {
+        for (int k = 0; k < K; ++k) {
+            HIPCHK(launch_unpack_rows(n->cur, lab, d_ids + (size_t)k * per, d_where, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+                                      n->d_stage, n->stream));
+            HIPCHK(hipMemcpyAsync(rowmajor + (size_t)k * per * n->N, n->d_stage, (size_t)rows_in(k) * row_bytes, hipMemcpyDeviceToHost, n->stream));
+        }
+        HIPCHK(hipStreamSynchronize(n->stream));
+        return SPDNN_OK;
+    }
     CopyCrew crew((size_t)nrows * row_bytes >= kCrewMinBytes ? n->pool.get() : nullptr, K, [&](int k, int part) {
         copy_part(rowmajor + (size_t)k * per * n->N, lease.at(k), (size_t)rows_in(k) * row_bytes, part);
     });

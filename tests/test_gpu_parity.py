@@ -2088,3 +2088,42 @@ def test_pinned_slots_are_shared_by_the_networks_of_a_process(gc):
         held = _device_file_bytes()
         assert 50 * MiB < held - before < 70 * MiB       # (in the place of the smaller one)
     assert held - _device_file_bytes() > 50 * MiB
+
+
+@pytest.mark.parametrize("N,B,asked", [
+    (1000, 3, 3),
+    (1024, 20000, 20000),   # 82 MB: several chunks each way
+    (3001, 4999, 4000),     # a last chunk that is not full
+    (65536, 300, 140),      # rows of 256 KiB, 128 of them at a time
+])
+def test_transfers_without_pinned_memory(gc, monkeypatch, N, B, asked):
+    """Where no memory can be pinned the same calls go through pageable memory: nothing is refused, nothing is pinned."""
+    print("transfers without pinned memory N=%d B=%d" % (N, B), flush=True)
+    rng = np.random.default_rng(N + B)
+    monkeypatch.setenv("SPDNN_PINNED_STAGING", "0")
+    rowptr, col = np.arange(N + 1, dtype=np.int32), rng.permutation(N).astype(np.int32)
+    with gc.Network(N, B, 1, bias=-0.25) as net:
+        net.set_layer_csr(0, rowptr, col, np.full(N, 0.5, np.float32))
+        net.inspect()
+        for part in (10, 1):      # (the first turn maps room of the runtime's own)
+            b = -(-B // part)
+            feats = rng.random((b, N), dtype=np.float32)
+            before = _device_file_bytes()
+            net.set_features_dense(feats)
+            rows = rng.integers(0, b, size=-(-asked // part)).astype(np.int32)
+            assert same_floats(net.activations(rows), feats[rows])
+            net.run(prune=True)
+            ids = net.categories()
+            assert np.array_equal(ids, np.flatnonzero((feats > 0.5).any(axis=1)))
+            got = net.activations(ids[:50])
+            assert same_floats(got, np.maximum(feats[ids[:50]][:, col] * np.float32(0.5) - np.float32(0.25), 0))
+            if part == 1 and asked == 20000:      # 32 MiB of device memory, no slots
+                assert _device_file_bytes() - before < 48 << 20
+        feats[B - 1, N - 1] = np.nan
+        with pytest.raises(gc.SpdnnError):
+            net.set_features_dense(feats)
+        feats[B - 1, N - 1] = 1e-35
+        with pytest.raises(gc.SpdnnError):
+            net.set_features_dense(feats)
+        with pytest.raises(gc.SpdnnError):
+            net.activations(np.array([0], np.int32))      # no features are set now
