@@ -164,10 +164,12 @@ class JobPool {
 // the parts handed out in order (a ticket) to a few workers of the pool and to the calling thread while it waits.  The
 // caller opens the pieces one after the other (their slot may be read or written) and waits for piece k's copies.
 // One thread moves 21 GB/s between touched buffers and 5 GB/s into pages that do not exist yet - what a read-back
-// into a fresh array meets - against the 57 GB/s of the link.
+// into a fresh array meets - against the 57 GB/s of the link.  A worker whose piece is not open yet looks for it for
+// kSpinUs and then sleeps until one is opened: the device may take its time.
 class CopyCrew {
   public:
     static constexpr int kParts = 16;
+    static constexpr int kSpinUs = 50;
     CopyCrew(JobPool* pool, int pieces, std::function<void(int, int)> copy)
         : pieces_(pieces), copy_(std::move(copy)), done_(new std::atomic<int>[(size_t)pieces]) {
         for (int k = 0; k < pieces; ++k) done_[(size_t)k].store(0, std::memory_order_relaxed);
@@ -191,13 +193,18 @@ class CopyCrew {
     }
     // (every return path ends the workers before the buffers they copy go away)
     ~CopyCrew() {
-        stop_.store(true, std::memory_order_release);
         std::unique_lock<std::mutex> lk(m_);
+        stop_.store(true, std::memory_order_release);
+        cv_open_.notify_all();
         cv_.wait(lk, [this] { return running_ == 0; });
     }
     CopyCrew(const CopyCrew&) = delete;
     CopyCrew& operator=(const CopyCrew&) = delete;
-    void open(int k) { open_.store(k + 1, std::memory_order_release); }
+    void open(int k) {
+        std::lock_guard<std::mutex> lk(m_);
+        open_.store(k + 1, std::memory_order_release);
+        if (asleep_ > 0) cv_open_.notify_all();
+    }
     void wait(int k) {
         while (done_[(size_t)k].load(std::memory_order_acquire) < kParts)
             if (!step(false)) std::this_thread::yield();
@@ -206,7 +213,8 @@ class CopyCrew {
   private:
     // takes the next part and copies it.  block: waits for its piece to be opened; false: nothing (more) to take
     bool step(bool block) {
-        for (unsigned spins = 0;; ++spins) {
+        std::chrono::steady_clock::time_point since{};
+        for (unsigned spins = 1;; ++spins) {
             if (stop_.load(std::memory_order_acquire)) return false;
             int t = next_.load(std::memory_order_relaxed);
             if (t >= pieces_ * kParts) return false;
@@ -217,7 +225,17 @@ class CopyCrew {
                 return true;
             }
             if (!block) return false;
-            if ((spins & 63) == 63) std::this_thread::yield();
+            if ((spins & 63) != 0) continue;
+            const auto now = std::chrono::steady_clock::now();
+            if (since.time_since_epoch().count() == 0) since = now;
+            if (now - since < std::chrono::microseconds(kSpinUs)) {
+                std::this_thread::yield();
+                continue;
+            }
+            std::unique_lock<std::mutex> lk(m_);
+            ++asleep_;
+            cv_open_.wait(lk, [&] { return stop_.load() || next_.load() / kParts < open_.load() || next_.load() >= pieces_ * kParts; });
+            --asleep_;
         }
     }
     const int pieces_;
@@ -226,8 +244,8 @@ class CopyCrew {
     std::atomic<int> next_{0}, open_{0};
     std::atomic<bool> stop_{false};
     std::mutex m_;
-    std::condition_variable cv_;
-    int running_ = 0;
+    std::condition_variable cv_, cv_open_;
+    int running_ = 0, asleep_ = 0;
 };
 
 // Pinned memory for transfers from and to a caller's memory: sets of four slots, lent to the network that transfers and

@@ -2127,3 +2127,29 @@ def test_transfers_without_pinned_memory(gc, monkeypatch, N, B, asked):
             net.set_features_dense(feats)
         with pytest.raises(gc.SpdnnError):
             net.activations(np.array([0], np.int32))      # no features are set now
+
+
+def test_copies_that_wait_for_the_device_sleep(gc, monkeypatch):
+    """While the device is late the workers that copy between the caller's memory and the pinned slots do not poll: the
+    process uses the time of the calling thread and little more, not that of all its workers."""
+    print("copies that wait", flush=True)
+    import time
+    monkeypatch.setenv("SPDNN_HOST_THREADS", "12")
+    N, B = 1024, 24000      # 98 MB: more pieces than slots either way
+    host = gc.synth_features_host(3, N, 0, B, 0.4, 0.6)
+    rows = np.arange(B, dtype=np.int32)
+    with gc.Network(N, B, 1, bias=-0.3) as net:
+        net.synth_layers(3, nnz_per_row=32, value=0.0625)
+        net.inspect()
+        net.set_features_dense(host)
+        net.activations(rows)
+        for turn in ("in", "out"):
+            wall, cpu = time.perf_counter(), time.process_time()
+            hold_device(0.6)
+            if turn == "in":
+                net.set_features_dense(host)
+            else:
+                assert same_floats(net.activations(rows), host)
+            wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+            assert wall > 0.5
+            assert cpu < 3.5 * wall, (turn, wall, cpu)
