@@ -812,6 +812,7 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
     plan.alt_ngroups = 0;
     plan.alt_full = false;
     plan.alt_walk = false;
+    plan.sum_cols.clear();
     plan.alt_cols.clear();
     plan.alt_cnt.clear();
     plan.alt_out_at.clear();

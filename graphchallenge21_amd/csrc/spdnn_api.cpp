@@ -1423,17 +1423,19 @@ static int spdnn_inspect_impl(spdnn_net* n) {
     n->pool->wait_all();
     // (streamed plans run layer by layer: no launch there reads this form)
     const bool streamed = n->plan_window >= 2 && n->plan_window < n->L;
-    n->layers[0].sum_cols.clear();
-    for (int l = 1; l < n->L; ++l) {
-        LayerPlan *prev = &n->layers[(size_t)l - 1], *cur = &n->layers[(size_t)l];
+    for (int l = 0; l < n->L; ++l) {
+        LayerPlan* cur = &n->layers[(size_t)l];
+        cur->info.plan_bytes -= (int64_t)(2 * cur->sum_cols.size());
         cur->sum_cols.clear();
+        if (l == 0 || streamed || !n->sums_mode || sum_groups(*cur) == 0) continue;
+        const LayerPlan* prev = cur - 1;
         const int N = n->N;
-        if (!streamed && n->sums_mode && sum_groups(*cur) > 0)
-            n->pool->submit([=] { link_sums(*prev, *cur, N); });
+        n->pool->submit([=] { link_sums(*prev, *cur, N); });
     }
     n->pool->wait_all();
     for (int l = 0; l < n->L; ++l) {
         LayerPlan& p = n->layers[(size_t)l];
+        p.info.plan_bytes += (int64_t)(2 * p.sum_cols.size());
         p.fuse_next = l + 1 < n->L && n->rl == 4 && pair_fusable(p, n->layers[(size_t)l + 1], n->N);
         p.info.fuse_next = p.fuse_next ? 1 : 0;
     }

@@ -415,6 +415,35 @@ def test_radix_layers_of_one_numbering_share_an_order(gc, orc):
         assert [net.layer_plan(l).common_order for l in range(len(layers))] == [1, 2, 0, 0, 1, 2, 2, 1, 0, 1]
 
 
+def test_plan_bytes_hold_the_lists_of_group_sums(gc, monkeypatch):
+    """A layer of equal groups behind another one holds 64 bytes per group for its inputs named by group; they are part
+    of its plan bytes, however often the network is inspected, and go with a neighbour that has no groups."""
+    N, L = 512, 4
+    rng = np.random.default_rng(4)
+    layers = [radix_like_csr(rng, N, 16 << l) for l in range(L)]
+
+    def plan_bytes(net):
+        return np.array([net.layer_plan(l).plan_bytes for l in range(L)])
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", mode)
+        with gc.Network(N, 64, L, bias=-0.3) as net:
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            for _ in range(2):
+                net.inspect()
+                assert mode not in got or np.array_equal(got[mode], plan_bytes(net))
+                got[mode] = plan_bytes(net)
+            net.set_layer_csr(2, *layers[2])
+            net.inspect()
+            assert np.array_equal(got[mode], plan_bytes(net))
+            net.set_layer_csr(1, *random_csr(rng, N, 5))
+            net.inspect()
+            other = plan_bytes(net)
+            assert other[0] == got["0"][0] and other[2] == got["0"][2] and other[3] == got[mode][3]
+    assert np.array_equal(got["1"] - got["0"], [0] + [64 * (N // 16)] * (L - 1))
+
+
 def test_forced_gather(gc, orc):
     with gc.Network(256, 4, 2, bias=-0.3, force_kernel=gc.KERNEL_GATHER) as net:
         net.synth_layers(0, nnz_per_row=8)
