@@ -2077,7 +2077,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
         for (int l = first; l <= last; ++l) h[l] = -1;
     }
     struct Rec { int l0, c, pl; };   // counts of layers [l0, l0+c) on their way to the host; pl: the persistent launch they come from (ordinal), or -1
-    struct Timed { int l0, c; };
+    struct Timed { int l0, c; size_t ev; };   // ev: the first of its two events
     std::vector<Rec> recs;
     std::vector<Timed> timed;
 
@@ -2091,18 +2091,30 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     State st{};
     st.l = first; st.dead = n->carried == 0; st.count_pending = false; st.last_launched = -1; st.newest_count = -1;
     st.c_prune = 1; st.pub = Publish{}; st.processed = 0; st.r = spdnn_run_result{}; st.sums = 0;
-    // the group sums that n->cur holds, written out for whatever reads the full columns next
+    // the group sums that n->cur holds, written out for whatever reads the full columns next: a launch that counts as part
+    // of the layer that computed them
+    size_t expansions = 0;
     auto expand_sums = [&]() -> hipError_t {
         const LayerPlan& p = n->layers[(size_t)n->cur_layer - 1];
         const DevLayer& d = n->dl[(size_t)n->cur_layer - 1];
         const Feat full = (n->cur == n->A) ? n->C : n->A;
-        const hipError_t e = launch_sums_expand(n->cur, full, p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst, n->N, st.sums,
-                                                n->carried / n->RB, n->rl, n->stream);
-        if (e == hipSuccess) {
-            n->cur = full;
-            st.sums = 0;
+        const size_t ev = 2 * ((size_t)n->L + expansions++);
+        hipError_t e = hipSuccess;
+        while (opt.time_layers && n->ev_layer.size() < ev + 2) {
+            hipEvent_t x;
+            if ((e = hipEventCreate(&x)) != hipSuccess) return e;
+            n->ev_layer.push_back(x);
         }
-        return e;
+        if (opt.time_layers && (e = hipEventRecord(n->ev_layer[ev], n->stream)) != hipSuccess) return e;
+        e = launch_sums_expand(n->cur, full, p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst, n->N, st.sums, n->carried / n->RB,
+                               n->rl, n->stream);
+        if (e != hipSuccess) return e;
+        n->cur = full;
+        st.sums = 0;
+        st.r.launches += 1;
+        if (!opt.time_layers) return hipSuccess;
+        timed.push_back({n->cur_layer - 1, 1, ev});
+        return hipEventRecord(n->ev_layer[ev + 1], n->stream);
     };
     // A run that ends in an error behind such a launch leaves full columns behind, as one that ends elsewhere does: the
     // state may be read, and a later run may continue it.  Where even that launch fails there is no state to speak of.
@@ -2480,7 +2492,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // the first layer's rows: nobody looks at active_mid again, so they are counted here
                 if (fused_count) HIPCHK(launch_count_stamped(n->d_active_mid, n->carried, stamp0, n->d_counts + l, n->stream));
             }
-            if (opt.time_layers) { HIPCHK(hipEventRecord(n->ev_layer[(size_t)(2 * l + 1)], n->stream)); timed.push_back({l, c}); }
+            if (opt.time_layers) { HIPCHK(hipEventRecord(n->ev_layer[(size_t)(2 * l + 1)], n->stream)); timed.push_back({l, c, (size_t)(2 * l)}); }
             st.r.layers_run += c;
             st.r.launches += (fb ? c : 1);
             if (pair) st.r.fused_pairs += 1;
@@ -2618,8 +2630,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     HIPCHK(hipEventElapsedTime(&r.ms_total, n->ev_start, n->ev_stop));
     for (const Timed& t : timed) {
         float ms = 0.0f;
-        HIPCHK(hipEventElapsedTime(&ms, n->ev_layer[(size_t)(2 * t.l0)], n->ev_layer[(size_t)(2 * t.l0 + 1)]));
-        for (int j = 0; j < t.c; ++j) n->layer_ms[(size_t)(t.l0 + j)] = ms / (float)t.c;
+        HIPCHK(hipEventElapsedTime(&ms, n->ev_layer[t.ev], n->ev_layer[t.ev + 1]));
+        for (int j = 0; j < t.c; ++j) n->layer_ms[(size_t)(t.l0 + j)] += ms / (float)t.c;
         r.ms_kernels += ms;
     }
     // per-layer counts: everything that was launched has finished now

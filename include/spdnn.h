@@ -124,7 +124,8 @@ typedef struct spdnn_run_result {
     float   ms_kernels;      /* sum of per-layer kernel times (time_layers only, else 0)          */
     double  alg_bytes;       /* sum over layers of 8*B_l*N + nnz_l*8 + 4*(N+1)                     */
     double  edges;           /* batch * nnz summed over the layers requested                      */
-    int32_t launches;        /* layer-kernel launches made (a fused launch counts once)           */
+    int32_t launches;        /* layer-kernel launches made (a fused launch counts once, and so does the expansion behind
+                                layers that carry one column per group)                           */
     int32_t fused_pairs;     /* of them, fused pairs of layers (intermediate tile in LDS)         */
     int32_t persistent_launches;   /* of them, persistent launches (several layers, a dependency per row block)   */
     int32_t persistent_fallbacks;  /* persistent launches that gave up and were finished by per-layer launches     */

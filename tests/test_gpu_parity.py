@@ -2153,3 +2153,29 @@ def test_copies_that_wait_for_the_device_sleep(gc, monkeypatch):
             wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
             assert wall > 0.5
             assert cpu < 3.5 * wall, (turn, wall, cpu)
+
+
+def test_the_expansion_of_group_sums_is_counted_and_timed(gc):
+    """The launch that writes the full columns behind layers of group sums is one of the launches, and its time part of the
+    last such layer's and of the kernel time."""
+    print("expansion counted and timed", flush=True)
+    N, B, L = 4096, 20000, 7
+    rng = np.random.default_rng(8)
+    base = [radix_like_csr(rng, N, 16 << k) for k in range(3)]
+    with gc.Network(N, B, L, bias=-0.35) as net:
+        for l in range(L):
+            net.set_layer_csr(l, *base[l % 3])
+        net.inspect()
+        net.synth_features(3, B, 0.5, 0.6)
+        net.run(prune=False)
+        r = net.run(prune=False, time_layers=True)
+        ms = net.layer_times()
+        # the head, one launch of six layers, the expansion (0.33 GB written: 0.04 ms at the very least)
+        assert (r.resident_launches, r.launches) == (1, 3)
+        assert (ms[1:-1] == ms[1]).all() and ms[-1] > ms[1] + 0.03
+        assert abs(ms.sum() - r.ms_kernels) < 1e-3 and r.ms_kernels < r.ms_total
+        # cut behind the fourth layer: an expansion at the end of each call
+        for kw, launches in (({"n_layers": 4}, 3), ({"first_layer": 4}, 3)):
+            r = net.run(prune=False, time_layers=True, **kw)
+            assert (r.resident_launches, r.launches) == (1, launches)
+            assert abs(net.layer_times()[kw.get("first_layer", 0):kw.get("n_layers", L)].sum() - r.ms_kernels) < 1e-3
