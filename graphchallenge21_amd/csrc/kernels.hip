@@ -426,7 +426,6 @@ __device__ __forceinline__ float relu_clamp(float y, float clampv) {
 // ------------------------------------------------------------------------------------------
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 load_const_u4(const __attribute__((address_space(4))) uint32_t* p) {
     const u32x4_t v = *(const __attribute__((address_space(4))) u32x4_t*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
@@ -2024,8 +2023,9 @@ __global__ __launch_bounds__(1024) void block_resident_kernel(ResidentArgs a) {
 // ------------------------------------------------------------------------------------------
 // Group sums (see launch_sums_head): layers of equal groups behind one another carry one column per group.
 // ------------------------------------------------------------------------------------------
-// The first layer of such a run: block_kernel's loads and sums, one store per group.
-// Every column is read by two groups; at 60000 x 65536 (15.7 GB) 4.5 ms, where the walk that writes full columns takes 5.25.
+// The first layer of such a run where its groups cannot be walked (narrow layers, groups that share inputs in other ways):
+// block_kernel's loads and sums, one store per group.  Every column is read by two groups; forced onto 60000 x 65536
+// (15.7 GB), where sums_walk_kernel runs, it takes 4.5 ms against 3.04.
 template <int RL, bool FULL>
 __global__ __launch_bounds__(256) void sums_head_kernel(
     Feat yin_all, Feat yout_all, const int32_t* __restrict__ grp_cols, const int32_t* __restrict__ grp_cnt,
@@ -2084,7 +2084,8 @@ __global__ __launch_bounds__(256) void sums_head_kernel(
 // The same where the groups are the tiles of a run-chain band: group t reads 32 of the columns [16 t - 32, 16 t + 16).  A
 // wave owns 64 rows, one to a lane, and walks a segment of the groups: sixteen new columns per group into its own
 // ring of 64 columns in LDS - requested two groups ahead, which is what keeps the memory busy - and 32 reads from it.
-// A lane only ever reads its own row, so there is no barrier.  Every column is read once: 60000 x 65536 3.04 ms
+// A lane only ever reads its own row, so there is no barrier.  Groups are taken in twos: there is a multiple of four of
+// them (N is a multiple of 64), and so there is in every segment.  Every column is read once: 60000 x 65536 3.04 ms
 // (16.7 GB, 5.5 TB/s) against 4.51 with every column read by two groups, 12000 x 16384 0.17 ms against 0.24.
 template <int RL>
 __global__ __launch_bounds__(64 * RL) void sums_walk_kernel(
@@ -2121,7 +2122,7 @@ __global__ __launch_bounds__(64 * RL) void sums_walk_kernel(
     keep((t0 + ngroups - 2) % ngroups, a);
 #pragma unroll
     for (int i = 0; i < 16; ++i) a[i] = c[i];
-    request(min(t0 + 1, t1 - 1), c);
+    request(t0 + 1, c);
     keep((t0 + ngroups - 1) % ngroups, b);
     float nz = 0.0f;
     auto group = [&](int t, float* next) {   // `next` holds the columns of group t, and takes those of t + 2
@@ -2138,12 +2139,10 @@ __global__ __launch_bounds__(64 * RL) void sums_walk_kernel(
         nz = nz_merge(nz, y);
         yout[(size_t)t * RB] = y;
     };
-    int t = t0;
-    for (; t + 1 < t1; t += 2) {
+    for (int t = t0; t < t1; t += 2) {
         group(t, a);
         group(t + 1, c);
     }
-    if (t < t1) group(t, a);
     if (nz > 0.0f) active[(size_t)rb * RB + wave * 64 + lane] = stamp;
 }
 
@@ -3729,15 +3728,21 @@ hipError_t launch_block(const BlockLaunch& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// groups of a segment of sums_walk_kernel: a segment reads two groups' columns in front of its first, so as long as still
+// leaves the chip a few workgroups per slot
+int sums_walk_segment(int nblk, int ngroups) {
+    int seg = 256;
+    while (seg > 16 && (long long)nblk * ((ngroups + seg - 1) / seg) < 2048) seg >>= 1;
+    return seg;
+}
+
 hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s) {
     if (a.N <= 0 || a.ngroups <= 0 || a.nblk <= 0 || !a.yin || !a.yout || a.yin == a.yout || !a.cols || !a.cnt || !a.active ||
         a.wmode != 0 || a.ngroups > a.N)
         return hipErrorInvalidValue;
     if (a.walk) {
         if (!a.full || (a.N % 64) != 0 || a.ngroups * 16 != a.N) return hipErrorInvalidValue;
-        // a segment reads two groups' columns in front of its first: as long as still leaves the chip a few workgroups per slot
-        int seg = 256;
-        while (seg > 16 && (long long)a.nblk * ((a.ngroups + seg - 1) / seg) < 2048) seg >>= 1;
+        const int seg = sums_walk_segment(a.nblk, a.ngroups);
         dim3 grid(a.nblk, (a.ngroups + seg - 1) / seg), block(64 * a.rl);
         if (grid.y > 65535) return hipErrorInvalidValue;
 #define SPDNN_WALK(RLv)                                                                                                   \
@@ -3800,16 +3805,22 @@ static hipError_t launch_sums_resident_r(const SumsLaunch& a, int nthr, hipStrea
     return hipGetLastError();
 }
 
+static int sums_threads(int ngroups) { return std::min(1024, (ngroups + 63) / 64 * 64); }
+
+// rows a workgroup of sums_resident_kernel keeps: fewer where four would leave CUs without a workgroup
+int sums_rows_per_workgroup(int ngroups, int rows, int n_cu) {
+    int R = 4;
+    while (R > 1 && (long long)(rows / R) * sums_threads(ngroups) < (long long)n_cu * 1024) R /= 2;
+    return R;
+}
+
 hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s) {
     // host-side shape checks: what the 16-bit lists and the two LDS buffers assume
     if (a.nlayers < 1 || !a.table || !a.yin || !a.yout || a.yin == a.yout || !a.active || a.ngroups <= 0 || a.ngroups > 4096 ||
         a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0)
         return hipErrorInvalidValue;
-    const int nthr = std::min(1024, (a.ngroups + 63) / 64 * 64);
-    // fewer rows per workgroup where four would leave CUs without one
-    const long long threads = (long long)a.n_cu * 1024;
-    int R = 4;
-    while (R > 1 && (long long)(a.rows / R) * nthr < threads) R /= 2;
+    const int nthr = sums_threads(a.ngroups);
+    const int R = sums_rows_per_workgroup(a.ngroups, a.rows, a.n_cu);
     return R == 4 ? launch_sums_resident_r<4>(a, nthr, s) : R == 2 ? launch_sums_resident_r<2>(a, nthr, s)
                                                                    : launch_sums_resident_r<1>(a, nthr, s);
 }

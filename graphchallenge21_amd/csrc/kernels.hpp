@@ -162,6 +162,7 @@ hipError_t launch_block(const BlockLaunch& a, hipStream_t s);
 //   launch_sums_expand: group sums written out as the full columns that any kernel may read
 // Buffers of group sums have the row-block layout with ngroups columns.
 hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s);
+int sums_walk_segment(int nblk, int ngroups);
 struct LayerDesc;   // (a.wmode 0; a.dst is not used)
 struct SumsLaunch {
     const LayerDesc* table;       // device pointer to the entry of the launch's first layer
@@ -175,6 +176,7 @@ struct SumsLaunch {
     Publish publish;
 };
 hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s);
+int sums_rows_per_workgroup(int ngroups, int rows, int n_cu);
 hipError_t launch_sums_expand(const Feat& sums, const Feat& full, const int32_t* dst, int N, int ngroups, int nblk, int rl,
                               hipStream_t s);
 

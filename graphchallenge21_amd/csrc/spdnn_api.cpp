@@ -2423,6 +2423,11 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 b.walk = alt && p.alt_walk ? 1 : 0;
                 b.wu = p.info.value; b.bias = n->bias; b.clampv = n->clampv; b.publish = st.pub;
                 HIPCHK(launch_sums_head(b, n->stream));
+                if (n->run_verbose && b.walk)
+                    fprintf(stderr, "spdnn: group sums, head (walk): layer %d, %d rows, %d groups, segments of %d\n", l, n->carried, b.ngroups,
+                            sums_walk_segment(nblk, b.ngroups));
+                else if (n->run_verbose)
+                    fprintf(stderr, "spdnn: group sums, head (lists): layer %d, %d rows, %d groups\n", l, n->carried, b.ngroups);
             } else if (chain) {
                 SumsLaunch sl{};
                 sl.table = n->d_table + l; sl.nlayers = c; sl.yin = in; sl.yout = out; sl.active = n->d_active; sl.ngroups = st.sums;
@@ -2430,7 +2435,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 sl.n_cu = n->n_cu; sl.bias = n->bias; sl.clampv = n->clampv; sl.publish = st.pub;
                 HIPCHK(launch_sums_resident(sl, n->stream));
                 if (n->run_verbose)
-                    fprintf(stderr, "spdnn: resident launch (group sums): layers %d..%d, %d rows, %d groups\n", l, l + c - 1, n->carried, st.sums);
+                    fprintf(stderr, "spdnn: resident launch (group sums): layers %d..%d, %d rows, %d rows per workgroup, %d groups\n", l, l + c - 1, n->carried,
+                            sums_rows_per_workgroup(st.sums, n->carried, n->n_cu), st.sums);
                 st.r.resident_launches += 1;
             } else if (resident) {
                 ResidentLaunch rl{};
