@@ -4,6 +4,8 @@ Bar: active-row sets (categories) identical after every layer; fp32 activations 
 (the requirement is 1e-5 relative / 1e-6 absolute; accumulating in the reference's order makes
 equality attainable, so equality is what is asserted).
 """
+import re
+
 import numpy as np
 import pytest
 
@@ -699,7 +701,7 @@ def test_resident_launches_of_band_layers(gc, orc, monkeypatch, N, B, K, values,
         elif values == "general":
             v = (rng.uniform(-0.05, 0.2, size=len(v)) * (32.0 / K)).astype(np.float32)
         else:
-            v = np.full(len(v), 2.0 / K, dtype=np.float32)
+            v = np.full(len(v), 2.0 / K if values == "uniform" else values, dtype=np.float32)
         layers.append((rp, c, v))
     dens = np.where(rng.random(B) < 0.4, 0.8, 0.05).astype(np.float32)
     feats = ((rng.random((B, N), dtype=np.float32) < dens[:, None]) * rng.uniform(0.5, 2.0, size=(B, N))).astype(np.float32)
@@ -1790,24 +1792,26 @@ def test_reference_side_binding(gc, orc, tmp_path):
     assert np.array_equal(got, ref["categories"])
 
 
-@pytest.mark.parametrize("N,B,kind,rl", [
-    (512, 300, "radix", 4),      # 32 groups: half a wave's lanes without one
-    (1008, 777, "radix", 2),     # 63 groups, rows one at a time
-    (1024, 17000, "radix", 4),   # four rows per workgroup
-    (1024, 9000, "hub", 4),      # two rows per workgroup; lists of fewer than 32 inputs
-    (4096, 700, "common", 4),    # one neuron order for all layers
-    (4160, 130, "radix", 1),     # 260 groups, walked in segments of which the last is short
-    (8192, 300, "radix", 2),
-    (16400, 90, "radix", 1),     # 1025 groups: a second trip for one of them
-    (65520, 40, "hub", 4),       # 4095 groups and the zero behind them: the last 16-bit offset
-    (65536, 70, "radix", 4),     # 4096 groups
+@pytest.mark.parametrize("N,B,kind,rl,head,R", [
+    (512, 300, "radix", 4, "lists", 1),      # 32 groups: half a wave's lanes without one
+    (1008, 777, "radix", 2, "lists", 1),     # 63 groups
+    (1024, 17000, "radix", 4, "lists", 4),   # four rows per workgroup
+    (1024, 9000, "hub", 4, "lists", 2),      # two rows per workgroup; lists of fewer than 32 inputs
+    (4096, 700, "common", 4, "walk", 1),     # one neuron order for all layers
+    (4160, 130, "radix", 1, "lists", 1),     # 260 groups, a width that is not walked
+    (4352, 130, "radix", 1, "walk", 1),      # 272 groups
+    (8192, 300, "radix", 2, "walk", 1),
+    (16400, 90, "radix", 1, "lists", 1),     # 1025 groups: a second trip for one of them
+    (65520, 40, "hub", 4, "lists", 1),       # 4095 groups and the zero behind them: the last 16-bit offset
+    (65536, 70, "radix", 4, "walk", 1),      # 4096 groups
 ])
-def test_group_sums(gc, orc, monkeypatch, N, B, kind, rl):
+def test_group_sums(gc, orc, monkeypatch, capfd, N, B, kind, rl, head, R):
     """Layers of equal groups behind one another carry one column per group between a head launch and an expansion:
     counts, categories and activations against the oracle bit for bit, pruned and unpruned, whole and cut into calls, and
     the same with the launches that carry full columns."""
     print("group sums N=%d B=%d %s rl=%d" % (N, B, kind, rl), flush=True)
     monkeypatch.setenv("SPDNN_ROWS_PER_LANE", str(rl))
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
     rng = np.random.default_rng(N + B)
     if kind == "hub":
         base = [hub_block_csr(rng, N) for _ in range(2)]
@@ -1831,9 +1835,16 @@ def test_group_sums(gc, orc, monkeypatch, N, B, kind, rl):
             net.inspect()
             net.set_features_dense(feats)
             for prune in (True, False):
+                _launch_kinds(capfd)
                 r = net.run(prune=prune, collect_counts=True)
+                made = _launch_kinds(capfd)
                 if mode == "1":
                     assert r.resident_launches >= 1 and r.persistent_launches == 0 and r.fused_pairs == 0
+                    assert [k for k, _ in made] == ["head, " + head] + ["group sums"] * r.resident_launches
+                    if not prune:
+                        assert "%d rows per workgroup," % R in made[1][1]
+                else:
+                    assert not {"group sums", "head, " + head} & {k for k, _ in made}
                 assert [net.active_count(l) for l in range(L)] == want
                 assert np.array_equal(net.categories(), cats)
                 assert same_floats(net.activations(cats), ref["y"])
@@ -1877,19 +1888,47 @@ def test_transfers(gc, N, B, asked):
             net.set_features_dense(feats)
 
 
-@pytest.mark.parametrize("N,B,K,rl", [(1024, 1500, 32, 4), (512, 900, 16, 2), (256, 300, 8, 1), (768, 400, 12, 4), (1024, 700, 20, 4)])
-def test_resident_launches_in_tiles(gc, orc, monkeypatch, N, B, K, rl):
+def _launch_kinds(capfd):
+    """The launches of several layers and the heads of group sums that networks made with SPDNN_RUN_VERBOSE=1 have reported
+    since the last look: [(kind, {number behind each word})]."""
+    out = []
+    for line in capfd.readouterr().err.splitlines():
+        m = re.match(r"spdnn: (resident launch|group sums, head) \(([a-z ]+)\): (.*)", line)
+        if m:
+            out.append((m.group(2) if m.group(1) == "resident launch" else "head, " + m.group(2), m.group(3)))
+    return out
+
+
+@pytest.mark.parametrize("N,B,K,weight,rl", [(1024, 1500, 32, 0.0625, 4), (512, 900, 16, 0.125, 2), (256, 300, 8, 0.25, 1),
+                                             (768, 400, 12, 0.125, 4), (1024, 700, 20, 0.125, 4), (768, 520, 32, 0.0625, 2)])
+def test_resident_launches_in_tiles(gc, orc, monkeypatch, capfd, N, B, K, weight, rl):
     """Bands under one power-of-two weight run their resident launches on the matrix cores (lists of 48 steps and of fewer):
     the same checks as for bands of any weights."""
     monkeypatch.setenv("SPDNN_BAND_TILES", "2")
-    test_resident_launches_of_band_layers(gc, orc, monkeypatch, N, B, K, "uniform", rl)
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    test_resident_launches_of_band_layers(gc, orc, monkeypatch, N, B, K, weight, rl)
+    kinds = [k for k, _ in _launch_kinds(capfd)]
+    assert len(kinds) > 10 and set(kinds) == {"band tiles"}
+
+
+@pytest.mark.parametrize("N,B,kind", [(1024, 4100, "band tiles"), (768, 4100, "band tiles"), (1024, 3800, "band quads"), (512, 4100, "band quads")])
+def test_where_resident_launches_run_in_tiles_by_default(gc, monkeypatch, capfd, N, B, kind):
+    """By default from 768 neurons and sixteen rows for every compute unit."""
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    with gc.Network(N, B, 8, bias=-0.3) as net:
+        net.synth_layers(3, nnz_per_row=32, value=0.0625)
+        net.inspect()
+        net.synth_features(3, B, 0.5, 0.6)
+        net.run(prune=False)
+        assert _launch_kinds(capfd) == [(kind, "layers 0..7, %d rows, 16 rows per workgroup" % (-(-B // 256) * 256))]
 
 
 @pytest.mark.parametrize("N,B,kind", [(1024, 60000, "radix"), (16384, 6000, "radix"), (1024, 60000, "band")])
-def test_resident_launches_with_one_survivor_per_row_block(gc, orc, monkeypatch, N, B, kind):
+def test_resident_launches_with_one_survivor_per_row_block(gc, orc, monkeypatch, capfd, N, B, kind):
     """One row of every 256 lives on, the others die layer by layer, and nothing is compacted: workgroups of a row block
     whose survivor's workgroup has finished already still write their dead rows as zeros.  Against one launch per layer."""
     print("one survivor per row block N=%d B=%d %s" % (N, B, kind), flush=True)
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
     rng = np.random.default_rng(N)
     L = 24
     base = [radix_like_csr(rng, N, 16 << k) for k in range(3)] if kind == "radix" else [orc.gen_layer_csr(5, l, N) for l in range(3)]
@@ -1910,8 +1949,16 @@ def test_resident_launches_with_one_survivor_per_row_block(gc, orc, monkeypatch,
             y = net.activations(cats)
             assert (B + 255) // 256 <= want[-1] < B // 100 and len(set(want)) > 3
             for fuse in (0, 2, 5):
+                _launch_kinds(capfd)
                 r = net.run(prune=True, collect_counts=True, fuse_layers=fuse, compact_threshold=1e-6)
-                assert r.compactions == 0 and (r.resident_launches > 0 or N > 4096 or fuse < 5)
+                kinds = {k for k, _ in _launch_kinds(capfd)}
+                assert r.compactions == 0
+                if kind == "radix" and fuse == 0 and sums == "1":
+                    assert kinds == {"group sums", "head, walk" if N > 1024 else "head, lists"}
+                elif kind == "radix":
+                    assert kinds == ({"groups"} if N <= 1024 else set())
+                elif fuse == 5:
+                    assert kinds == {"band tiles" if sums == "1" else "band quads"}
                 assert [net.active_count(l) for l in range(L)] == want
                 assert np.array_equal(net.categories(), cats)
                 assert same_floats(net.activations(cats), y)
@@ -2179,3 +2226,50 @@ def test_the_expansion_of_group_sums_is_counted_and_timed(gc):
             r = net.run(prune=False, time_layers=True, **kw)
             assert (r.resident_launches, r.launches) == (1, launches)
             assert abs(net.layer_times()[kw.get("first_layer", 0):kw.get("n_layers", L)].sum() - r.ms_kernels) < 1e-3
+
+
+@pytest.mark.parametrize("N,B,rl,R,segment", [
+    (65536, 1100, 4, 4, 16),      # four rows of 4096 groups and the zero behind them: 131 KB of LDS; four trips
+    (65536, 600, 4, 2, 16),       # two rows
+    (65536, 8192, 1, 4, 256),     # the longest segments of the walk
+    (20480, 1100, 4, 4, 16),      # 1280 groups: a second trip for a quarter of the threads
+    (16640, 8000, 1, 4, 64),      # 1040 groups: one wave with a second trip, a last segment of a quarter of the others
+])
+def test_group_sums_of_large_launches(gc, orc, monkeypatch, capfd, N, B, rl, R, segment):
+    """Group sums with several rows per workgroup on layers with more groups than a workgroup has threads, and the walk's longer
+    segments: a part of the rows against the oracle, all of them against launches that carry full columns."""
+    print("large group sums N=%d B=%d" % (N, B), flush=True)
+    monkeypatch.setenv("SPDNN_ROWS_PER_LANE", str(rl))
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    rng = np.random.default_rng(N + B)
+    L, lo, hi, few = 4, 0.1, 0.8, 24
+    base = [radix_like_csr(rng, N, 16 << k) for k in range(2)]
+    layers = [base[l % 2] for l in range(L)]
+    ref = orc.infer(gc.synth_features_host(3, N, 0, few, lo, hi), layers, -0.4, prune=True)
+    assert 0 < len(ref["categories"]) < few
+    seen = []
+    for mode in ("1", "0"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", mode)
+        with gc.Network(N, B, L, bias=-0.4) as net:
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            net.inspect()
+            net.synth_features(3, B, lo, hi)
+            for prune in (False, True):
+                _launch_kinds(capfd)
+                net.run(prune=prune, collect_counts=True)
+                made = _launch_kinds(capfd)
+                if mode == "1":
+                    assert made[0][0] == "head, walk" and made[0][1].endswith("segments of %d" % segment)
+                    assert {k for k, _ in made[1:]} == {"group sums"}
+                    if not prune:
+                        assert "layers 1..3" in made[1][1] and "%d rows per workgroup," % R in made[1][1]
+                else:
+                    assert not made
+                cats = net.categories()
+                mine = cats[cats < few]
+                assert np.array_equal(mine, ref["categories"]) and same_floats(net.activations(mine), ref["y"])
+                ask = cats[::max(1, len(cats) // 700)]
+                seen.append(([net.active_count(l) for l in range(L)], cats, net.activations(ask)))
+    for counts, cats, y in seen[1:]:
+        assert counts == seen[0][0] and np.array_equal(cats, seen[0][1]) and same_floats(y, seen[0][2])
