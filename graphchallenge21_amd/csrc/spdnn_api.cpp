@@ -170,11 +170,17 @@ class CopyCrew {
   public:
     static constexpr int kParts = 16;
     static constexpr int kSpinUs = 50;
-    CopyCrew(JobPool* pool, int pieces, std::function<void(int, int)> copy)
+    // `most`: workers at most.  Seven and the calling thread keep up with the link where both sides' pages exist (features
+    // handed over: 120 MB 2.65 ms, 2.75 with fifteen; 25 MB 0.68 ms, 0.75) and in read-backs of less than 64 MiB (29 MB
+    // 0.71 ms, 0.77; 9 MB 0.29, 0.35), at half the processor time; larger ones into a fresh array need fifteen (240 MB
+    // 5.4 ms, 6.1 with seven; 590 MB 12.3, 13.5).
+    static int workers_in() { return 7; }
+    static int workers_out(size_t bytes) { return bytes < (size_t)64 << 20 ? 7 : kParts - 1; }
+    CopyCrew(JobPool* pool, int most, int pieces, std::function<void(int, int)> copy)
         : pieces_(pieces), copy_(std::move(copy)), done_(new std::atomic<int>[(size_t)pieces]) {
         for (int k = 0; k < pieces; ++k) done_[(size_t)k].store(0, std::memory_order_relaxed);
         if (pool) {
-            const int workers = std::min(kParts - 1, pool->size());
+            const int workers = std::min(most, pool->size());
             for (int w = 0; w < workers; ++w) {
                 { std::lock_guard<std::mutex> lk(m_); ++running_; }
                 try {
@@ -609,14 +615,15 @@ int ensure_device(spdnn_net* n) {
     return rc;
 }
 
-// Pinned slots for a transfer of `bytes` in units of `unit`: a quarter of it each, 16 MiB at most (or one unit, where that
-// is more).  At 16 MiB a slot takes the link 0.3 ms, against which the launch and the waits around it are small (590 MB
-// read back in 12.2 ms; with slots of 8 MiB 13.6).
+// Pinned slots for a transfer of `bytes` in units of `unit`: a quarter of it each, between 1 and 16 MiB (or one unit, where
+// that is more).  At 16 MiB a slot takes the link 0.3 ms, against which the launch and the waits around it are small (590
+// MB read back in 12.2 ms; with slots of 8 MiB 13.6); transfers of 1 MB are quicker in one or two pieces than in
+// four (1.2 MB 89 us against 99).
 // Where pinned memory is refused (or not wanted, SPDNN_PINNED_STAGING=0) the lease stays empty: such a transfer goes
 // between the caller's pageable memory and the device as the runtime does it.
 int lend_staging(spdnn_net* n, size_t bytes, size_t unit, StageLease* lease) {
     if (!n->pinned_staging) return SPDNN_OK;
-    size_t slot = std::min<size_t>(kStageMaxSlot, std::max<size_t>(bytes / kStageSlots, (size_t)256 << 10));
+    size_t slot = std::min<size_t>(kStageMaxSlot, std::max<size_t>(bytes / kStageSlots, (size_t)1 << 20));
     slot = (std::max(slot, unit) + 4095) & ~(size_t)4095;
     for (hipEvent_t& e : n->ev_stage)
         if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1627,7 +1634,7 @@ static int spdnn_set_features_dense_impl(spdnn_net* n, const float* rowmajor, in
         for (size_t p = c; p < end; p += lease.slot) pieces.push_back({p, std::min(lease.slot, end - p), p + lease.slot >= end});
     }
     {
-        CopyCrew crew(total >= kCrewMinBytes ? n->pool.get() : nullptr, (int)pieces.size(), [&](int k, int part) {
+        CopyCrew crew(total >= kCrewMinBytes ? n->pool.get() : nullptr, CopyCrew::workers_in(), (int)pieces.size(), [&](int k, int part) {
             copy_part(lease.at(k), (const char*)rowmajor + pieces[(size_t)k].at, pieces[(size_t)k].bytes, part);
         });
         const int K = (int)pieces.size();
@@ -2754,7 +2761,8 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         HIPCHK(hipStreamSynchronize(n->stream));
         return SPDNN_OK;
     }
-    CopyCrew crew((size_t)nrows * row_bytes >= kCrewMinBytes ? n->pool.get() : nullptr, K, [&](int k, int part) {
+    const size_t bytes = (size_t)nrows * row_bytes;
+    CopyCrew crew(bytes >= kCrewMinBytes ? n->pool.get() : nullptr, CopyCrew::workers_out(bytes), K, [&](int k, int part) {
         copy_part(rowmajor + (size_t)k * per * n->N, lease.at(k), (size_t)rows_in(k) * row_bytes, part);
     });
     auto ready = [&](int k) -> hipError_t {   // slot k's rows have arrived: handed to the crew
