@@ -257,7 +257,7 @@ class CopyCrew {
 // Pinned memory for transfers from and to a caller's memory: sets of four slots, lent to the network that transfers and
 // shared by all networks of the process.  What a new set costs is not the allocation (0.05 - 0.4 ms) but the host's
 // first touch of its pages, 0.4 ms per MiB: held by each network, a network's first read-back of 9 MB took 2.1 - 2.3 ms,
-// more than through pageable memory (0.76); out of a set that is there it takes 0.6.
+// more than through pageable memory (0.76); out of a set that is there it takes 0.37.
 // At most two sets stay here idle (two threads that transfer in turn find theirs), none with slots above kStageMaxSlot;
 // without a network in the process one is left, of kStageMaxRest bytes at most, for the next one.
 constexpr int kStageSlots = 4;
@@ -2268,7 +2268,9 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // While the counts still move a launch holds about 120 us of layers (an estimate: a read of four rows takes
                 // a CU's LDS 20 cycles for 64 groups): counting, the host's look, scan and repack behind a launch take 50 to
                 // 70 us, and workgroups whose rows have died leave by themselves.  Layers of 60000 x 1024, 30000 x 4096 and
-                // 12000 x 16384 with 25 us of layers at first: 422, 730 and 864 us; with 60 410, 730, 870; with 120 347, 617, 800.
+                // 12000 x 16384 with 25 us of layers at first: 422, 730 and 864 us; with 60 410, 730, 870; with 120 347, 617, 800.  Longer
+                // ones change little (measured later, with 120, 240, 480: 351, 344, 366 and 610, 583, 609 and 811, 820, 800, and 60000 x
+                // 65536 8.7, 8.15, 8.3 ms).
                 const double us = 1.0 + (double)n->carried * st.sums * 32.0 * 0.08 / ((double)n->n_cu * 2400.0);
                 int kmax = n->persist_layers;
                 if (opt.prune) kmax = std::min(kmax, std::max(st.c_prune, (int)(120.0 / us)));
