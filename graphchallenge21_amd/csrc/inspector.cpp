@@ -680,47 +680,44 @@ static void build_quad_form(int N, const std::vector<int32_t>& rowptr, const std
 // outputs merge to more than 48 of them.
 static void build_tile_form(int N, const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col, float value,
                             LayerPlan& plan) {
-    static_assert(kQuadMaxNeurons <= 1024, "a tile's inputs are a set of 1024 bits");
     const int nt = N / 16;
     uint32_t wbits;
     memcpy(&wbits, &value, 4);
-    plan.tile_rec.assign((size_t)nt * 96, 0u);
-    std::vector<uint32_t> recs((size_t)nt * 96, 0u);
+    std::vector<uint32_t>& recs = plan.tile_rec;
+    recs.assign((size_t)nt * 256, 0u);
     int steps = 0;
+    const int words = (N + 63) / 64;
     for (int c = 0; c < nt; ++c) {
-        uint64_t set[16] = {};      // the inputs of the tile's outputs; an input's step is its rank in the set
-        int before[16];
+        uint64_t set[(kTileMaxNeurons + 63) / 64] = {};   // the inputs of the tile's outputs; an input's step is its rank in the set
+        int before[(kTileMaxNeurons + 63) / 64];
         for (int j = 0; j < 16; ++j) {
             const int row = plan.out_at[(size_t)16 * c + j];
             for (int e = rowptr[row]; e < rowptr[row + 1]; ++e) set[col[e] >> 6] |= 1ull << (col[e] & 63);
         }
         int m = 0;
-        for (int w = 0; w < 16; ++w) {
+        for (int w = 0; w < words; ++w) {
             before[w] = m;
             m += __builtin_popcountll(set[w]);
         }
-        if (m < 1 || m > 48) return;
+        if (m < 1 || m > 48) return;   // (what there is of the form stays as room)
         steps = std::max(steps, m);
-        uint32_t* rec = &recs[(size_t)c * 96];
+        uint32_t* rec = &recs[(size_t)c * 256];
+        auto column = [&](int s) -> uint32_t& { return rec[((s & 3) * 16 + (s >> 2)) * 4 + 3]; };
         int s = 0;
-        for (int w = 0; w < 16; ++w)
+        for (int w = 0; w < words; ++w)
             for (uint64_t left = set[w]; left; left &= left - 1)
-                rec[s++] = (uint32_t)plan.in_pos[(size_t)(w * 64 + __builtin_ctzll(left))] * (uint32_t)kQuadColumnBytes;
-        for (; s < 48; ++s) rec[s] = rec[m - 1];
+                column(s++) = (uint32_t)plan.in_pos[(size_t)(w * 64 + __builtin_ctzll(left))] * (uint32_t)kQuadColumnBytes;
+        for (; s < 48; ++s) column(s) = column(m - 1);   // (behind the list the last column again, which no output uses)
+        for (int k = 0; k < 4; ++k) rec[(k * 16 + 15) * 4 + 3] = wbits;
         for (int j = 0; j < 16; ++j) {
             const int row = plan.out_at[(size_t)16 * c + j];
-            uint64_t use = 0;
             for (int e = rowptr[row]; e < rowptr[row + 1]; ++e) {
-                const int w = col[e] >> 6;
-                use |= 1ull << (before[w] + __builtin_popcountll(set[w] & ((1ull << (col[e] & 63)) - 1)));
+                const int w = col[e] >> 6, at = before[w] + __builtin_popcountll(set[w] & ((1ull << (col[e] & 63)) - 1));
+                rec[((at & 3) * 16 + j) * 4 + (at >> 4)] |= 1u << (8 * (at >> 2 & 3));
             }
-            rec[48 + j] = (uint32_t)use;
-            rec[64 + j] = (uint32_t)(use >> 32);
-            rec[80 + j] = wbits;
         }
     }
     plan.tile_steps = (steps + 3) / 4 * 4;
-    plan.tile_rec.swap(recs);
 }
 
 void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<int32_t>& col,
@@ -945,8 +942,8 @@ void inspect_layer(int N, const std::vector<int32_t>& rowptr, const std::vector<
         if (N <= kQuadMaxNeurons) build_quad_form(N, rowptr, col, val, plan);
         // (bands of other exact weights share resident launches with these in their QUAD form, which asks for plans at equal
         // distances: they keep the room)
-        if (N <= kQuadMaxNeurons && (N % 64) == 0 && plan.wmode == 0) build_tile_form(N, rowptr, col, plan.info.value, plan);
-        else if (N <= kQuadMaxNeurons && (N % 64) == 0 && plan.wmode == 1) plan.tile_rec.assign((size_t)N / 16 * 96, 0u);
+        if (N <= kTileMaxNeurons && plan.wmode == 0) build_tile_form(N, rowptr, col, plan.info.value, plan);
+        else if (N <= kQuadMaxNeurons && plan.wmode == 1) plan.tile_rec.assign((size_t)N / 16 * 256, 0u);
     } else if (force_kernel != SPDNN_KERNEL_GATHER && !(getenv("SPDNN_TILED") && atoi(getenv("SPDNN_TILED")) == 0) &&
                build_tiled_plan(N, rowptr, col, val, plan)) {
         plan.kernel = SPDNN_KERNEL_TILED;

@@ -17,6 +17,7 @@ namespace spdnn {
 constexpr int kTileOutputs = 1024;  // TILED: outputs per tile (16 waves x 64)
 constexpr int kPanelCols = 512;     // TILED: input columns staged in LDS at a time
 constexpr int kQuadMaxNeurons = 1024;  // BAND: widest layer that carries its QUAD form (two buffers of N x 16 rows in LDS)
+constexpr int kTileMaxNeurons = 2304;  // BAND: widest layer that carries its TILE form (N x 16 rows in LDS)
 constexpr int kQuadColumnBytes = 64;   // ... whose columns are 16 rows of 4 bytes: the form holds byte offsets
 
 struct LayerPlan {
@@ -80,9 +81,10 @@ struct LayerPlan {
     std::vector<float> quad_w;
     int quad_groups = 0;
     // ... and, under one exact weight, its TILE form, for the matrix cores: the sixteen outputs at band positions 16 c ..
-    // 16 c + 15 merge into one list of steps (K + 15 for a circulant band, 48 at most).  tile_rec [N/16][6][16]: the steps'
-    // input columns as byte offsets (three sixteens; behind the list the last one again), the steps each output uses as
-    // a 48-bit mask (low words, high words), the weight's bits sixteen times.  tile_steps 0: no such form, tile_rec is room.
+    // 16 c + 15 merge into one list of steps (K + 15 for a circulant band, 48 at most), four to an instruction.  tile_rec
+    // [N/16][64 lanes][4]: lane 16 k + i holds, as a byte for each of twelve instructions (words 0 .. 2), whether output i
+    // uses the instruction's step k, and in word 3 the input column of step k of instruction i, as the byte offset in a buffer
+    // of 16 rows per column (i < 12; behind the list the last column again) or, in lane 15 of each sixteen, the weight's bits.  tile_steps 0: no such form, tile_rec is room.
     std::vector<uint32_t> tile_rec;
     int tile_steps = 0;
     // BAND: neuron j sits at the same band position as an input and as an output (see

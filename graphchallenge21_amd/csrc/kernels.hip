@@ -2688,30 +2688,38 @@ __global__ __launch_bounds__(1024) void band_resident_kernel(ResidentArgs a) {
     if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
 }
 
-// The resident launch of BAND layers under one exact weight, on the matrix cores.  A wave owns 64 neighbouring band
-// positions as four tiles of sixteen; v_mfma_f32_16x16x1_4b adds one step of all four tiles' merged lists to sixteen
-// rows: D[row][output] += x[row] * w[output], one rounding per product as in the multiply-add of the other kernels, and
-// a step an output does not use enters it with weight 0.  So the order of every sum stays ascending input index, and
-// the bits stay those of the oracle - which a form that adds several products in one instruction would not promise.
-// The lanes of tile b = lane / 16 read the step's column from LDS (sixteen rows, 64 bytes) and hold output lane % 16's
-// use mask; the steps' columns lie in three registers across the tile's lanes and enter the address add by DPP.
-// The rows stay in place: a wave's 64 x 16 results wait in its registers until every wave has read the layer's inputs,
-// so the buffer is N x 16 floats and two workgroups of 1024 threads share a CU (which is what limits a thread to 64
-// registers).  1024 neurons, 32 entries, 39700 rows: 62 us a layer against 68 of the QUAD form; the matrix cores are
-// busy 48 % of the cycles (48 instructions a tile and layer, a third of them on zeros), the LDS 38 %, over half of that
-// in bank conflicts of the steps' columns, the vector ALUs 35 %.  The frame around it - rows in and out, stamps, early
-// exit - is band_resident_kernel's.
-template <int NS>   // steps (a multiple of 4), 0: as the launch says
-__global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArgs a) {
+// The resident launch of BAND layers under one exact weight, on the matrix cores.  Sixteen outputs at neighbouring band
+// positions (a tile) merge into one list of steps in ascending input index; v_mfma_f32_16x16x4 takes four steps of a tile
+// for sixteen rows: D[output][row] += sum over k of use[output][k] * x[k][row].  Its four products are added one after the
+// other in the order of k, each sum rounded (what the hardware does, tested bit for bit against the oracle over the whole
+// range of accepted values), a step an output does not use enters with 0, and the one weight scales the finished sum
+// inside the epilogue's fma, which is exact for a power of two: the bits are those of the other kernels.
+// A wave owns T tiles.  Lane 16 k + i reads row i (rows 2 i and 2 i + 1 where a workgroup keeps two halves of sixteen,
+// H = 2) of the column of step k - the column's offset lies in lane i' of each sixteen for instruction i' and enters the
+// address add by DPP - and turns a byte of its tile's record into the use of output i.  A record of 16 bytes per lane and
+// tile is requested a layer ahead, into the registers whose layer has just been read.  Results: lane 16 k + i holds
+// outputs 4 k .. 4 k + 3 of rows i, so the sixteen lanes of a store write one whole column, free of bank conflicts like
+// the reads (as D[row][output], sixteen lanes wrote sixteen columns at the same bank: 3.5 of 12 us).  The rows stay in
+// place: the results wait in registers until every wave has read the layer's inputs.
+// What bounds it: the issue of matrix and vector instructions together - the vector instructions between the products do
+// not hide behind them on this chip (13.8 ns per product and SIMD alone, 15.9 with the address and the use, one of each for
+// two products with H = 2; 19.3 with H = 1) - so the steps come in batches: G instructions' addresses, reads and uses, then
+// the products of the batch before.  1024 neurons, 32 entries: 60000 rows 62.6 us a layer, 40000 39.4 (80 and 54 with
+// v_mfma_f32_16x16x1_4b, four tiles to an instruction), 4096 rows, sixteen to a workgroup, 5.1 (6.8); two thirds of
+// the products are useful, that is 63 TFLOP/s of multiply-adds in a layer, 94 of the 140 the instruction reaches.  The
+// frame around it - rows in and out, stamps, early exit - is band_resident_kernel's.
+template <int G, int NB, int T, int H>   // a tile's steps: NB batches of G instructions of four; tiles per wave; halves of sixteen rows
+__global__ __launch_bounds__(1024, 4) void band_tile_resident_kernel(ResidentArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int sh_alive[3];
-    __shared__ int sh_last[16];
-    typedef float f32x16_t __attribute__((ext_vector_type(16)));
-    constexpr int R = 16, PARTS = 4;
-    using GU = const __attribute__((address_space(1))) uint32_t*;
+    constexpr int R = 16 * H, PARTS = R / 4, COL = R * 4;   // COL: bytes of a column
+    __shared__ int sh_last[R];
+    using V = typename VecOf<H>::type;
+    using GQ = const __attribute__((address_space(1))) u32x4_t*;
+    using GI = const __attribute__((address_space(1))) int32_t*;
     using GB = const __attribute__((address_space(1))) unsigned char*;
     publish_counts(a.pub);
-    const int t = (int)threadIdx.x, lane = t & 63, nthr = a.N;   // (launched with N threads)
+    const int t = (int)threadIdx.x, lane = t & 63, nthr = (int)blockDim.x;
     const int RB = 64 * a.rl;
     const unsigned nwg = gridDim.x;
     const unsigned wg = (nwg % 8u) == 0u ? (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u : blockIdx.x;
@@ -2723,90 +2731,112 @@ __global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArg
         if (__syncthreads_or(alive) == 0) return;
     }
     const size_t blkf = (size_t)a.N * RB;
+    constexpr int IO = T * H;   // (launched with N / T threads a tile: 16-byte pieces of the rows per thread)
     {
         const float* __restrict__ gin = block_base(a.first_in, rb, blkf) + rin;
-        float4 v[4];
+        float4 v[IO];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < IO; ++u) {
             const int idx = t + u * nthr;
             v[u] = *reinterpret_cast<const float4*>(gin + (size_t)(idx / PARTS) * RB + (idx % PARTS) * 4);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) *reinterpret_cast<float4*>(smem + (size_t)(t + u * nthr) * 16) = v[u];
+        for (int u = 0; u < IO; ++u) *reinterpret_cast<float4*>(smem + (size_t)(t + u * nthr) * 16) = v[u];
     }
     if (t < 3) sh_alive[t] = 0;
     if (t < R) sh_last[t] = -1;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    // this lane's words of its tile's record (requested a layer ahead), and the columns its four tiles' outputs go to
-    // (requested as their layer begins)
-    const uint32_t rec_off = ((uint32_t)(t >> 4) * 96u + (uint32_t)(lane & 15)) * 4u;
-    const uint32_t dst_off = ((uint32_t)wave * 64u + (uint32_t)(lane & 15)) * 4u;
-    uint32_t rec_next[6];
-    auto request = [&](int j) {
-        const GB rec = (GB)a.tile_rec + (long long)j * a.quad_stride;
+    const uint32_t rec_off = ((uint32_t)(wave * T) * 64u + (uint32_t)lane) * 16u;
+    const uint32_t dst_off = ((uint32_t)(wave * T) * 16u + (uint32_t)(lane >> 4) * 4u + (uint32_t)(lane & 3)) * 4u;
+    u32x4_t rec[T];
+    auto request = [&](int b, int j) { rec[b] = *(GQ)((GB)a.tile_rec + (long long)j * a.quad_stride + b * 1024 + rec_off); };
 #pragma unroll
-        for (int i = 0; i < 6; ++i) rec_next[i] = *(GU)(rec + i * 64 + rec_off);
-    };
-    request(0);
-    const int steps = NS ? NS : a.ngroups;
-    uint32_t last_nz = 0;   // per row of this lane, a byte: the last layer that left it nonzero, from 1 (kTileMaxLayers at most)
+    for (int b = 0; b < T; ++b) request(b, 0);
+    int last_nz[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) last_nz[h] = -1;
     bool all_dead = false;
+    unsigned char* const mine = smem + (lane & 15) * (H * 4);   // this lane's rows of column 0
     ring_barrier<1>();
     for (int j = 0; j < a.nlayers; ++j) {
-        const unsigned char* const in = smem + (lane & 15) * 4;
-        unsigned char* const out = smem + (lane >> 4) * 16;
-        uint32_t rec[5], dst[4];
+        const float wu = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)rec[0].w, 15));
+        uint32_t dst[T];
 #pragma unroll
-        for (int i = 0; i < 5; ++i) rec[i] = rec_next[i];
-        const uint32_t wbits = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec_next[5]);
+        for (int b = 0; b < T; ++b) dst[b] = (uint32_t)*(GI)((GB)a.quad_dst + (long long)j * a.quad_stride + b * 64 + dst_off);
+        const int ahead = min(j + 1, a.nlayers - 1);
+        f32x4_t acc[T][H] = {};
+        float x[2][G][H], use[2][G];
+        auto fetch = [&](int i, float (&xv)[G][H], float (&uv)[G]) {
+            const int b = i / NB;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) dst[b] = *(GU)((GB)a.quad_dst + (long long)j * a.quad_stride + b * 64 + dst_off);
-        if (j + 1 < a.nlayers) request(j + 1);   // in flight under this layer's arithmetic
-        f32x16_t acc = {};
-#pragma unroll
-        for (int s0 = 0; s0 < 48; s0 += 4) {
-            if (s0 < steps) {
-#pragma unroll
-                for (int s = s0; s < s0 + 4; ++s) {
-                    const float x = *reinterpret_cast<const float*>(in + row_lane(rec[s >> 4], s & 15));
-                    const uint32_t use = (uint32_t)((int32_t)(rec[3 + (s >> 5)] << (31 - (s & 31))) >> 31);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(x, __uint_as_float(use & wbits), acc, 0, 0, 0);
-                }
+            for (int g = 0; g < G; ++g) {
+                const int m = (i % NB) * G + g;
+                const V v = *reinterpret_cast<const V*>(mine + row_lane(rec[b].w * (uint32_t)H, m));
+                vec_to_arr<H>(v, xv[g]);
             }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int m = (i % NB) * G + g;
+                uv[g] = (float)((rec[b][m >> 2] >> (8 * (m & 3))) & 0xffu);
+            }
+        };
+        fetch(0, x[0], use[0]);
+#pragma unroll
+        for (int i = 0; i < T * NB; ++i) {
+            if (i + 1 < T * NB) fetch(i + 1, x[(i + 1) & 1], use[(i + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+            if ((i + 1) % NB == NB - 1) request((i + 1) / NB, ahead);   // (this layer's has just been used for the last time)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+                    acc[i / NB][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(use[i & 1][g], x[i & 1][g][h], acc[i / NB][h], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // register 4 b + q: row 4 (lane / 16) + q of output lane % 16 of tile b
-        float top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        // register q of tile b: output 4 (lane / 16) + q, row H (lane % 16) + h
+        float top[H];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
+        for (int h = 0; h < H; ++h) {
+            top[h] = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                acc[4 * b + q] = relu_clamp(acc[4 * b + q] + a.bias, a.clampv);
-                top[q] = nz_merge(top[q], acc[4 * b + q]);
-            }
+            for (int b = 0; b < T; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    acc[b][h][q] = relu_clamp(__builtin_fmaf(acc[b][h][q], wu, a.bias), a.clampv);
+                    top[h] = nz_merge(top[h], acc[b][h][q]);
+                }
         }
         float any = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (top[q] > 0.0f) last_nz = (last_nz & ~(255u << (8 * q))) | ((uint32_t)(j + 1) << (8 * q));
-            any = nz_merge(any, top[q]);
+        for (int h = 0; h < H; ++h) {
+            if (top[h] > 0.0f) last_nz[h] = j;
+            any = nz_merge(any, top[h]);
         }
         if (__ballot(any > 0.0f ? 1 : 0) != 0ull && lane == 0) sh_alive[j % 3] = 1;
         ring_barrier<1>();   // all of the layer's inputs have been read
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-            *reinterpret_cast<float4*>(out + dst[b] * (uint32_t)(R * 4)) = float4{acc[4 * b], acc[4 * b + 1], acc[4 * b + 2], acc[4 * b + 3]};
+        for (int b = 0; b < T; ++b) {
+            const uint32_t col = dst[b] * (uint32_t)COL;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float y[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h) y[h] = acc[b][h][q];
+                *reinterpret_cast<V*>(mine + row_lane(col, q)) = arr_to_vec<H>(y);
+            }
+        }
         ring_barrier<1>();
         const int some = sh_alive[j % 3];
         if (t == 0) sh_alive[(j + 2) % 3] = 0;
         if (some == 0 && a.bias <= 0.0f) { all_dead = true; break; }   // zero rows stay zero
     }
-    // the last layer that left each of the 16 rows nonzero: the largest over the lanes that hold the row's outputs
+    // the last layer that left each of the rows nonzero: the largest over the lanes that hold the row's outputs
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        int v = (int)((last_nz >> (8 * q)) & 255u) - 1;
-#pragma unroll
-        for (int sft = 1; sft < 16; sft <<= 1) v = max(v, __shfl_xor(v, sft, 64));
-        if ((lane & 15) == 0 && v >= 0) atomicMax(&sh_last[(lane >> 4) * 4 + q], v);
+    for (int h = 0; h < H; ++h) {
+        int v = last_nz[h];
+        v = max(v, __shfl_xor(v, 16, 64));
+        v = max(v, __shfl_xor(v, 32, 64));
+        if (lane < 16 && v >= 0) atomicMax(&sh_last[lane * H + h], v);
     }
     __syncthreads();
     const int last_alive = t < R ? sh_last[t] : -1;
@@ -2817,7 +2847,7 @@ __global__ __launch_bounds__(1024, 8) void band_tile_resident_kernel(ResidentArg
     float* const o_h1 = to_c ? a.buf_c.half[1] : a.buf_a.half[1];
     float* __restrict__ gout = ((rb & 1) ? o_h1 : o_h0) + (size_t)(rb >> 1) * blkf + rin;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < IO; ++u) {
         const int idx = t + u * nthr;
         float4 v{};
         if (!all_dead) v = *reinterpret_cast<const float4*>(smem + (size_t)idx * 16);
@@ -3515,28 +3545,54 @@ hipError_t launch_band_resident(const ResidentLaunch& a, int wmode, hipStream_t 
     return hipGetLastError();
 }
 
+// Two halves share addresses and uses, but a workgroup of one half leaves twice as many workgroups: 1024 neurons 4096 rows
+// 5.1 us a layer against 8.1 with two, 6000 rows 9.7 against 8.2, 40000 46 against 39.  Up to 18 rows for every CU (of 1024
+// neurons) launches keep to one half; that loses from 16 to 18 (9.6 against 8.1), where tests look for it.  Wider
+// bands have no room for two halves (N x 16 floats; 2304 neurons are 144 KiB).
+int band_tile_rows(int N, int rows, int n_cu) {
+    if (N % 256 != 0 || N < 256 || N > 9 * 256) return 0;
+    return N <= 1024 && (long long)rows * N > 18ll * 1024 * n_cu ? 32 : 16;
+}
+
+template <int G, int NB, int T, int H>
+static hipError_t launch_band_tile_inst(const ResidentArgs& k, int rows, hipStream_t s) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(band_tile_resident_kernel<G, NB, T, H>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (T == 4 ? 1024 : T * 256) * H * 64);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((band_tile_resident_kernel<G, NB, T, H>), dim3((unsigned)(rows / (16 * H))), dim3((unsigned)(k.N / T * 4)),
+                       (size_t)k.N * H * 64, s, k);
+    return hipGetLastError();
+}
+template <int G, int NB>
+static hipError_t launch_band_tile_steps(const ResidentArgs& k, int rows, bool halves, hipStream_t s) {
+    switch (k.N <= 1024 ? 4 : k.N / 256) {
+        case 4: return halves ? launch_band_tile_inst<G, NB, 4, 2>(k, rows, s) : launch_band_tile_inst<G, NB, 4, 1>(k, rows, s);
+        case 5: return launch_band_tile_inst<G, NB, 5, 1>(k, rows, s);
+        case 6: return launch_band_tile_inst<G, NB, 6, 1>(k, rows, s);
+        case 7: return launch_band_tile_inst<G, NB, 7, 1>(k, rows, s);
+        case 8: return launch_band_tile_inst<G, NB, 8, 1>(k, rows, s);
+        case 9: return launch_band_tile_inst<G, NB, 9, 1>(k, rows, s);
+        default: return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s) {
-    // host-side shape checks: as launch_band_resident, and the waves' 64 band positions
-    if (a.nlayers < 1 || a.nlayers > kTileMaxLayers || !a.tile_rec || !a.quad_dst || (a.quad_stride % 4) != 0 || !a.first_in || !a.buf_a || !a.buf_c ||
+    // host-side shape checks: what the kernel's LDS buffer, its tiles and threads and its plan stream assume
+    const int wg_rows = band_tile_rows(a.N, a.rows, a.n_cu);
+    if (a.nlayers < 1 || !a.tile_rec || !a.quad_dst || (a.quad_stride % 16) != 0 || !a.first_in || !a.buf_a || !a.buf_c ||
         a.buf_a == a.buf_c || !a.active || a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0 ||
-        band_resident_rows(a.N) != 16 || (a.N % 64) != 0 || a.ngroups < 4 || a.ngroups > 48 || (a.ngroups % 4) != 0)
+        wg_rows == 0 || a.ngroups < 4 || a.ngroups > 48 || (a.ngroups % 4) != 0)
         return hipErrorInvalidValue;
     ResidentArgs k{};
     k.nlayers = a.nlayers; k.first_in = a.first_in; k.buf_a = a.buf_a; k.buf_c = a.buf_c; k.active = a.active;
     k.N = a.N; k.ngroups = a.ngroups; k.rl = a.rl; k.stamp0 = a.stamp0; k.prev_stamp = a.prev_stamp; k.check_dead = a.check_dead;
     k.bias = a.bias; k.clampv = a.clampv; k.pub = a.publish;
     k.quad_dst = a.quad_dst; k.quad_stride = a.quad_stride; k.tile_rec = a.tile_rec;
-    dim3 grid((unsigned)(a.rows / 16)), block((unsigned)a.N);
-#define SPDNN_TILE_RESIDENT(NS)                                                                                            \
-    do {                                                                                                                   \
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(band_tile_resident_kernel<NS>),   \
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);        \
-        if (attr != hipSuccess) return attr;                                                                               \
-        hipLaunchKernelGGL(band_tile_resident_kernel<NS>, grid, block, (size_t)a.N * 16 * 4, s, k);                        \
-    } while (0)
-    if (a.ngroups == 48) SPDNN_TILE_RESIDENT(48); else SPDNN_TILE_RESIDENT(0);
-#undef SPDNN_TILE_RESIDENT
-    return hipGetLastError();
+    const bool halves = wg_rows == 32;
+    // (36 steps: bands of 20 entries, 35; bands of 8 and of 16 take 23 and 31)
+    if (a.ngroups <= 24) return launch_band_tile_steps<3, 2>(k, a.rows, halves, s);
+    if (a.ngroups <= 32) return launch_band_tile_steps<4, 2>(k, a.rows, halves, s);
+    if (a.ngroups <= 36) return launch_band_tile_steps<3, 3>(k, a.rows, halves, s);
+    return launch_band_tile_steps<4, 3>(k, a.rows, halves, s);
 }
 
 int count_stamp_partial_words() { return kCountTicket + 1; }

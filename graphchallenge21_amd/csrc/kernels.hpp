@@ -286,6 +286,7 @@ struct ResidentLaunch {
     const int32_t* quad_dst;
     long long quad_stride;
     const uint32_t* tile_rec = nullptr;   // launch_band_tile_resident: the TILE form, at the same distances (ngroups: its steps)
+    int n_cu = 256;
 };
 // The same for TILED layers in their ROWTILE form (any sparsity pattern): `nlayers` consecutive such layers of one
 // weight mode, the R rows of a workgroup in LDS from the first layer to the last, every thread computing whole outputs
@@ -304,10 +305,10 @@ int band_resident_rows(int N);
 // rows a workgroup keeps (16 or 4), 0 if the shape does not fit: two buffers of (N + 1) x R floats in LDS
 // (N <= 1024: 16 rows, N <= 4096: 4) and one (group, row) item per thread of 1024
 int resident_rows_per_workgroup(int N, int ngroups);
-// Their TILE form (one exact weight): sixteen outputs by sixteen rows on the matrix cores.  kTileMaxLayers layers per
-// launch at most: a byte per row holds the last layer that left it nonzero.
-constexpr int kTileMaxLayers = 254;
+// Their TILE form (one exact weight, up to kTileMaxNeurons neurons): sixteen outputs by sixteen rows on the matrix cores
 hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s);
+// rows such a workgroup keeps (16 or 32), 0 = the shape does not fit
+int band_tile_rows(int N, int rows, int n_cu);
 hipError_t launch_block_resident(const ResidentLaunch& a, hipStream_t s);
 
 // counts[i] = number of rows r < rows with stamps[r] >= stamp_lo + i, for i in [0, n): with bias <= 0 a

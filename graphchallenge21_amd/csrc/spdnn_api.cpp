@@ -1978,21 +1978,27 @@ struct ResidentSig {
     int rows = 0;    // rows a workgroup keeps
     bool operator==(const ResidentSig& o) const { return ok == o.ok && full == o.full && ngroups == o.ngroups && wmode == o.wmode; }
 };
+// Where bands of one exact weight run as tiles.  Up to 1024 neurons against QUAD, 32 entries, us per layer: 1024 neurons
+// 300 rows 4.8 and 5.7, 2000 4.9 and 5.6, 4352 9.6 and 11.9, 40000 39 and 54, 60000 63 and 80; 768 neurons 3.7 and 4.5
+// at 300, 30 and 41 at 40000; 512 2.7 and 3.3 at 300, 8.3 and 10.8 at 16000, 30 and 37 at 60000; 256 15 and 19 at 60000.
+// Launches of 12 to 16 rows (20, below 768 neurons) for every CU stay with QUAD, where they have always run and the
+// tests look for them (1024 neurons, 3840 rows: 6.3 against 5.1).  Wider bands have no QUAD form; tiles against one walk
+// per layer: 2048 neurons 9.4 and 9.0 at 300 rows, 9.7 and 18 at 4096, 136 and 197 at 60000; 1536 neurons 103 and 148.
+static bool tiles_by_size(const spdnn_net* n) {
+    const int cu = n->n_cu;
+    return n->N > 1024 || n->carried < 12 * cu || n->carried >= (n->N >= 768 ? 16 : 20) * cu;
+}
 static ResidentSig resident_sig(const spdnn_net* n, int l, bool tiles = true) {   // tiles = false: not the TILE form
     const LayerPlan& p = n->layers[(size_t)l];
     ResidentSig g;
     if (p.kernel == SPDNN_KERNEL_BAND && p.alt_ngroups > 0) { g.ok = 1; g.full = p.alt_full ? 1 : 0; g.ngroups = p.alt_ngroups; }
     else if (p.kernel == SPDNN_KERNEL_BLOCK && p.wmode == 0) { g.ok = 1; g.full = p.blk_full ? 1 : 0; g.ngroups = p.ngroups; }
     else if (p.kernel == SPDNN_KERNEL_TILED && !p.rt_ent.empty() && n->rowtile_mode) { g.ok = 2; g.wmode = p.wmode; }
-    // Band tiles need two workgroups on a CU to hide a layer's latency, and waves enough in each: 60 layers of 8, 20 and 32
-    // entries against QUAD, times faster: 1024 neurons, 60000 rows 1.05, 1.25, 1.05, 6000 rows 0.99, 1.19, 1.01, 700 rows
-    // 0.89, 1.11, 0.95; 768 neurons 1.18, 1.41, 1.08 and 1.09, 1.31, 1.01 and 0.90, 1.14, 0.92; 512 neurons 0.97, 1.14, 0.96
-    // and 0.86, 1.02, 0.80 and 1.05, 1.25, 0.84.  So: from 768 neurons and a workgroup of 16 rows for every CU.
     else if (tiles && p.kernel == SPDNN_KERNEL_BAND && p.tile_steps > 0 && n->band_resident_mode &&
-             (n->tile_mode == 2 || (n->tile_mode == 1 && n->N >= 768 && n->carried >= 16 * n->n_cu))) { g.ok = 4; g.ngroups = p.tile_steps; }
+             (n->tile_mode == 2 || (n->tile_mode == 1 && tiles_by_size(n)))) { g.ok = 4; g.ngroups = p.tile_steps; }
     else if (p.kernel == SPDNN_KERNEL_BAND && p.quad_groups > 0 && n->band_resident_mode) { g.ok = 3; g.ngroups = p.quad_groups; g.wmode = p.wmode == 2 ? 2 : 1; }
     if (g.ok) {
-        g.rows = g.ok == 1 ? resident_rows_per_workgroup(n->N, g.ngroups) : g.ok == 2 ? rowtile_resident_rows(n->N) : band_resident_rows(n->N);
+        g.rows = g.ok == 1 ? resident_rows_per_workgroup(n->N, g.ngroups) : g.ok == 2 ? rowtile_resident_rows(n->N) : g.ok == 4 ? band_tile_rows(n->N, n->carried, n->n_cu) : band_resident_rows(n->N);
         if (g.rows == 0 || n->RB % g.rows != 0) g.ok = 0;
     }
     return g;
@@ -2295,7 +2301,6 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 const int room = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
                 // layers from l0 on that one launch takes in the form g, of `most`
                 auto run_of = [&](int l0, const ResidentSig& g, int most, bool tiles) {
-                    if (g.ok == 4) most = std::min(most, kTileMaxLayers);
                     int k = 1;
                     while (k < most && resident_sig(n, l0 + k, tiles) == g && (g.ok < 3 || band_plans_equidistant(n, l0, l0 + k, g.ok == 4))) ++k;
                     return k;
@@ -2450,7 +2455,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             } else if (resident) {
                 ResidentLaunch rl{};
                 rl.table = n->d_table + l; rl.nlayers = c; rl.first_in = in; rl.buf_a = n->A; rl.buf_c = n->C; rl.active = n->d_active;
-                rl.N = n->N; rl.ngroups = rsig.ngroups; rl.rows = n->carried; rl.rl = n->rl; rl.full = rsig.full;
+                rl.n_cu = n->n_cu; rl.N = n->N; rl.ngroups = rsig.ngroups; rl.rows = n->carried; rl.rl = n->rl; rl.full = rsig.full;
                 rl.stamp0 = stamp0; rl.prev_stamp = prev_stamp; rl.check_dead = check_dead; rl.bias = n->bias; rl.clampv = n->clampv;
                 rl.publish = st.pub;
                 if (rsig.ok >= 3) {

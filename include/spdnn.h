@@ -97,7 +97,7 @@ typedef struct spdnn_run_options {
                                     (RadiX-Net layers) or are TILED layers, at most 4096 neurons wide, or are BAND layers
                                     at most 1024 neurons wide (from 6 layers on, from 16 at 16384 rows and more; under one
                                     power-of-two weight, 768 neurons or wider and with 16 rows for every compute unit,
-                                    from 4 on and 254 at most, on the matrix cores): a workgroup keeps 16, 8 or 4 rows
+                                    from 4 on, on the matrix cores): a workgroup keeps 16, 8 or 4 rows
                                     in LDS through up to 64 layers (SPDNN_RESIDENT=0: never; SPDNN_BAND_RESIDENT=0: not
                                     the BAND layers);
                                     three or more consecutive layers with such a BLOCK form, of any width up to 65536, carry

@@ -1911,6 +1911,39 @@ def test_resident_launches_in_tiles(gc, orc, monkeypatch, capfd, N, B, K, weight
     assert len(kinds) > 10 and set(kinds) == {"band tiles"}
 
 
+@pytest.mark.parametrize("N,B,K,w,rows", [(256, 200, 8, 2.0 ** -24, 16), (1024, 5000, 32, 2.0 ** -24, 32), (512, 9500, 16, -0.5, 32),
+                                          (1280, 300, 20, 2.0 ** 21, 16), (2048, 200, 32, 2.0 ** -24, 16), (2304, 300, 12, -2.0 ** 21, 16)])
+def test_tiles_add_in_ascending_order_over_the_whole_range(gc, orc, monkeypatch, capfd, N, B, K, w, rows):
+    """Every number of tiles per wave at its narrowest and widest, both numbers of rows per workgroup, lists of all
+    lengths.  Features of both signs from 2^-100 up to where a sum reaches the clamp, neighbours that cancel to
+    their last bits: a sum in another order, or rounded once for several inputs, would show."""
+    print("tiles N=%d B=%d K=%d w=%g" % (N, B, K, w), flush=True)
+    monkeypatch.setenv("SPDNN_BAND_TILES", "2")
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    rng = np.random.default_rng(N + K)
+    L = 3
+    layers = [orc.gen_layer_csr(17, l, N, K, w) for l in range(L)]
+    top = 4 - int(np.log2(abs(w)))
+    mag = np.ldexp(rng.uniform(1.0, 2.0, size=(B, N)), np.where(rng.random((B, N)) < 0.8, rng.integers(top - 12, top, size=(B, N)), rng.integers(-100, top, size=(B, N))))
+    feats = (mag * rng.choice([-1.0, 1.0], size=(B, N)) * (rng.random((B, N)) < 0.8)).astype(np.float32)
+    feats[:, 1::2] = np.where(rng.random((B, N // 2)) < 0.3, -np.nextafter(feats[:, 0::2], np.float32(0)), feats[:, 1::2])
+    ref = orc.infer(feats, layers, -2.0 ** -30, prune=False, keep=set(range(L)))
+    first = ref["kept"][0][1]
+    assert np.mean((first > 0) & (first < 32)) > 0.2     # (most of what the first layer adds up can be seen)
+    with gc.Network(N, B, L, bias=-2.0 ** -30) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        every = np.arange(B, dtype=np.int32)
+        for n in (1, 2, 3):      # (one layer alone runs as the walk: the same bits)
+            _launch_kinds(capfd)
+            net.run(prune=False, n_layers=n, fuse_layers=L)
+            if n > 1:
+                assert _launch_kinds(capfd) == [("band tiles", "layers 0..%d, %d rows, %d rows per workgroup" % (n - 1, -(-B // 256) * 256, rows))]
+            assert same_floats(net.activations(every), ref["kept"][n - 1][1])
+
+
 @pytest.mark.parametrize("N,B,kind", [(1024, 4100, "band tiles"), (768, 4100, "band tiles"), (1024, 3800, "band quads"), (512, 4100, "band quads")])
 def test_where_resident_launches_run_in_tiles_by_default(gc, monkeypatch, capfd, N, B, kind):
     """By default from 768 neurons and sixteen rows for every compute unit."""
