@@ -2146,20 +2146,44 @@ __global__ __launch_bounds__(64 * RL) void sums_walk_kernel(
     if (nz > 0.0f) active[(size_t)rb * RB + wave * 64 + lane] = stamp;
 }
 
-// Group sums written out: column dst[16 g + o] of the full layout is group g's, for every output o of the group.
-template <int RL>
+// Group sums written out: column dst[16 g + o] of the full layout is group g's, for every output o of the group.  LISTED:
+// of the rows that a scan found (see SumsRows), row blocks behind their last one are left alone - a run whose rows
+// died inside one launch writes out what is left of them in the same pass (60000 x 1024 with 2093 rows left: 7 us, 55 with
+// every row carried written out).
+template <int RL, bool LISTED>
 __global__ __launch_bounds__(256) void sums_expand_kernel(Feat sums, Feat full, const int32_t* __restrict__ dst, int N,
-                                                          int ngroups, int gpw) {
+                                                          int ngroups, int gpw, SumsRows rows) {
     using V = typename VecOf<RL>::type;
     constexpr int RB = 64 * RL;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int rb = blockIdx.x, loff = (threadIdx.x & 63) * RL;
-    const float* __restrict__ in = block_base(sums, rb, (size_t)ngroups * RB) + loff;
+    const float* in[RL];
+    if (LISTED) {
+        const int cnt = rows.count[0];
+        if (rb * RB >= cnt) return;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) {
+            const int k = rb * RB + loff + r;
+            const int src = k < cnt ? rows.src[k] : -1;
+            in[r] = src >= 0 ? block_base(sums, src / RB, (size_t)ngroups * RB) + src % RB : nullptr;
+            if (blockIdx.y == 0 && wave == 0) rows.gid_out[k] = src >= 0 ? rows.gid[k] : -1;
+        }
+    } else {
+        in[0] = block_base(sums, rb, (size_t)ngroups * RB) + loff;
+    }
     float* __restrict__ out = block_base(full, rb, (size_t)N * RB) + loff;
     const int g0 = (blockIdx.y * 4 + wave) * gpw;
     const int g1 = min(ngroups, g0 + gpw);
     for (int g = g0; g < g1; ++g) {
-        const V v = *reinterpret_cast<const V*>(in + (size_t)g * RB);
+        V v;
+        if (LISTED) {
+            float x[RL];
+#pragma unroll
+            for (int r = 0; r < RL; ++r) x[r] = in[r] ? in[r][(size_t)g * RB] : 0.0f;
+            v = arr_to_vec<RL>(x);
+        } else {
+            v = *reinterpret_cast<const V*>(in[0] + (size_t)g * RB);
+        }
 #pragma unroll
         for (int o = 0; o < 16; ++o) {
             const int d = dst[(size_t)g * 16 + o];
@@ -2303,6 +2327,286 @@ __global__ __launch_bounds__(1024) void sums_resident_kernel(SumsArgs a) {
         *reinterpret_cast<V*>(gout + (size_t)g * RB) = v;
     }
     if (t < R && last_alive >= 0) a.active[row0 + t] = a.stamp0 + last_alive;
+}
+
+// The same for launches of many rows, and where rows die: a workgroup takes S rows (up to 128 KiB of sums) in fours
+// (quads).  An item is a group and a quad; consecutive threads take consecutive quads of a group, so that a wave reads
+// pieces of 16 Q bytes (Q quads) instead of 16 at random places, which is what bounds these kernels: 4096 groups with 8 rows
+// take 22 us a layer, with 4 rows in sums_resident_kernel's two buffers 30; a layer of 60160 x 65536 with its rows in and out
+// 1.36 ms against 1.57.  The sums wait in registers until every input has been read, so one buffer does (where two fit,
+// two, and one barrier less); when rows have died the others close up as they are written, so that a launch's cost follows
+// the rows that are left without the host: 120 layers of 60000 x 1024 0.32 ms against 0.35, 30000 x 4096 0.52 against
+// 0.61, 12000 x 16384 0.74 against 0.83, 40 of 60000 x 65536 7.0 against 8.7.  A compaction between two such launches is made by the
+// second as it loads its rows (SumsRows).  Inputs are added and the one weight applied once, in the epilogue's fma, as
+// in the band walk; the order is ascending.  With a dozen rows left a layer is latency: 0.95 us, of which
+// 0.4 are the LDS reads and 0.3 the adds.
+struct SumsSlabArgs {
+    SumsArgs s;
+    int S, rows;   // rows per workgroup (a multiple of 4), carried rows
+    SumsRows from;
+};
+
+// a place's byte offset (number of the group x 16, from half HI of a list's word) in a buffer of Q quads per group, from `base`
+template <int HI> __device__ __forceinline__ uint32_t slab_place(uint32_t word, uint32_t Q, uint32_t base) {
+    uint32_t r;
+    if (HI) asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(r) : "v"(word), "v"(Q), "v"(base));
+    else asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(r) : "v"(word), "v"(Q), "v"(base));
+    return r;
+}
+
+constexpr int kSlabRows = 256;   // rows per workgroup at most
+
+template <int TRIPS, bool DB>
+__global__ __launch_bounds__(1024, 4) void sums_slab_kernel(SumsSlabArgs p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ uint16_t sh_row[2][kSlabRows];       // the row (of the slab) in each slot
+    __shared__ int16_t sh_last[kSlabRows + 4];      // per row: the last layer that left it nonzero, -1 before the first (then a place for slots without a row)
+    __shared__ unsigned long long sh_cols[kSlabLayers];
+    __shared__ float sh_wu[kSlabLayers];
+    constexpr int W = kSlabRows / 64, B = TRIPS == 1 ? 8 : 4;   // B: reads of a batch
+    using GQ = const __attribute__((address_space(1))) u32x4_t*;
+    const SumsArgs& a = p.s;
+    publish_counts(a.pub);
+    const int t = (int)threadIdx.x, lane = t & 63, nthr = (int)blockDim.x;
+    const int RB = 64 * a.rl, G = a.ngroups;
+    const unsigned nwg = gridDim.x;
+    const unsigned wg = (nwg % 8u) == 0u ? (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u : blockIdx.x;
+    const int row0 = (int)wg * p.S;
+    const int here = min(p.S, p.rows - row0);       // rows of this workgroup
+    const size_t blkf = (size_t)G * RB;
+    const bool dies = a.bias <= 0.0f;               // zero rows stay zero
+    // sets of slots or rows as bit masks of 64, the same in every wave
+    auto rank = [&](const unsigned long long (&m)[W], int i) {   // how many of m lie before i
+        int r = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const unsigned long long part = w < (i >> 6) ? m[w] : w == (i >> 6) ? m[w] & ((1ull << (i & 63)) - 1ull) : 0ull;
+            r += (int)__popcll(part);
+        }
+        return r;
+    };
+    auto total = [&](const unsigned long long (&m)[W]) {
+        int r = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) r += (int)__popcll(m[w]);
+        return r;
+    };
+    unsigned long long alive[W];
+    const bool stamped = a.check_dead && a.prev_stamp != 0;
+    const int listed = p.from.src ? p.from.count[0] : p.rows;
+    auto starts = [&](int r) { return r < here && row0 + r < listed && (!stamped || a.active[row0 + r] >= a.prev_stamp); };
+#pragma unroll
+    for (int w = 0; w < W; ++w) alive[w] = w * 64 < here ? __ballot(starts(w * 64 + lane) ? 1 : 0) : 0ull;
+    int n = total(alive);                           // slots in use
+    int Q = (n + 3) >> 2, cur = 0;
+    if (starts(t)) sh_row[0][rank(alive, t)] = (uint16_t)t;
+    for (int i = t; i < p.S; i += nthr) sh_last[i] = -1;
+    if (p.from.src && t < here) p.from.gid_out[row0 + t] = row0 + t < listed ? p.from.gid[row0 + t] : -1;
+    __syncthreads();
+    // thread t takes quad t % Q of the groups t / Q, t / Q + step, ... (a thread behind the last of them none)
+    int q = 0, g0 = 0, step = 1, trips = 0;
+    int slot_row[W], row[4];                        // rows of slots 64 w + lane, and of this thread's quad
+    auto share = [&]() {
+        const int per = nthr / Q;                   // groups of a trip
+        q = t % Q; g0 = t / Q; step = per;
+        trips = (G + per - 1) / per;
+        if (g0 >= per) g0 = G;
+#pragma unroll
+        for (int w = 0; w < W; ++w) slot_row[w] = w * 64 + lane < n ? (int)sh_row[cur][w * 64 + lane] : kSlabRows;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) row[r] = 4 * q + r < n ? (int)sh_row[cur][4 * q + r] : kSlabRows;
+    };
+    if (n > 0) {
+        share();
+        // in: slot k of group g at 4 Q g + k; slots behind the last row are zero, as is the place behind the groups
+        const int per = nthr / (4 * Q), k = t % (4 * Q), at = t / (4 * Q);
+        const float* from = nullptr;
+        if (k < n) {
+            int r = row0 + (int)sh_row[0][k];
+            if (p.from.src) r = p.from.src[r];
+            from = block_base(a.yin, r / RB, blkf) + r % RB;
+        }
+        if (at < per) {
+            for (int g = at; g <= G; g += 8 * per) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = from && g + u * per < G ? from[(size_t)(g + u * per) * RB] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (g + u * per <= G) *reinterpret_cast<float*>(smem + (uint32_t)((g + u * per) * 4 * Q + k) * 4u) = v[u];
+            }
+        }
+    }
+    u32x4_t next[4];
+    auto request = [&](GQ cols, int g) {
+        const int gg = min(g, G - 1);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) next[c] = cols[(size_t)c * G + gg];
+    };
+    // (the layers' entries of the table through LDS: a scalar load inside the loop would be waited for with the next LDS read)
+    for (int i = t; i < a.nlayers; i += nthr) {
+        sh_cols[i] = (unsigned long long)a.table[i].sum_cols;
+        sh_wu[i] = a.table[i].wu;
+    }
+    auto uniform = [&](unsigned long long v) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+        return (GQ)(((unsigned long long)hi << 32) | lo);
+    };
+    __syncthreads();
+    GQ cols_here = uniform(sh_cols[0]), cols_next = uniform(sh_cols[min(1, a.nlayers - 1)]);
+    request(cols_here, g0);
+    uint32_t in = 0u, out = DB ? (uint32_t)(G + 1) * (uint32_t)p.S * 4u : 0u;   // byte offsets of the buffers
+    const uint32_t lds0 = (uint32_t)(size_t)((__attribute__((address_space(3))) unsigned char*)smem);
+    for (int j = 0; n > 0 && j < a.nlayers; ++j) {
+        const unsigned long long cols_ahead = sh_cols[min(j + 2, a.nlayers - 1)];
+        const float wu = sh_wu[j];
+        // Whether rows have died is looked at in the first layers and in every eighth (0.3 us of 1.6 with 12 rows of 64
+        // groups), behind the layer's first barrier or, with two buffers and one barrier, for the layer before (whose marks
+        // are read here and used behind the sums; other waves may have marked rows for this layer already).
+        const bool look = dies && (j < 8 || (j & 7) == 0) && (!DB || j > 0);
+        int seen[W];
+        auto marks = [&]() {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                seen[w] = -1;
+                if (w * 64 < n) seen[w] = (int)sh_last[slot_row[w]];
+            }
+        };
+        if (DB && look) marks();
+        const uint32_t base = lds0 + in + (uint32_t)q * 16u;
+        float y[TRIPS][4];
+        float nz[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int trip = 0; trip < TRIPS; ++trip) {
+            if (trip < trips) {
+                u32x4_t list[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) list[c] = next[c];
+                if (trip + 1 < trips) request(cols_here, g0 + (trip + 1) * step);
+                else request(cols_next, g0);
+                if (g0 + trip * step < G) {
+                    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    float x[2][B][4];
+                    auto fetch = [&](int c, float (&v)[B][4]) {
+#pragma unroll
+                        for (int k = 0; k < B; k += 2) {
+                            const uint32_t d = list[(c * B + k) >> 3][((c * B + k) & 7) >> 1];
+                            lds_read<4>(slab_place<0>(d, (uint32_t)Q, base), v[k]);
+                            lds_read<4>(slab_place<1>(d, (uint32_t)Q, base), v[k + 1]);
+                        }
+                    };
+                    fetch(0, x[0]);
+#pragma unroll
+                    for (int c = 0; c < 32 / B; ++c) {
+                        if (c + 1 < 32 / B) fetch(c + 1, x[(c + 1) & 1]);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int k = 0; k < B; ++k)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[r] += x[c & 1][k][r];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        y[trip][r] = relu_clamp(__builtin_fmaf(acc[r], wu, a.bias), a.clampv);
+                        nz[r] = nz_merge(nz[r], y[trip][r]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (nz[r] > 0.0f) sh_last[row[r]] = (int16_t)j;
+        if (!DB) {
+            ring_barrier<1>();   // every input of the layer has been read, and every row that is nonzero marked
+            if (look) marks();
+        }
+        int m = n;
+        if (look) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) alive[w] = w * 64 < n ? __ballot((w * 64 + lane < n && seen[w] >= (DB ? j - 1 : j)) ? 1 : 0) : 0ull;
+            m = total(alive);
+        }
+        const int Q2 = (m + 3) >> 2;
+        const bool fewer = Q2 < Q;
+        unsigned char* const to = smem + out;
+        if (fewer) {
+            // the rows that are left move together: each result goes to its row's new slot
+            if (t < n) {
+                bool keeps = false;
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (w == (t >> 6)) keeps = (alive[w] >> (t & 63)) & 1ull;
+                if (keeps) sh_row[cur ^ 1][rank(alive, t)] = sh_row[cur][t];
+            }
+            int slot[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = 4 * q + r;
+                bool keeps = false;
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (w == (k >> 6)) keeps = (alive[w] >> (k & 63)) & 1ull;
+                slot[r] = keeps ? rank(alive, k) : -1;
+            }
+#pragma unroll
+            for (int trip = 0; trip < TRIPS; ++trip) {
+                const int g = g0 + trip * step;
+                if (trip < trips && g < G) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (slot[r] >= 0) *reinterpret_cast<float*>(to + (uint32_t)(g * Q2 * 4 + slot[r]) * 4u) = y[trip][r];
+                }
+            }
+            const int pad = 4 * Q2 - m;   // slots behind the last row
+            for (int g = t; pad > 0 && g < G; g += nthr)
+                for (int k = 0; k < pad; ++k) *reinterpret_cast<float*>(to + (uint32_t)(g * Q2 * 4 + m + k) * 4u) = 0.0f;
+        } else {
+#pragma unroll
+            for (int trip = 0; trip < TRIPS; ++trip) {
+                const int g = g0 + trip * step;
+                if (trip < trips && g < G)
+                    *reinterpret_cast<float4*>(to + (uint32_t)(g * Q + q) * 16u) = float4{y[trip][0], y[trip][1], y[trip][2], y[trip][3]};
+            }
+        }
+        if (t < Q2) *reinterpret_cast<float4*>(to + (uint32_t)(G * Q2 + t) * 16u) = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        ring_barrier<1>();
+        if (fewer) {
+            n = m;
+            Q = Q2;
+            cur ^= 1;
+            if (n > 0) {
+                share();
+                request(cols_next, g0);
+            }
+        }
+        if (DB) { const uint32_t u = in; in = out; out = u; }
+        cols_here = cols_next; cols_next = uniform(cols_ahead);
+    }
+    // out: every row of the slab, those that died as zeros
+    __syncthreads();
+    for (int i = t; i < here; i += nthr) {
+        const int last = sh_last[i];
+        if (last >= 0) a.active[row0 + i] = a.stamp0 + last;
+    }
+    uint16_t* const slot_of = sh_row[cur ^ 1];
+    for (int i = t; i < here; i += nthr) slot_of[i] = 0xffffu;
+    __syncthreads();
+    if (t < n) slot_of[sh_row[cur][t]] = (uint16_t)t;
+    __syncthreads();
+    const int quads = here >> 2, per = nthr / quads, k = t % quads, at = t / quads;
+    if (at < per) {
+        float* const dst = block_base(a.yout, (row0 + 4 * k) / RB, blkf) + (row0 + 4 * k) % RB;
+        uint32_t from[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) from[r] = slot_of[4 * k + r];
+        for (int g = at; g < G; g += per) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = from[r] != 0xffffu ? *reinterpret_cast<const float*>(smem + in + ((uint32_t)(g * Q) * 4u + from[r]) * 4u) : 0.0f;
+            *reinterpret_cast<float4*>(dst + (size_t)g * RB) = float4{v[0], v[1], v[2], v[3]};
+        }
+    }
 }
 
 // The resident launch of TILED layers: block_resident_kernel's frame (R rows of a workgroup in LDS through all layers
@@ -3832,32 +4136,36 @@ hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s) {
 }
 
 hipError_t launch_sums_expand(const Feat& sums, const Feat& full, const int32_t* dst, int N, int ngroups, int nblk, int rl,
-                              hipStream_t s) {
-    if (N <= 0 || ngroups <= 0 || ngroups > N || nblk <= 0 || !sums || !full || sums == full || !dst) return hipErrorInvalidValue;
+                              const SumsRows& rows, hipStream_t s) {
+    if (N <= 0 || ngroups <= 0 || ngroups > N || nblk <= 0 || !sums || !full || sums == full || !dst ||
+        (rows.src && (!rows.gid || !rows.count || !rows.gid_out)))
+        return hipErrorInvalidValue;
     int gpw = 8;
     while (gpw > 1 && (long long)nblk * ((ngroups + 4 * gpw - 1) / (4 * gpw)) < 2048) gpw >>= 1;
     dim3 grid(nblk, (ngroups + 4 * gpw - 1) / (4 * gpw)), block(256);
     if (grid.y > 65535) return hipErrorInvalidValue;
+#define SPDNN_EXPAND(RL)                                                                                                       \
+    do {                                                                                                                       \
+        if (rows.src) hipLaunchKernelGGL((sums_expand_kernel<RL, true>), grid, block, 0, s, sums, full, dst, N, ngroups, gpw, rows); \
+        else hipLaunchKernelGGL((sums_expand_kernel<RL, false>), grid, block, 0, s, sums, full, dst, N, ngroups, gpw, rows);   \
+    } while (0)
     switch (rl) {
-        case 4: hipLaunchKernelGGL(sums_expand_kernel<4>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
-        case 2: hipLaunchKernelGGL(sums_expand_kernel<2>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
-        case 1: hipLaunchKernelGGL(sums_expand_kernel<1>, grid, block, 0, s, sums, full, dst, N, ngroups, gpw); break;
+        case 4: SPDNN_EXPAND(4); break;
+        case 2: SPDNN_EXPAND(2); break;
+        case 1: SPDNN_EXPAND(1); break;
         default: return hipErrorInvalidValue;
     }
+#undef SPDNN_EXPAND
     return hipGetLastError();
 }
 
 template <int R>
-static hipError_t launch_sums_resident_r(const SumsLaunch& a, int nthr, hipStream_t s) {
-    SumsArgs k{};
-    k.table = a.table; k.nlayers = a.nlayers; k.yin = a.yin; k.yout = a.yout; k.active = a.active; k.ngroups = a.ngroups; k.rl = a.rl;
-    k.stamp0 = a.stamp0; k.prev_stamp = a.prev_stamp; k.check_dead = a.check_dead; k.bias = a.bias; k.clampv = a.clampv;
-    k.pub = a.publish;
+static hipError_t launch_sums_resident_r(const SumsArgs& k, int rows, int nthr, hipStream_t s) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(sums_resident_kernel<R>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024);
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(sums_resident_kernel<R>, dim3((unsigned)(a.rows / R)), dim3((unsigned)nthr),
-                       (size_t)(a.ngroups + 1) * R * 8, s, k);
+    hipLaunchKernelGGL(sums_resident_kernel<R>, dim3((unsigned)(rows / R)), dim3((unsigned)nthr),
+                       (size_t)(k.ngroups + 1) * R * 8, s, k);
     return hipGetLastError();
 }
 
@@ -3870,15 +4178,65 @@ int sums_rows_per_workgroup(int ngroups, int rows, int n_cu) {
     return R;
 }
 
+// trips of a workgroup of nthr threads over G groups with Q quads of rows
+static int slab_trips(int G, int Q, int nthr) { return Q > nthr ? INT_MAX : (G + nthr / Q - 1) / (nthr / Q); }
+
+// Below four rows for every CU sums_resident_kernel's two rows or one spread over more CUs (1024 groups, 512 rows: 2.6 us a
+// layer against 4.3 in quads).  Without pruning from 128 rows per CU up: smaller launches keep the workgroups that
+// the tests look for (1024 neurons, 17152 rows).  As many rows per workgroup as make the fewest rounds.
+int sums_slab_rows(int ngroups, int rows, int n_cu, bool prune) {
+    if (rows < 4 * n_cu || (!prune && rows < 128 * n_cu)) return 0;
+    int most = std::min(kSlabRows, 32768 / ngroups) & ~3;
+    while (most > 4 && slab_trips(ngroups, most / 4, 1024) > 8) most -= 4;
+    const int rounds = (rows + most * n_cu - 1) / (most * n_cu);
+    return std::min(most, ((rows + rounds * n_cu - 1) / (rounds * n_cu) + 3) & ~3);
+}
+
+double sums_layer_us(int ngroups, int rows, int n_cu, bool prune) {
+    const int S = sums_slab_rows(ngroups, rows, n_cu, prune);
+    if (!S) return 1.0 + (double)rows * ngroups * 32.0 * 0.08 / ((double)n_cu * 2400.0);   // (a read of four rows takes a CU's LDS 20 cycles for 64 groups)
+    const int Q = S / 4, items = ngroups * Q, wgs = (rows + S - 1) / S;
+    const double read = (Q == 1 ? 2.5 : Q == 2 ? 1.8 : Q < 8 ? 1.5 : 1.15) * items * 32 * 16 / 128.0 / 2400.0;   // 16 bytes an item and read, 128 a cycle
+    const int at_once = std::max(1, std::min(1024 / std::max(64, std::min(1024, items)), (int)(160 * 1024 / ((size_t)(ngroups + 1) * S * 4))));
+    return ((wgs + n_cu * at_once - 1) / (n_cu * at_once)) * (0.7 + std::min(at_once, (wgs + n_cu - 1) / n_cu) * read);
+}
+
+template <int TRIPS, bool DB>
+static hipError_t launch_sums_slab(const SumsSlabArgs& p, int nthr, hipStream_t s) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(sums_slab_kernel<TRIPS, DB>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((sums_slab_kernel<TRIPS, DB>), dim3((unsigned)((p.rows + p.S - 1) / p.S)), dim3((unsigned)nthr),
+                       (size_t)(p.s.ngroups + 1) * p.S * (DB ? 8 : 4), s, p);
+    return hipGetLastError();
+}
+
 hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s) {
-    // host-side shape checks: what the 16-bit lists and the two LDS buffers assume
+    // host-side shape checks: what the 16-bit lists and the LDS buffers assume
     if (a.nlayers < 1 || !a.table || !a.yin || !a.yout || a.yin == a.yout || !a.active || a.ngroups <= 0 || a.ngroups > 4096 ||
         a.rows <= 0 || (a.rl != 1 && a.rl != 2 && a.rl != 4) || (a.rows % (64 * a.rl)) != 0)
         return hipErrorInvalidValue;
+    SumsArgs k{};
+    k.table = a.table; k.nlayers = a.nlayers; k.yin = a.yin; k.yout = a.yout; k.active = a.active; k.ngroups = a.ngroups; k.rl = a.rl;
+    k.stamp0 = a.stamp0; k.prev_stamp = a.prev_stamp; k.check_dead = a.check_dead; k.bias = a.bias; k.clampv = a.clampv;
+    k.pub = a.publish;
+    if (const int S = sums_slab_rows(a.ngroups, a.rows, a.n_cu, a.prune != 0)) {
+        if (a.rows_from.src && (!a.rows_from.gid || !a.rows_from.count || !a.rows_from.gid_out || a.prev_stamp != 0)) return hipErrorInvalidValue;
+        const SumsSlabArgs p{k, S, a.rows, a.rows_from};
+        const int nthr = std::min(1024, std::max((a.ngroups * (S / 4) + 63) / 64 * 64, (S + 63) / 64 * 64));
+        const int trips = slab_trips(a.ngroups, S / 4, nthr);
+        const bool db = (size_t)(a.ngroups + 1) * S * 8 <= 132 * 1024;
+        if (trips > 8 || a.nlayers > kSlabLayers) return hipErrorInvalidValue;
+        if (trips <= 1) return db ? launch_sums_slab<1, true>(p, nthr, s) : launch_sums_slab<1, false>(p, nthr, s);
+        if (trips <= 2) return db ? launch_sums_slab<2, true>(p, nthr, s) : launch_sums_slab<2, false>(p, nthr, s);
+        if (trips <= 4) return db ? launch_sums_slab<4, true>(p, nthr, s) : launch_sums_slab<4, false>(p, nthr, s);
+        return launch_sums_slab<8, false>(p, nthr, s);
+    }
+    if (a.rows_from.src) return hipErrorInvalidValue;
     const int nthr = sums_threads(a.ngroups);
     const int R = sums_rows_per_workgroup(a.ngroups, a.rows, a.n_cu);
-    return R == 4 ? launch_sums_resident_r<4>(a, nthr, s) : R == 2 ? launch_sums_resident_r<2>(a, nthr, s)
-                                                                   : launch_sums_resident_r<1>(a, nthr, s);
+    return R == 4 ? launch_sums_resident_r<4>(k, a.rows, nthr, s) : R == 2 ? launch_sums_resident_r<2>(k, a.rows, nthr, s)
+                                                                           : launch_sums_resident_r<1>(k, a.rows, nthr, s);
 }
 
 hipError_t launch_scan_active(const int32_t* active, const int32_t* gid, int rows, int stamp, int32_t* count,

@@ -164,6 +164,12 @@ hipError_t launch_block(const BlockLaunch& a, hipStream_t s);
 hipError_t launch_sums_head(const BlockLaunch& a, hipStream_t s);
 int sums_walk_segment(int nblk, int ngroups);
 struct LayerDesc;   // (a.wmode 0; a.dst is not used)
+// Rows taken from where a scan found them, what a repack in front of the launch would do: row k is row src[k] of the
+// input, for k < count[0] (zero from there on), and gid_out[k] becomes gid[k] (-1).  src nullptr: the rows as they lie.
+struct SumsRows {
+    const int32_t *src = nullptr, *gid = nullptr, *count = nullptr;
+    int32_t* gid_out = nullptr;
+};
 struct SumsLaunch {
     const LayerDesc* table;       // device pointer to the entry of the launch's first layer
     int nlayers;
@@ -171,14 +177,20 @@ struct SumsLaunch {
     int32_t* active;
     int ngroups, rows, rl;        // rows: carried rows (whole row blocks)
     int stamp0, prev_stamp, check_dead;
-    int n_cu;
+    int n_cu, prune;
     float bias, clampv;
     Publish publish;
+    SumsRows rows_from;           // (launches of sums_slab_kernel, prev_stamp 0)
 };
 hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s);
 int sums_rows_per_workgroup(int ngroups, int rows, int n_cu);
+// ... of sums_slab_kernel, which such a launch runs where this is not 0
+constexpr int kSlabLayers = 128;   // layers of such a launch at most
+int sums_slab_rows(int ngroups, int rows, int n_cu, bool prune);
+// about what a layer of such a launch takes, in microseconds
+double sums_layer_us(int ngroups, int rows, int n_cu, bool prune);
 hipError_t launch_sums_expand(const Feat& sums, const Feat& full, const int32_t* dst, int N, int ngroups, int nblk, int rl,
-                              hipStream_t s);
+                              const SumsRows& rows, hipStream_t s);
 
 // ------------------------------------------------------------------------------------------
 // Several layers per launch ("persistent" launches): the per-layer decomposition - many segments

@@ -1916,7 +1916,9 @@ static hipError_t launch_layer(spdnn_net* n, int l, const Feat& in, const Feat& 
 // a failed launch ends the wait: asking puts a marker into the queue, which between two short
 // layers costs as much as a layer.  The wait is bounded: after count_timeout_ms without the counts
 // of one layer (a kernel that never finishes) the call gives up with SPDNN_E_DEVICE.
-static int wait_counts(spdnn_net* n, int l0, int c) {
+// idle: the device has nothing queued behind the launch whose counts these are - what a sleep here oversleeps, it waits
+// (0.1 ms behind each of the first launches of group sums of 60000 x 65536).
+static int wait_counts(spdnn_net* n, int l0, int c, bool idle) {
     volatile int32_t* h = n->h_counts;
     for (int j = l0; j < l0 + c; ++j) {
         if (h[j] >= 0) continue;
@@ -1927,7 +1929,8 @@ static int wait_counts(spdnn_net* n, int l0, int c) {
             auto now = std::chrono::steady_clock::now();
             if (now - t_start < std::chrono::microseconds(300)) continue;  // short layers: poll as fast as possible
             // behind a long layer nothing is lost by sleeping between looks: the device has its next launch queued
-            std::this_thread::sleep_for(std::chrono::microseconds(50));
+            if (idle && now - t_start < std::chrono::milliseconds(20)) std::this_thread::yield();
+            else std::this_thread::sleep_for(std::chrono::microseconds(50));
             now = std::chrono::steady_clock::now();
             if (now - t0 < std::chrono::milliseconds(100)) continue;
             t0 = now;
@@ -2107,7 +2110,9 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     // the group sums that n->cur holds, written out for whatever reads the full columns next: a launch that counts as part
     // of the layer that computed them
     size_t expansions = 0;
-    auto expand_sums = [&]() -> hipError_t {
+    bool closed_up = false;   // the expansion has left the rows that are alive, and only those
+    bool gather = false;   // the rows of n->cur are to be taken from where the last scan found them (a compaction that the next launch makes)
+    auto expand_sums = [&](bool compact = false) -> hipError_t {   // compact: the rows the last scan found, and only those
         const LayerPlan& p = n->layers[(size_t)n->cur_layer - 1];
         const DevLayer& d = n->dl[(size_t)n->cur_layer - 1];
         const Feat full = (n->cur == n->A) ? n->C : n->A;
@@ -2119,9 +2124,17 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             n->ev_layer.push_back(x);
         }
         if (opt.time_layers && (e = hipEventRecord(n->ev_layer[ev], n->stream)) != hipSuccess) return e;
+        SumsRows rows;
+        if (compact) { rows.src = n->d_alive_src; rows.gid = n->d_alive_gid; rows.count = n->d_count; rows.gid_out = n->d_gid_tmp; }
         e = launch_sums_expand(n->cur, full, p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst, n->N, st.sums, n->carried / n->RB,
-                               n->rl, n->stream);
+                               n->rl, rows, n->stream);
         if (e != hipSuccess) return e;
+        if (compact) {
+            std::swap(n->d_gid, n->d_gid_tmp);
+            n->gid_dirty = true;
+            n->last_stamp = 0;
+            n->blocks_skipped = false;
+        }
         n->cur = full;
         st.sums = 0;
         st.r.launches += 1;
@@ -2135,7 +2148,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
         std::function<void()> f;
         ~AtEnd() { f(); }
     } at_end{[&] {
-        if (st.sums != 0 && n->carried > 0 && expand_sums() != hipSuccess) n->have_features = false;
+        if (st.sums != 0 && n->carried > 0 && (gather || expand_sums() != hipSuccess)) n->have_features = false;
     }};
     auto save = [&]() {
         State s = st;
@@ -2271,14 +2284,12 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             const bool chain = st.sums != 0;
             const bool head = sums_on && !chain && takes_sums(l + 1) && takes_sums(l + 2);
             if (chain) {
-                // While the counts still move a launch holds about 120 us of layers (an estimate: a read of four rows takes
-                // a CU's LDS 20 cycles for 64 groups): counting, the host's look, scan and repack behind a launch take 50 to
-                // 70 us, and workgroups whose rows have died leave by themselves.  Layers of 60000 x 1024, 30000 x 4096 and
-                // 12000 x 16384 with 25 us of layers at first: 422, 730 and 864 us; with 60 410, 730, 870; with 120 347, 617, 800.  Longer
-                // ones change little (measured later, with 120, 240, 480: 351, 344, 366 and 610, 583, 609 and 811, 820, 800, and 60000 x
-                // 65536 8.7, 8.15, 8.3 ms).
-                const double us = 1.0 + (double)n->carried * st.sums * 32.0 * 0.08 / ((double)n->n_cu * 2400.0);
+                // While the counts still move a launch holds about 120 us of layers (counting, the host's look, scan and repack
+                // behind it take 40 to 60 us)
+                const double us = sums_layer_us(st.sums, n->carried, n->n_cu, opt.prune != 0);
                 int kmax = n->persist_layers;
+                const int slab_rows = sums_slab_rows(st.sums, n->carried, n->n_cu, opt.prune != 0);
+                if (slab_rows) kmax = std::min(kmax, kSlabLayers);
                 if (opt.prune) kmax = std::min(kmax, std::max(st.c_prune, (int)(120.0 / us)));
                 kmax = std::max(1, std::min(kmax, last - l + 1));
                 while (c < kmax && takes_sums(l + c)) ++c;
@@ -2443,14 +2454,20 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 else if (n->run_verbose)
                     fprintf(stderr, "spdnn: group sums, head (lists): layer %d, %d rows, %d groups\n", l, n->carried, b.ngroups);
             } else if (chain) {
+                const int slab = sums_slab_rows(st.sums, n->carried, n->n_cu, opt.prune != 0);
                 SumsLaunch sl{};
                 sl.table = n->d_table + l; sl.nlayers = c; sl.yin = in; sl.yout = out; sl.active = n->d_active; sl.ngroups = st.sums;
                 sl.rows = n->carried; sl.rl = n->rl; sl.stamp0 = stamp0; sl.prev_stamp = prev_stamp; sl.check_dead = check_dead;
-                sl.n_cu = n->n_cu; sl.bias = n->bias; sl.clampv = n->clampv; sl.publish = st.pub;
+                sl.n_cu = n->n_cu; sl.prune = opt.prune ? 1 : 0; sl.bias = n->bias; sl.clampv = n->clampv; sl.publish = st.pub;
+                if (gather) { sl.rows_from.src = n->d_alive_src; sl.rows_from.gid = n->d_alive_gid; sl.rows_from.count = n->d_count; sl.rows_from.gid_out = n->d_gid_tmp; }
                 HIPCHK(launch_sums_resident(sl, n->stream));
+                if (gather) {
+                    std::swap(n->d_gid, n->d_gid_tmp);
+                    gather = false;
+                }
                 if (n->run_verbose)
                     fprintf(stderr, "spdnn: resident launch (group sums): layers %d..%d, %d rows, %d rows per workgroup, %d groups\n", l, l + c - 1, n->carried,
-                            sums_rows_per_workgroup(st.sums, n->carried, n->n_cu), st.sums);
+                            slab ? slab : sums_rows_per_workgroup(st.sums, n->carried, n->n_cu), st.sums);
                 st.r.resident_launches += 1;
             } else if (resident) {
                 ResidentLaunch rl{};
@@ -2526,7 +2543,13 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                                           n->d_alive_gid, n->stream));
                 HIPCHK(hipMemcpyAsync(n->d_counts + l, n->d_count, 4, hipMemcpyDeviceToDevice, n->stream));
             }
-            if (fused_count && group) {
+            // (behind a head the next launch skips the rows that died by itself: nobody needs their number before that)
+            const bool look_later = head && opt.prune && sums_slab_rows(st.sums, n->carried, n->n_cu, true) != 0;
+            if (fused_count && group && look_later) {
+                if (polled && st.pub.n > 0) recs.push_back({(int)(st.pub.src - n->d_counts), st.pub.n, -1});
+                st.pub = Publish{};
+                st.count_pending = true;
+            } else if (fused_count && group) {
                 // The rows the layers of the launch left active, from the stamps behind it: a row that carries the
                 // stamp of layer j or of a later one was active after layer j (bias <= 0: a zero row stays zero).
                 // The layer before the launch is counted the same way if nobody has counted it yet.  The kernel
@@ -2559,10 +2582,10 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             // a record is pushed when the launch that hands it over is queued, i.e. one launch late
             // (while the counts are unknown or still moving the host waits for each launch's counts: a launch made on rows
             // that have died since costs more than the round trip)
-            const size_t lookahead = st.c_prune <= 1 ? 0 : lookahead_for(n->carried) - 1;
+            const size_t lookahead = look_later ? recs.size() : st.c_prune <= 1 ? 0 : lookahead_for(n->carried) - 1;
             while (recs.size() - st.processed > lookahead && !st.dead && failed < 0) {
                 const Rec rc = recs[st.processed++];
-                const int wrc = wait_counts(n, rc.l0, rc.c);
+                const int wrc = wait_counts(n, rc.l0, rc.c, st.processed == recs.size());
                 if (wrc) return wrc;
                 if (rc.pl >= 0) {   // counts taken behind a persistent launch mean something only if it completed
                     const int src = settle(true, rc.pl, &failed);
@@ -2585,8 +2608,11 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             }
             if (failed >= 0) break;
             if (st.dead) { n->carried = 0; continue; }
-            if (st.newest_count > 0 && (double)st.newest_count <= (double)thr * (double)n->carried && st.l < n->L) {
-                const int nb = (int)((st.newest_count + n->RB - 1) / n->RB);  // upper bound of what is alive now
+            const int nb = (int)((std::max<int64_t>(st.newest_count, 0) + n->RB - 1) / n->RB);  // upper bound of what is alive now
+            bool worth = (double)st.newest_count <= (double)thr * (double)n->carried;
+            if (!worth && thr >= 0.75f && st.newest_count > 0 && st.sums && nb * n->RB < n->carried)   // (fewer rounds of workgroups)
+                worth = (sums_layer_us(st.sums, n->carried, n->n_cu, true) - sums_layer_us(st.sums, nb * n->RB, n->n_cu, true)) * (last - st.l + 1) > 60.0;
+            if (st.newest_count > 0 && worth && st.l < n->L) {
                 if (nb * n->RB < n->carried) {
                     if (!pending.empty()) {   // the repack overwrites a work buffer: not on the ruins of a persistent launch
                         const int rc = settle(true, INT_MAX, &failed);
@@ -2600,6 +2626,13 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                         HIPCHK(hipMemcpyAsync(n->d_counts + (st.l - 1), n->d_count, 4, hipMemcpyDeviceToDevice, n->stream));
                         st.count_pending = false;
                     }
+                    if (st.sums && st.l <= last && !n->layers[(size_t)st.l].sum_cols.empty() && sums_slab_rows(st.sums, nb * n->RB, n->n_cu, true) != 0) {
+                        gather = true;   // the next launch, of further group sums, takes the rows from where they are
+                        n->carried = nb * n->RB;
+                        n->last_stamp = 0;
+                        st.r.compactions++;
+                        continue;
+                    }
                     HIPCHK(launch_repack(n->cur, dstbuf, n->d_count, n->d_alive_src, n->d_alive_gid, n->d_gid_tmp,
                                          st.sums ? st.sums : n->N, n->rl, nb, n->stream));
                     std::swap(n->d_gid, n->d_gid_tmp);
@@ -2612,7 +2645,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 }
             }
         }
-        if (failed < 0 && st.sums && !st.dead) HIPCHK(expand_sums());
+        const bool close_up = failed < 0 && st.sums && !st.dead && opt.prune && n->last_stamp != 0 && st.last_launched == last;
+        if (failed < 0 && st.sums && !st.dead && !close_up) HIPCHK(expand_sums());
         if (failed < 0) {
             // categories of the last layer: survivor list by the scan.  After a final repack the list
             // produced for the repack is that list already.
@@ -2621,6 +2655,10 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 if (n->last_stamp != 0) {
                     HIPCHK(launch_scan_active(n->d_active, n->d_gid, n->carried, n->last_stamp, n->d_count, n->d_alive_src,
                                               n->d_alive_gid, n->stream));
+                }
+                if (close_up) {
+                    HIPCHK(expand_sums(true));
+                    closed_up = true;
                 }
                 HIPCHK(hipMemcpyAsync(n->h_count, n->d_count, 4, hipMemcpyDeviceToHost, n->stream));
                 if (st.count_pending)  // no launch follows the last layer: the scan's count is its count
@@ -2665,6 +2703,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     }
     if (st.dead || zero_seen) { if (opt.prune) n->carried = 0; n->alive = 0; }
     else if (n->alive_list_valid) n->alive = n->h_count[0];
+    if (closed_up) n->carried = std::min(n->carried, (int)((n->alive + n->RB - 1) / n->RB) * n->RB);
     if (n->alive == 0) n->alive_list_valid = true;  // the empty list
     // byte model: rows entering each launched layer
     int64_t entering = alive_at_start;

@@ -91,13 +91,14 @@ typedef struct spdnn_run_options {
     int32_t n_layers;          /* number of layers to run, -1 = through the last                   */
     int32_t collect_counts;    /* 1: record the active-row count after every layer                 */
     int32_t time_layers;       /* 1: bracket every layer with HIP events                           */
-    float   compact_threshold; /* prune: repack when active <= threshold * carried (0 = default .75) */
+    float   compact_threshold; /* prune: repack when active <= threshold * carried (0 = default .75;
+                                  from .75 up also where fewer rows take a launch fewer rounds of workgroups)      */
     int32_t fuse_layers;       /* launches that hold more than one layer.  1 = every layer its own launch.  0 = default:
                                   - resident launches where consecutive layers have a BLOCK form with one exact weight
                                     (RadiX-Net layers) or are TILED layers, at most 4096 neurons wide, or are BAND layers
                                     at most 1024 neurons wide (from 6 layers on, from 16 at 16384 rows and more; under one
-                                    power-of-two weight, 768 neurons or wider and with 16 rows for every compute unit,
-                                    from 4 on, on the matrix cores): a workgroup keeps 16, 8 or 4 rows
+                                    power-of-two weight up to 2304 neurons, from 4 layers on, on the matrix cores but
+                                    for launches of 12 - 16 rows per compute unit): a workgroup keeps 32, 16, 8 or 4 rows
                                     in LDS through up to 64 layers (SPDNN_RESIDENT=0: never; SPDNN_BAND_RESIDENT=0: not
                                     the BAND layers);
                                     three or more consecutive layers with such a BLOCK form, of any width up to 65536, carry

@@ -2306,3 +2306,61 @@ def test_group_sums_of_large_launches(gc, orc, monkeypatch, capfd, N, B, rl, R, 
                 seen.append(([net.active_count(l) for l in range(L)], cats, net.activations(ask)))
     for counts, cats, y in seen[1:]:
         assert counts == seen[0][0] and np.array_equal(cats, seen[0][1]) and same_floats(y, seen[0][2])
+
+
+@pytest.mark.parametrize("N,B,kind,rl,S", [
+    (512, 33000, "radix", 1, 132),     # 32 groups; slabs across row blocks of 64 rows, the last one shorter
+    (1008, 20000, "radix", 2, 80),     # 63 groups
+    (1024, 66000, "radix", 4, 132),    # two rounds of workgroups
+    (1024, 9000, "hub", 4, 36),        # lists of fewer than 32 inputs
+    (4160, 3000, "radix", 1, 12),      # 260 groups
+    (4096, 30000, "common", 4, 120),   # 30 quads of 256 groups: eight trips
+    (16400, 1300, "radix", 1, 8),      # 1025 groups
+    (65520, 1500, "hub", 4, 8),        # 4095 groups and the zero behind them
+    (65536, 1100, "radix", 4, 8),      # 4096 groups, eight trips of two quads; compacted to fewer rows than CUs x 4
+])
+def test_slabs_of_group_sums(gc, orc, monkeypatch, capfd, N, B, kind, rl, S):
+    """Group sums with many rows to a workgroup, rows dying in and between its launches and closing up: counts, categories and
+    activations against launches that carry full columns, and a part of the rows against the oracle."""
+    print("slabs of group sums N=%d B=%d %s" % (N, B, kind), flush=True)
+    monkeypatch.setenv("SPDNN_ROWS_PER_LANE", str(rl))
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    rng = np.random.default_rng(N + B)
+    L, few = 14, 40
+    if kind == "hub":
+        base = [hub_block_csr(rng, N) for _ in range(2)]
+    else:
+        perm = rng.permutation(N) if kind == "common" else None
+        base = [radix_like_csr(rng, N, 16 << k, perm=perm) for k in range(2 if N > 20000 else 4)]
+    layers = [base[l % len(base)] for l in range(L)]
+    bias = -0.3 if N <= 1024 else -0.35 if N <= 4096 else -0.4
+    lo, hi = (0.05, 0.9) if kind == "hub" else (-bias * 0.6, -bias * 1.12)
+    ref = orc.infer(gc.synth_features_host(3, N, 0, few, lo, hi), layers, bias, prune=True)
+    seen = []
+    for mode in ("1", "0"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", mode)
+        with gc.Network(N, B, L, bias=bias) as net:
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            net.inspect()
+            net.synth_features(3, B, lo, hi)
+            for kw in ({"prune": True}, {"prune": True, "compact_threshold": 1e-6}, {"prune": False}):
+                _launch_kinds(capfd)
+                r = net.run(collect_counts=True, **kw)
+                made = _launch_kinds(capfd)
+                if mode == "1" and kw["prune"]:
+                    assert "%d rows per workgroup," % S in made[1][1]
+                cats = net.categories()
+                mine = cats[cats < few]
+                assert np.array_equal(mine, ref["categories"]) and same_floats(net.activations(mine), ref["y"])
+                ask = cats[::max(1, len(cats) // 300)]
+                dead = np.setdiff1d(np.arange(B), cats)[::max(1, B // 200)].astype(np.int32)
+                assert not net.activations(dead).any()
+                seen.append(([net.active_count(l) for l in range(L)], cats, net.activations(ask)))
+            net.run(prune=True, n_layers=9)       # the state that a run leaves behind inside, continued
+            r = net.run(prune=True, first_layer=9, collect_counts=True)
+            assert np.array_equal(net.categories(), seen[0][1]) and same_floats(net.activations(ask), seen[0][2])
+    counts = seen[0][0]
+    assert 0 < counts[-1] < counts[0] and len(set(counts)) > 3
+    for got in seen[1:]:
+        assert got[0] == counts and np.array_equal(got[1], seen[0][1]) and same_floats(got[2], seen[0][2])
