@@ -3223,7 +3223,8 @@ __global__ __launch_bounds__(1024) void count_stamp_range_kernel(const int32_t* 
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void scan_active_kernel(
     const int32_t* __restrict__ active, const int32_t* __restrict__ gid, int rows, int stamp,
-    int32_t* __restrict__ count, int32_t* __restrict__ alive_src, int32_t* __restrict__ alive_gid) {
+    int32_t* __restrict__ count, int32_t* __restrict__ alive_src, int32_t* __restrict__ alive_gid, ScanEnd end) {
+    publish_counts(end.publish);
     __shared__ int wave_tot[16];
     __shared__ int wave_before[16];
     const int lane = threadIdx.x & 63;
@@ -3261,8 +3262,16 @@ __global__ __launch_bounds__(1024) void scan_active_kernel(
         const int k = base + (int)__popcll(mask & ((1ull << lane) - 1ull));
         alive_src[k] = r;
         alive_gid[k] = g;
+        if (end.list_host) end.list_host[k] = g;
     }
-    if (tile == (int)gridDim.x - 1 && threadIdx.x == 0) count[0] = total;
+    if (tile == (int)gridDim.x - 1 && threadIdx.x == 0) {
+        count[0] = total;
+        if (end.count_host) __hip_atomic_store(end.count_host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (end.last_dev) {
+            end.last_dev[0] = total;
+            __hip_atomic_store(end.last_host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
 }
 
 // Repack survivors into dense row blocks.  Thread = destination row slot; loops over a chunk of
@@ -3383,6 +3392,22 @@ __global__ void scatter_where_kernel(const int32_t* __restrict__ gid, int carrie
     if (r >= carried) return;
     const int g = gid[r];
     if (g >= 0 && g < batch) where[g] = r;
+}
+// phys[i] = the row whose global id is ids[i], -1 if none is left: the ids of the carried rows ascend (rows keep their order
+// in every compaction) up to the -1 of the slots behind them, which as unsigned numbers come last.  One launch, and the
+// ids straight from pinned memory, in the place of a table that is cleared, filled and read (two launches and a copy:
+// 187 rows of 1024 read back in 65 us against 76).
+__global__ __launch_bounds__(256) void find_rows_kernel(const int32_t* __restrict__ ids, int n, const int32_t* __restrict__ gid, int carried,
+                                                        int32_t* __restrict__ phys) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t id = (uint32_t)ids[i];
+    int lo = 0, hi = carried;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((uint32_t)gid[mid] < id) lo = mid + 1; else hi = mid;
+    }
+    phys[i] = lo < carried && (uint32_t)gid[lo] == id ? lo : -1;
 }
 __global__ void lookup_rows_kernel(const int32_t* __restrict__ ids, int n, const int32_t* __restrict__ where,
                                    int32_t* __restrict__ phys) {
@@ -3858,6 +3883,14 @@ int band_tile_rows(int N, int rows, int n_cu) {
     return N <= 1024 && (long long)rows * N > 18ll * 1024 * n_cu ? 32 : 16;
 }
 
+// (the figures of band_tile_resident_kernel, scaled; a CU holds sixteen waves)
+double band_tile_layer_us(int N, int steps, int rows, int n_cu) {
+    const int wg_rows = band_tile_rows(N, rows, n_cu), at_once = N <= 1024 ? 1024 / N : 1;
+    if (wg_rows == 0) return 0.0;
+    const int wgs = rows / wg_rows, rounds = (wgs + n_cu * at_once - 1) / (n_cu * at_once);
+    return rounds * (0.4 + (wg_rows == 32 ? 7.6 : 4.7) * steps / 48.0 * N * std::min(at_once, (wgs + n_cu - 1) / n_cu) / 1024.0);
+}
+
 template <int G, int NB, int T, int H>
 static hipError_t launch_band_tile_inst(const ResidentArgs& k, int rows, hipStream_t s) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(band_tile_resident_kernel<G, NB, T, H>),
@@ -4240,10 +4273,10 @@ hipError_t launch_sums_resident(const SumsLaunch& a, hipStream_t s) {
 }
 
 hipError_t launch_scan_active(const int32_t* active, const int32_t* gid, int rows, int stamp, int32_t* count,
-                              int32_t* alive_src, int32_t* alive_gid, hipStream_t s) {
-    if (rows < 0 || !active || !gid || !count || !alive_src || !alive_gid) return hipErrorInvalidValue;
+                              int32_t* alive_src, int32_t* alive_gid, hipStream_t s, const ScanEnd& end) {
+    if (rows < 0 || !active || !gid || !count || !alive_src || !alive_gid || (end.last_dev && !end.last_host)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(scan_active_kernel, dim3(std::max(1, (rows + 1023) / 1024)), dim3(1024), 0, s, active, gid, rows,
-                       stamp, count, alive_src, alive_gid);
+                       stamp, count, alive_src, alive_gid, end);
     return hipGetLastError();
 }
 
@@ -4328,6 +4361,11 @@ hipError_t launch_row_table(const int32_t* gid, int carried, int batch, int32_t*
     return hipGetLastError();
 }
 
+hipError_t launch_find_rows(const int32_t* ids, int n, const int32_t* gid, int carried, int32_t* phys, hipStream_t s) {
+    if (n <= 0 || carried < 0 || !ids || !phys || (carried > 0 && !gid)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(find_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, s, ids, n, gid, carried, phys);
+    return hipGetLastError();
+}
 hipError_t launch_lookup_rows(const int32_t* ids, int n, const int32_t* where, int32_t* phys, hipStream_t s) {
     if (n <= 0 || !ids || !where || !phys) return hipErrorInvalidValue;
     hipLaunchKernelGGL(lookup_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, s, ids, n, where, phys);

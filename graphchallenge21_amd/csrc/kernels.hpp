@@ -321,6 +321,8 @@ int resident_rows_per_workgroup(int N, int ngroups);
 hipError_t launch_band_tile_resident(const ResidentLaunch& a, hipStream_t s);
 // rows such a workgroup keeps (16 or 32), 0 = the shape does not fit
 int band_tile_rows(int N, int rows, int n_cu);
+// about what a layer of such a launch takes, in microseconds
+double band_tile_layer_us(int N, int steps, int rows, int n_cu);
 hipError_t launch_block_resident(const ResidentLaunch& a, hipStream_t s);
 
 // counts[i] = number of rows r < rows with stamps[r] >= stamp_lo + i, for i in [0, n): with bias <= 0 a
@@ -366,8 +368,16 @@ hipError_t launch_count_stamped(const int32_t* stamps, int rows, int stamp, int3
 // Active-row scan: rows with active[row] == stamp and gid[row] >= 0 survive, in order.
 // Writes count[0] = number of survivors, alive_src[k] = physical row of survivor k,
 // alive_gid[k] = its global id.
+// `end`: what the scan behind a run's last layer hands to the host (pinned memory) in place of copies behind it - the
+// count, the list of ids, the newest layer's count (also to the device counter) and the counts of earlier layers.
+struct ScanEnd {
+    int32_t* count_host = nullptr;
+    int32_t* list_host = nullptr;
+    int32_t *last_dev = nullptr, *last_host = nullptr;
+    Publish publish;
+};
 hipError_t launch_scan_active(const int32_t* active, const int32_t* gid, int rows, int stamp,
-                              int32_t* count, int32_t* alive_src, int32_t* alive_gid, hipStream_t s);
+                              int32_t* count, int32_t* alive_src, int32_t* alive_gid, hipStream_t s, const ScanEnd& end = ScanEnd{});
 
 // Repack: row slot k of the destination takes physical row alive_src[k] of the source for
 // k < count[0]; the remaining slots of the last block are zero-filled; gid_out likewise (-1).
@@ -397,6 +407,9 @@ hipError_t launch_fill_i32(int32_t* p, int n, int32_t v, hipStream_t s);
 hipError_t launch_iota_gid(int32_t* gid, int rows, int batch, hipStream_t s);
 // where[g] = physical row (< carried) whose global id is g, -1 if none, for g in [0, batch)
 hipError_t launch_row_table(const int32_t* gid, int carried, int batch, int32_t* where, hipStream_t s);
+// phys[i] = the row r < carried with gid[r] == ids[i], -1 if there is none (gid ascends, -1 behind the last row; ids may lie
+// in pinned host memory)
+hipError_t launch_find_rows(const int32_t* ids, int n, const int32_t* gid, int carried, int32_t* phys, hipStream_t s);
 // phys[i] = where[ids[i]] (ids already checked against the batch on the host)
 hipError_t launch_lookup_rows(const int32_t* ids, int n, const int32_t* where, int32_t* phys, hipStream_t s);
 hipError_t launch_copy_f4(const float* src, float* dst, int64_t n_floats, hipStream_t s);

@@ -439,6 +439,8 @@ struct spdnn_net {
     hipEvent_t ev_stage[kStageSlots] = {};
     float* d_stage = nullptr;
     size_t d_stage_bytes = 0;
+    int32_t* h_list = nullptr;        // pinned [rows_cap]: the ids of the rows that the last run left active, where list_on_host
+    bool list_on_host = false;
     int32_t* d_rowtab = nullptr;      // see spdnn_get_activations
     size_t rowtab_bytes = 0;
     std::vector<hipEvent_t> ev_layer;
@@ -536,6 +538,8 @@ void release_device_base(spdnn_net* n) {
     n->h_pwords = nullptr;
     if (n->h_count) hipHostFree(n->h_count);
     if (n->h_counts) hipHostFree(n->h_counts);
+    if (n->h_list) hipHostFree(n->h_list);
+    n->h_list = nullptr;
     n->d_active = n->d_gid = n->d_gid_tmp = n->d_alive_src = n->d_alive_gid = nullptr;
     n->d_count_partial = nullptr;
     n->d_count = n->d_nonfinite = n->d_counts = n->h_count = n->h_counts = nullptr;
@@ -595,6 +599,7 @@ int init_device(spdnn_net* n) {
     HIPCHK(hipHostMalloc(&n->h_count, 64, hipHostMallocCoherent | hipHostMallocMapped));
     HIPCHK(dev_malloc(&n->d_counts, (size_t)n->L * 4));
     HIPCHK(hipHostMalloc(&n->h_counts, (size_t)n->L * 4, hipHostMallocCoherent | hipHostMallocMapped));
+    HIPCHK(hipHostMalloc(&n->h_list, rows * 4, hipHostMallocCoherent | hipHostMallocMapped));
     HIPCHK(hipMemset(n->d_active, 0, rows * 4));
     // persistent launches: units finished per layer and row block, control words per launch, completion words
     n->done_stride = n->rows_cap / n->RB;
@@ -2054,7 +2059,9 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     const bool fused_count = n->bias <= 0.0f;
     const bool scan_count = !fused_count && opt.collect_counts;
     const bool have_counts = fused_count || scan_count;
-    if (fused_count) HIPCHK(hipMemsetAsync(n->d_counts + first, 0, (size_t)nl * 4, n->stream));
+    // (the counters that layer kernels add to, and the words of persistent launches, are cleared in front of the first launch
+    // that needs them: most runs of few rows make none)
+    bool counts_clear = !fused_count, persist_clear = false;
     // Launches that hold more than one layer need all their plans resident and count on the device:
     // fused pairs (by default and with fused launches asked for, not with fuse_layers = 1) and persistent
     // launches (asked for with fuse_layers >= 2 layers per launch, else by default where a layer moves
@@ -2065,10 +2072,6 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     bool persist_on = !no_fusion && (persist_asked || n->persist_mode == 1);
     const int persist_cmax = persist_asked ? opt.fuse_layers : n->persist_layers;
     const long long persist_wait_us = opt.persist_wait_us < 0 ? 0 : (opt.persist_wait_us > 0 ? opt.persist_wait_us : n->persist_wait_us);
-    if (persist_on) {
-        HIPCHK(hipMemsetAsync(n->d_done + (size_t)first * n->done_stride, 0, (size_t)nl * n->done_stride * 4, n->stream));
-        HIPCHK(hipMemsetAsync(n->d_ctl, 0, (size_t)nl * sizeof(PersistCtl), n->stream));
-    }
     if (plans_streamed(n))
         for (int l = first; l <= last && l < first + n->plan_window; ++l) HIPCHK(plan_fetch(n, l));
 
@@ -2100,7 +2103,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     // Everything the layer loop changes, so that it can go back to where a persistent launch started.
     struct State {
         Feat cur; int cur_layer, carried, stamp, last_stamp; bool blocks_skipped;
-        int l; bool dead, count_pending; int last_launched; int64_t newest_count; int c_prune;
+        int l; bool dead, count_pending; int last_launched; int64_t newest_count; int c_prune; bool settling;
         Publish pub; size_t nrecs, processed, ntimed; spdnn_run_result r;
         int sums;   // columns of n->cur where it holds group sums (see launch_sums_head), 0: the full layout
     };
@@ -2110,7 +2113,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     // the group sums that n->cur holds, written out for whatever reads the full columns next: a launch that counts as part
     // of the layer that computed them
     size_t expansions = 0;
-    bool closed_up = false;   // the expansion has left the rows that are alive, and only those
+    bool closed_up = false;   // the expansion, or a last repack, has left the rows that are alive, and only those
+    bool unlooked = false;    // the last launch was made while the counts moved
     bool gather = false;   // the rows of n->cur are to be taken from where the last scan found them (a compaction that the next launch makes)
     auto expand_sums = [&](bool compact = false) -> hipError_t {   // compact: the rows the last scan found, and only those
         const LayerPlan& p = n->layers[(size_t)n->cur_layer - 1];
@@ -2295,6 +2299,14 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 while (c < kmax && takes_sums(l + c)) ++c;
             }
             if (!fb && !chain && !head && persist_on && n->resident_mode && n->d_table && (rsig = resident_sig(n, l)).ok) {
+                // (tiles while the counts move: where fewer rows would take as long, one workgroup or less to a compute unit, or
+                // where the last layer looked at left three rows in four, about 120 us of layers to a launch and four at least.
+                // Looking behind every layer cost 25 us; 300 x 1024, six layers: 71 us a run against 113, 120 layers of 6000
+                // x 1024 0.77 ms against 1.28)
+                int most_here = cmax;
+                const bool one_round = (int64_t)n->carried * n->N <= (int64_t)16 * 1024 * n->n_cu;
+                if (rsig.ok == 4 && opt.prune && !persist_asked && (one_round || st.settling))
+                    most_here = std::max(cmax, std::min({persist_cmax, last - l + 1, std::max(4, (int)(120.0 / band_tile_layer_us(n->N, rsig.ngroups, n->carried, n->n_cu)))}));
                 // Bringing the rows in and out costs such a launch as much as two layers save it with 16 rows per workgroup
                 // (64-byte pieces of a column) and as much as eight save it with 4 rows (16-byte pieces): measured
                 // at 2048 and at 60000 rows.  So left to the library: from 2 layers (even while the counts still move -
@@ -2309,7 +2321,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                     if (g.ok < 3) return 8;
                     return n->band_resident_min_layers >= 2 ? n->band_resident_min_layers : g.ok == 4 ? 4 : (n->carried >= 16384 ? 16 : 6);
                 };
-                const int room = std::min(wide_rows ? std::max(cmax, 2) : cmax, last - l + 1);
+                const int room = std::min(wide_rows ? std::max(cmax, 2) : most_here, last - l + 1);
                 // layers from l0 on that one launch takes in the form g, of `most`
                 auto run_of = [&](int l0, const ResidentSig& g, int most, bool tiles) {
                     int k = 1;
@@ -2405,6 +2417,16 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             }
             const int stamp0 = n->stamp + 1;
             n->stamp += c;
+            if (!group && !counts_clear) {
+                const int from = st.count_pending ? std::max(first, l - 1) : l;   // (launches of several layers have stored theirs)
+                HIPCHK(launch_fill_i32(n->d_counts + from, last - from + 1, 0, n->stream));
+                counts_clear = true;
+            }
+            if (persist && !persist_clear) {
+                HIPCHK(launch_fill_i32(n->d_done + (size_t)first * n->done_stride, nl * n->done_stride, 0, n->stream));
+                HIPCHK(launch_fill_i32(reinterpret_cast<int32_t*>(n->d_ctl), (int)((size_t)nl * sizeof(PersistCtl) / 4), 0, n->stream));
+                persist_clear = true;
+            }
             if (opt.time_layers) HIPCHK(hipEventRecord(n->ev_layer[(size_t)(2 * l)], n->stream));
             if (persist) {
                 PersistLaunch pl{};
@@ -2577,7 +2599,12 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 st.count_pending = true;
             }
             st.l = l + c;
+            // (nothing comes behind the network's last layer: what is left is counted and written out without a look in between)
             if (!opt.prune) continue;
+            if (st.l == n->L) {
+                unlooked = resident && rsig.ok == 4 && st.c_prune < persist_cmax && thr >= 0.75f;
+                continue;
+            }
 
             // a record is pushed when the launch that hands it over is queued, i.e. one launch late
             // (while the counts are unknown or still moving the host waits for each launch's counts: a launch made on rows
@@ -2602,6 +2629,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // layers per multi-layer launch while pruning: all that are allowed once a layer has left the count as it
                 // was, doubled while the counts hold still (within 3 % from one record to the next), one layer per
                 // launch again when they move
+                st.settling = layer_before > 0 && st.newest_count * 4 >= layer_before * 3;
                 if (layer_before > 0 && st.newest_count == layer_before) st.c_prune = std::max(2, persist_cmax);
                 else if (before > 0 && st.newest_count * 100 >= before * 97) st.c_prune = std::min(persist_cmax, std::max(2, st.c_prune * 2));
                 else st.c_prune = 1;
@@ -2610,8 +2638,15 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             if (st.dead) { n->carried = 0; continue; }
             const int nb = (int)((std::max<int64_t>(st.newest_count, 0) + n->RB - 1) / n->RB);  // upper bound of what is alive now
             bool worth = (double)st.newest_count <= (double)thr * (double)n->carried;
-            if (!worth && thr >= 0.75f && st.newest_count > 0 && st.sums && nb * n->RB < n->carried)   // (fewer rounds of workgroups)
-                worth = (sums_layer_us(st.sums, n->carried, n->n_cu, true) - sums_layer_us(st.sums, nb * n->RB, n->n_cu, true)) * (last - st.l + 1) > 60.0;
+            if (!worth && thr >= 0.75f && st.newest_count > 0 && st.l <= last && nb * n->RB < n->carried) {   // (fewer rounds of workgroups)
+                const LayerPlan& q = n->layers[(size_t)st.l];
+                const bool tiles = !st.sums && persist_on && n->resident_mode && resident_sig(n, st.l).ok == 4;
+                auto layer_us = [&](int rows) {
+                    return st.sums ? sums_layer_us(st.sums, rows, n->n_cu, true) : tiles ? band_tile_layer_us(n->N, q.tile_steps, rows, n->n_cu) : 0.0;
+                };
+                worth = (layer_us(n->carried) - layer_us(nb * n->RB)) * (last - st.l + 1) >
+                        60.0 + 8.0 * (double)nb * n->RB * (st.sums ? st.sums : n->N) / 4.0e6;   // looking and packing
+            }
             if (st.newest_count > 0 && worth && st.l < n->L) {
                 if (nb * n->RB < n->carried) {
                     if (!pending.empty()) {   // the repack overwrites a work buffer: not on the ruins of a persistent launch
@@ -2645,28 +2680,51 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 }
             }
         }
-        const bool close_up = failed < 0 && st.sums && !st.dead && opt.prune && n->last_stamp != 0 && st.last_launched == last;
+        const bool close_up = failed < 0 && st.sums && !st.dead && opt.prune && thr >= 0.75f && n->last_stamp != 0 && st.last_launched == last;
         if (failed < 0 && st.sums && !st.dead && !close_up) HIPCHK(expand_sums());
         if (failed < 0) {
             // categories of the last layer: survivor list by the scan.  After a final repack the list
             // produced for the repack is that list already.
             n->alive_list_valid = false;
+            n->list_on_host = false;
+            bool counts_over = false;   // every layer's count is on its way to the host
             if (!st.dead && st.last_launched == last) {
+                n->list_on_host = n->last_stamp != 0;
                 if (n->last_stamp != 0) {
+                    // the scan hands over what the host needs; its count is the last layer's where no launch has taken that
+                    ScanEnd end;
+                    end.count_host = n->h_count;
+                    end.list_host = n->h_list;
+                    if (st.count_pending) { end.last_dev = n->d_counts + last; end.last_host = n->h_counts + last; }
+                    if (have_counts) end.publish = {n->d_counts + first, n->h_counts + first, last - first + (st.count_pending ? 0 : 1)};
+                    counts_over = have_counts;
                     HIPCHK(launch_scan_active(n->d_active, n->d_gid, n->carried, n->last_stamp, n->d_count, n->d_alive_src,
-                                              n->d_alive_gid, n->stream));
+                                              n->d_alive_gid, n->stream, end));
+                } else {
+                    HIPCHK(hipMemcpyAsync(n->h_count, n->d_count, 4, hipMemcpyDeviceToHost, n->stream));
+                    if (st.count_pending)
+                        HIPCHK(hipMemcpyAsync(n->d_counts + last, n->d_count, 4, hipMemcpyDeviceToDevice, n->stream));
                 }
                 if (close_up) {
                     HIPCHK(expand_sums(true));
                     closed_up = true;
+                } else if (unlooked && !st.sums && n->last_stamp != 0 && 8ll * n->carried * n->N <= 64ll << 20) {
+                    // (a run whose rows died inside its last launch leaves the others together, as one with a look behind every
+                    // layer does; a few microseconds where the buffers stay on chip)
+                    const Feat dstbuf = (n->cur == n->A) ? n->C : n->A;
+                    HIPCHK(launch_repack(n->cur, dstbuf, n->d_count, n->d_alive_src, n->d_alive_gid, n->d_gid_tmp, n->N, n->rl,
+                                         n->carried / n->RB, n->stream));
+                    std::swap(n->d_gid, n->d_gid_tmp);
+                    n->gid_dirty = true;
+                    n->cur = dstbuf;
+                    n->last_stamp = 0;
+                    n->blocks_skipped = false;
+                    closed_up = true;
                 }
-                HIPCHK(hipMemcpyAsync(n->h_count, n->d_count, 4, hipMemcpyDeviceToHost, n->stream));
-                if (st.count_pending)  // no launch follows the last layer: the scan's count is its count
-                    HIPCHK(hipMemcpyAsync(n->d_counts + last, n->d_count, 4, hipMemcpyDeviceToDevice, n->stream));
                 n->alive_list_valid = true;
             }
             HIPCHK(hipEventRecord(n->ev_stop, n->stream));
-            if (have_counts && st.last_launched >= first)   // all of them once more (the last launch's have no launch after it)
+            if (have_counts && st.last_launched >= first && !counts_over)   // all of them once more (the last launch's have no launch after it)
                 HIPCHK(hipMemcpyAsync(n->h_counts + first, n->d_counts + first, (size_t)(st.last_launched - first + 1) * 4,
                                       hipMemcpyDeviceToHost, n->stream));
             HIPCHK(hipStreamSynchronize(n->stream));
@@ -2703,7 +2761,11 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
     }
     if (st.dead || zero_seen) { if (opt.prune) n->carried = 0; n->alive = 0; }
     else if (n->alive_list_valid) n->alive = n->h_count[0];
-    if (closed_up) n->carried = std::min(n->carried, (int)((n->alive + n->RB - 1) / n->RB) * n->RB);
+    if (closed_up) {
+        const int left = (int)((n->alive + n->RB - 1) / n->RB) * n->RB;
+        if (left < n->carried && left > 0) r.compactions++;
+        n->carried = std::min(n->carried, left);
+    }
     if (n->alive == 0) n->alive_list_valid = true;  // the empty list
     // byte model: rows entering each launched layer
     int64_t entering = alive_at_start;
@@ -2743,6 +2805,10 @@ static int spdnn_get_categories_impl(spdnn_net* n, int32_t* ids, int64_t cap, in
     if (cap < n->alive) return fail(SPDNN_E_ARG, "ids buffer too small");
     if (!n->alive_list_valid) return fail(SPDNN_E_STATE, "no active list available");
     const size_t bytes = (size_t)n->alive * 4;
+    if (n->list_on_host) {   // (handed over by the run's last scan: 1 us for 2000 ids, 20 as a copy of its own)
+        memcpy(ids, n->h_list, bytes);
+        return SPDNN_OK;
+    }
     // (2000 ids: 20 us through pinned memory, 27 - 36 through pageable; a new set for them alone would cost more)
     StageLease lease(n->stream);
     if (!n->pinned_staging || !StagePool::get().lend_idle((bytes + kStageSlots - 1) / kStageSlots, &lease.set)) {
@@ -2775,9 +2841,9 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         if (rc) return rc;
     }
     const int per = (int)std::min<size_t>(65535, (pinned ? lease.slot : n->d_stage_bytes) / row_bytes);   // rows per slot
-    // global id -> physical row of the current buffer, and the ids asked for: kept until another batch size comes (an
-    // allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
-    const size_t table_bytes = (size_t)n->batch * 4 + id_bytes;
+    // the rows' places in the current buffer, and the ids asked for where they don't go through a slot: kept until another batch
+    // size comes (an allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
+    const size_t table_bytes = 2 * id_bytes;
     if (n->rowtab_bytes < table_bytes) {
         hipFree(n->d_rowtab);
         n->d_rowtab = nullptr;
@@ -2785,22 +2851,22 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         HIPCHK(dev_malloc(&n->d_rowtab, table_bytes));
         n->rowtab_bytes = table_bytes;
     }
-    int32_t* const d_where = n->d_rowtab;
-    int32_t* const d_ids = d_where + n->batch;
-    HIPCHK(launch_row_table(n->d_gid, n->carried, n->batch, d_where, n->stream));
-    const void* ids_from = rows;
-    if (id_bytes <= lease.slot) {   // (from pinned memory where they fit the last slot, whose rows come behind this copy)
+    int32_t* const d_phys = n->d_rowtab;
+    const int32_t* ids_from = d_phys + nrows;
+    if (id_bytes <= lease.slot) {   // (in the last slot, whose rows come behind their use)
         memcpy(lease.at(kStageSlots - 1), rows, id_bytes);
-        ids_from = lease.at(kStageSlots - 1);
+        ids_from = (const int32_t*)lease.at(kStageSlots - 1);
+    } else {
+        HIPCHK(hipMemcpyAsync(d_phys + nrows, rows, id_bytes, hipMemcpyHostToDevice, n->stream));
     }
-    HIPCHK(hipMemcpyAsync(d_ids, ids_from, id_bytes, hipMemcpyHostToDevice, n->stream));
+    HIPCHK(launch_find_rows(ids_from, nrows, n->d_gid, n->carried, d_phys, n->stream));
     const int32_t* lab = nullptr;
     HIPCHK(labelling_dev(n, n->cur_layer, &lab));
     const int K = (nrows + per - 1) / per;
     auto rows_in = [&](int k) { return std::min(per, nrows - k * per); };
     if (!pinned) {
         for (int k = 0; k < K; ++k) {
-            HIPCHK(launch_unpack_rows(n->cur, lab, d_ids + (size_t)k * per, d_where, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+            HIPCHK(launch_unpack_rows(n->cur, lab, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
                                       n->d_stage, n->stream));
             HIPCHK(hipMemcpyAsync(rowmajor + (size_t)k * per * n->N, n->d_stage, (size_t)rows_in(k) * row_bytes, hipMemcpyDeviceToHost, n->stream));
         }
@@ -2822,7 +2888,7 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
             HIPCHK(ready(arrived++));
             crew.wait(k - kStageSlots);
         }
-        HIPCHK(launch_unpack_rows(n->cur, lab, d_ids + (size_t)k * per, d_where, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
                                   (float*)lease.at(k), n->stream));
         HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
     }
