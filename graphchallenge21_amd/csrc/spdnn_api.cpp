@@ -24,6 +24,8 @@
 #include <thread>
 #include <vector>
 
+#include <emmintrin.h>
+
 #include "../../include/spdnn.h"
 #include "inspector.hpp"
 #include "kernels.hpp"
@@ -441,6 +443,8 @@ struct spdnn_net {
     size_t d_stage_bytes = 0;
     int32_t* h_list = nullptr;        // pinned [rows_cap]: the ids of the rows that the last run left active, where list_on_host
     bool list_on_host = false;
+    std::vector<uint16_t> group_of;   // group of equal outputs that every neuron of layer group_layer belongs to (see output_groups)
+    int group_layer = -1;
     int32_t* d_rowtab = nullptr;      // see spdnn_get_activations
     size_t rowtab_bytes = 0;
     std::vector<hipEvent_t> ev_layer;
@@ -648,6 +652,38 @@ int ensure_d_stage(spdnn_net* n, size_t bytes) {
     HIPCHK(dev_malloc(&n->d_stage, bytes));
     n->d_stage_bytes = bytes;
     return SPDNN_OK;
+}
+bool plans_streamed(const spdnn_net* n);
+// Groups of equal outputs of the layer run last, 0 where it has none or they do not save the link much: layers whose
+// outputs come in groups of up to 16 that read the same inputs under one exact weight (see launch_sums_head).  n->group_of then
+// names the group of every neuron.
+int output_groups(spdnn_net* n) {
+    const int l = n->cur_layer - 1;
+    if (l < 0 || !n->sums_mode || plans_streamed(n)) return 0;   // (a streamed plan may be another layer's by now)
+    const LayerPlan& p = n->layers[(size_t)l];
+    const int G = sum_groups(p);
+    if (G == 0 || G > 65535 || 4 * G > n->N) return 0;
+    if (n->group_layer != l) {
+        const std::vector<int32_t>& out_at = p.kernel == SPDNN_KERNEL_BAND ? p.alt_out_at : p.out_at;
+        n->group_layer = -1;
+        n->group_of.assign((size_t)n->N, 0);
+        int named = 0;
+        for (int s = 0; s < 16 * G; ++s) {
+            if (out_at[(size_t)s] < 0) continue;
+            n->group_of[(size_t)out_at[(size_t)s]] = (uint16_t)(s / 16);
+            ++named;
+        }
+        if (named != n->N) return 0;
+        n->group_layer = l;
+    }
+    return G;
+}
+// A row from its group values.  `stream`: past the caches (a transfer larger than those; rows start at 16 bytes)
+void expand_row(float* out, const float* sums, const uint16_t* group, int N, bool stream) {
+    int j = 0;
+    if (stream)
+        for (; j + 4 <= N; j += 4) _mm_stream_ps(out + j, _mm_setr_ps(sums[group[j]], sums[group[j + 1]], sums[group[j + 2]], sums[group[j + 3]]));
+    for (; j < N; ++j) out[j] = sums[group[j]];
 }
 // Part `part` of CopyCrew::kParts of a piece of `bytes`
 void copy_part(void* dst, const void* src, size_t bytes, int part) {
@@ -1452,6 +1488,7 @@ static int spdnn_inspect_impl(spdnn_net* n) {
         p.info.fuse_next = p.fuse_next ? 1 : 0;
     }
     if (n->uploaded) free_device(n);  // plans changed: upload again on next use
+    n->group_layer = -1;
     n->tuned.clear();
     n->exploring.clear();
     for (const spdnn_net::Trial& t : n->trials) { n->ev_free.push_back(t.e0); n->ev_free.push_back(t.e1); }
@@ -2831,16 +2868,23 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         if (rows[i] < 0 || rows[i] >= n->batch) return fail(SPDNN_E_ARG, "row id out of range");
     // The rows go through pinned slots: a kernel finds a slot's rows and writes them into it (over the link: as fast as a
     // copy command, and no copy in device memory in between), the host copies them out while the next slots are filled.
+    // Behind a layer of equal groups a group's value goes over the link once, a sixteenth of the row, and the host writes it
+    // to the group's neurons: what is left is the rate at which the host's threads write (9 MB 0.16
+    // ms, 0.28 with whole rows over the link; 29 MB 0.29, 0.72; 590 MB into a fresh array 6.3, 12.2).
     const size_t row_bytes = (size_t)n->N * 4, id_bytes = (size_t)nrows * 4;
+    int groups = n->pinned_staging ? output_groups(n) : 0;
     StageLease lease(n->stream);
-    int rc = lend_staging(n, (size_t)nrows * row_bytes, row_bytes, &lease);
+    const size_t lent_bytes = groups ? (size_t)groups * 4 : row_bytes;
+    int rc = lend_staging(n, (size_t)nrows * lent_bytes, lent_bytes, &lease);
     if (rc) return rc;
     const bool pinned = lease.set.p != nullptr;
+    if (!pinned) groups = 0;
+    const size_t slot_row = groups ? lent_bytes : row_bytes;   // bytes of a row in a slot
     if (!pinned) {   // through device memory then, 32 MiB of rows at a time
         rc = ensure_d_stage(n, std::max(row_bytes, std::min((size_t)nrows * row_bytes, (size_t)32 << 20)));
         if (rc) return rc;
     }
-    const int per = (int)std::min<size_t>(65535, (pinned ? lease.slot : n->d_stage_bytes) / row_bytes);   // rows per slot
+    const int per = (int)std::min<size_t>(65535, (pinned ? lease.slot : n->d_stage_bytes) / slot_row);   // rows per slot
     // the rows' places in the current buffer, and the ids asked for where they don't go through a slot: kept until another batch
     // size comes (an allocation and its release, which waits for the device, cost as much as reading back half a megabyte)
     const size_t table_bytes = 2 * id_bytes;
@@ -2874,9 +2918,22 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         return SPDNN_OK;
     }
     const size_t bytes = (size_t)nrows * row_bytes;
+    // (18 MB 0.20 ms, 0.28 through the caches; 29 MB 0.29, 0.35)
+    const bool stream = bytes >= (size_t)16 << 20 && (n->N % 4) == 0 && ((uintptr_t)rowmajor & 15) == 0;
     CopyCrew crew(bytes >= kCrewMinBytes ? n->pool.get() : nullptr, CopyCrew::workers_out(bytes), K, [&](int k, int part) {
-        copy_part(rowmajor + (size_t)k * per * n->N, lease.at(k), (size_t)rows_in(k) * row_bytes, part);
+        float* const to = rowmajor + (size_t)k * per * n->N;
+        if (!groups) { copy_part(to, lease.at(k), (size_t)rows_in(k) * row_bytes, part); return; }
+        const int lo = (int)((int64_t)rows_in(k) * part / CopyCrew::kParts), hi = (int)((int64_t)rows_in(k) * (part + 1) / CopyCrew::kParts);
+        for (int i = lo; i < hi; ++i)
+            expand_row(to + (size_t)i * n->N, (const float*)lease.at(k) + (size_t)i * groups, n->group_of.data(), n->N, stream);
+        if (stream) _mm_sfence();
     });
+    const int32_t* cols = lab;
+    if (groups) {   // the column of a group's first output
+        const LayerPlan& p = n->layers[(size_t)n->cur_layer - 1];
+        const DevLayer& d = n->dl[(size_t)n->cur_layer - 1];
+        cols = p.kernel == SPDNN_KERNEL_BAND ? d.alt_dst : d.dst;
+    }
     auto ready = [&](int k) -> hipError_t {   // slot k's rows have arrived: handed to the crew
         const hipError_t e = hipEventSynchronize(n->ev_stage[k % kStageSlots]);
         if (e == hipSuccess) crew.open(k);
@@ -2888,8 +2945,8 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
             HIPCHK(ready(arrived++));
             crew.wait(k - kStageSlots);
         }
-        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
-                                  (float*)lease.at(k), n->stream));
+        HIPCHK(launch_unpack_rows(n->cur, cols, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+                                  (float*)lease.at(k), n->stream, groups ? groups : n->N, groups ? 16 : 1));
         HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
     }
     while (arrived < K) HIPCHK(ready(arrived++));

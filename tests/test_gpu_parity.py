@@ -2364,3 +2364,40 @@ def test_slabs_of_group_sums(gc, orc, monkeypatch, capfd, N, B, kind, rl, S):
     assert 0 < counts[-1] < counts[0] and len(set(counts)) > 3
     for got in seen[1:]:
         assert got[0] == counts and np.array_equal(got[1], seen[0][1]) and same_floats(got[2], seen[0][2])
+
+
+@pytest.mark.parametrize("N,B,asked,window", [
+    (512, 40, 70, 0),         # one piece, written by the calling thread
+    (1008, 900, 1300, 0),     # past the size from which the writing is shared out
+    (1024, 6000, 5000, 0),    # 20 MB, written past the caches
+    (16384, 300, 520, 0),     # 34 MB, several pieces
+    (1024, 700, 900, 3),      # streamed plans: another layer's plan may lie where this layer's did
+])
+def test_rows_read_back_by_group(gc, monkeypatch, N, B, asked, window):
+    """Behind layers of equal groups one value per group goes over the link: the rows come out as with whole rows, in any
+    order, dead ones as zeros, behind every layer and into memory that starts at an odd word."""
+    print("rows read back by group N=%d B=%d" % (N, B), flush=True)
+    rng = np.random.default_rng(N + B)
+    L = 5
+    layers = [radix_like_csr(rng, N, 16 << (l % 3)) for l in range(L)]
+    rows = rng.integers(0, B, size=asked).astype(np.int32)
+    got = []
+    for sums in ("1", "0"):
+        monkeypatch.setenv("SPDNN_GROUP_SUMS", sums)
+        with gc.Network(N, B, L, bias=-0.3 if N <= 1024 else -0.4) as net:
+            if window:
+                net.set_plan_window(window)
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            net.inspect()
+            net.synth_features(3, B, 0.05, 0.9)
+            for n in (1, 2, 4, 5):
+                net.run(prune=n != 2, n_layers=n)
+                y = net.activations(rows)
+                odd = np.empty(asked * N + 1, np.float32)[1:].reshape(asked, N)
+                assert net._lib.spdnn_get_activations(net._h, rows, asked, odd) == 0
+                assert same_floats(odd, y)
+                got.append(y)
+    assert 0 < got[3].any(axis=1).sum() < asked
+    for a, b in zip(got[:4], got[4:]):
+        assert same_floats(a, b)
