@@ -335,14 +335,16 @@ int spdnn_get_categories(spdnn_net* net, int32_t* ids, int64_t cap, int64_t* n);
  * (all_network.cu:521).
  * The rows go through pinned slots that the networks of a process share: four of at most 16 MiB (or of one row, where that
  * is more) for each transfer under way, at most two such sets kept when none is, one of at most 16 MiB when the last
- * network has been destroyed.  Where no memory can be pinned (or SPDNN_PINNED_STAGING=0) they go through pageable memory. */
+ * network has been destroyed.  Where no memory can be pinned (or SPDNN_PINNED_STAGING=0) they go through pageable memory.
+ * Behind a layer of equal groups (a BLOCK form with one exact weight, plans resident) one value per group goes over the
+ * link and the host's threads write it to the group's neurons (SPDNN_GROUP_SUMS=0: whole rows). */
 int spdnn_get_activations(spdnn_net* net, const int32_t* rows, int nrows, float* rowmajor);
 
 /* spdnn_get_activations for callers that cannot allocate device memory (tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  It allocates nothing, but it
  * is not a call for inside a HIP graph capture: it synchronises its stream once per pass and copies
  * to and from pageable host memory.  Same arguments and results as spdnn_get_activations, but where that call allocates
- * (its row table, at the first call for a batch size and when more rows are asked for than before; pinned slots, when the
+ * (the rows' places, at the first call for a batch size and when more rows are asked for than before; pinned slots, when the
  * process has none that are large enough), this one calls no hipMalloc / hipFree:
  * it works in a 12.1 MiB scratch array that is part of the library's device code (one copy per GPU,
  * held until the process ends): a row table (global id -> physical row, filled by two small
