@@ -459,7 +459,7 @@ struct spdnn_net {
     int stamp = 0;
     int64_t alive = 0;        // rows active after the last layer run
     bool alive_list_valid = false;
-    bool gid_dirty = false;   // a repack permuted d_gid since it was last initialised
+    bool gid_dirty = false;   // a compaction changed d_gid since it was last initialised
     int last_stamp = 0;       // stamp of the newest layer, valid for the current row slots (0 = none)
     // A launch that skips row blocks without an active row leaves those blocks of its output buffer
     // unwritten (they hold an older layer's values).  Consumers that look at the stamps never read
@@ -1100,6 +1100,13 @@ hipError_t labelling_dev(spdnn_net* n, int layers_done, const int32_t** out) {
     }
     *out = second;
     return hipSuccess;
+}
+
+// The carried rows have moved (or are about to, in a launch that has just been queued) and d_gid_tmp holds their ids: the
+// one place where the two change, so that no compaction leaves reset_state without the mark that d_gid has to be written anew.
+void take_moved_ids(spdnn_net* n) {
+    std::swap(n->d_gid, n->d_gid_tmp);
+    n->gid_dirty = true;
 }
 
 void reset_state(spdnn_net* n) {
@@ -2172,8 +2179,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                                n->rl, rows, n->stream);
         if (e != hipSuccess) return e;
         if (compact) {
-            std::swap(n->d_gid, n->d_gid_tmp);
-            n->gid_dirty = true;
+            take_moved_ids(n);
             n->last_stamp = 0;
             n->blocks_skipped = false;
         }
@@ -2522,7 +2528,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 if (gather) { sl.rows_from.src = n->d_alive_src; sl.rows_from.gid = n->d_alive_gid; sl.rows_from.count = n->d_count; sl.rows_from.gid_out = n->d_gid_tmp; }
                 HIPCHK(launch_sums_resident(sl, n->stream));
                 if (gather) {
-                    std::swap(n->d_gid, n->d_gid_tmp);
+                    take_moved_ids(n);
                     gather = false;
                 }
                 if (n->run_verbose)
@@ -2708,8 +2714,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                     }
                     HIPCHK(launch_repack(n->cur, dstbuf, n->d_count, n->d_alive_src, n->d_alive_gid, n->d_gid_tmp,
                                          st.sums ? st.sums : n->N, n->rl, nb, n->stream));
-                    std::swap(n->d_gid, n->d_gid_tmp);
-                    n->gid_dirty = true;
+                    take_moved_ids(n);
                     n->cur = dstbuf;
                     n->carried = nb * n->RB;
                     n->last_stamp = 0;  // the row slots moved: the stamps no longer describe them
@@ -2752,8 +2757,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                     const Feat dstbuf = (n->cur == n->A) ? n->C : n->A;
                     HIPCHK(launch_repack(n->cur, dstbuf, n->d_count, n->d_alive_src, n->d_alive_gid, n->d_gid_tmp, n->N, n->rl,
                                          n->carried / n->RB, n->stream));
-                    std::swap(n->d_gid, n->d_gid_tmp);
-                    n->gid_dirty = true;
+                    take_moved_ids(n);
                     n->cur = dstbuf;
                     n->last_stamp = 0;
                     n->blocks_skipped = false;

@@ -2401,3 +2401,38 @@ def test_rows_read_back_by_group(gc, monkeypatch, N, B, asked, window):
     assert 0 < got[3].any(axis=1).sum() < asked
     for a, b in zip(got[:4], got[4:]):
         assert same_floats(a, b)
+
+@pytest.mark.parametrize("how", ["low threshold", "another class behind", "all rows die"])
+def test_runs_after_a_compaction_made_by_a_launch_of_group_sums(gc, orc, monkeypatch, capfd, how):
+    """A compaction that a launch of group sums makes as it takes its rows in renumbers them, like any other: runs over the
+    same features afterwards start from all rows again.  Three ways to end without a later repack that would hide it."""
+    print("compaction inside group sums,", how, flush=True)
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    monkeypatch.setenv("SPDNN_PERSIST_LAYERS", "3")      # looks behind layers 3, 6 and 9
+    rng = np.random.default_rng(8)
+    N, B, L = 512, 6000, 25 if how == "all rows die" else 13
+    layers = [radix_like_csr(rng, N, 16 << (l % 4)) for l in range(L)]
+    if how == "another class behind":
+        layers[7:] = [random_csr(rng, N, rng.integers(20, 40, size=N), "uniform") for _ in range(L - 7)]
+    if how == "all rows die":
+        layers[7] = (layers[7][0], layers[7][1], -layers[7][2])
+    feats = (rng.random((B, N)) < np.where(rng.random((B, 1)) < 0.3, 0.5, 0.2)).astype(np.float32)
+    ref = orc.infer(feats, layers, -0.3, prune=False, keep=set(range(L)))
+    thr = 0.5 if how == "low threshold" else 0.75
+    every = np.arange(B, dtype=np.int32)
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        for n, kw in ((L, {"prune": True}), (6, {"prune": False}), (L, {"prune": True}), (2, {"prune": True}), (L, {"prune": True}), (L, {"prune": False})):
+            _launch_kinds(capfd)
+            r = net.run(n_layers=n, compact_threshold=thr, **kw)
+            if n == L and kw["prune"]:     # one compaction, made by the second launch of group sums
+                carried = [int(re.search(r"(\d+) rows,", what).group(1)) for kind, what in _launch_kinds(capfd) if kind == "group sums"]
+                assert r.compactions == 1 and carried[0] > 6000 and 1024 <= carried[1] < 3000 and set(carried[2:]) <= {carried[1]}
+                assert r.carried_rows == (0 if how == "all rows die" else carried[1])
+                assert (r.layers_run < L) == (how == "all rows die")      # (the host has seen the end, and has not packed what is left)
+            assert np.array_equal(net.categories(), ref["active_ids"][n - 1])
+            assert same_floats(net.activations(every), ref["kept"][n - 1][1])
+            assert same_floats(net.activations_noalloc(every[::7]), ref["kept"][n - 1][1][::7])
