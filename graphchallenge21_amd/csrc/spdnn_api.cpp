@@ -660,7 +660,9 @@ bool plans_streamed(const spdnn_net* n);
 // names the group of every neuron.
 int output_groups(spdnn_net* n) {
     const int l = n->cur_layer - 1;
-    if (l < 0 || !n->sums_mode || plans_streamed(n)) return 0;   // (a streamed plan may be another layer's by now)
+    // (a streamed plan may be another layer's by now; and from the moment a layer is handed over anew its plan here is not the
+    // one that computed the rows, and a worker may be writing it)
+    if (l < 0 || !n->inspected || !n->sums_mode || plans_streamed(n)) return 0;
     const LayerPlan& p = n->layers[(size_t)l];
     const int G = sum_groups(p);
     if (G == 0 || G > 65535 || 4 * G > n->N) return 0;

@@ -2436,3 +2436,29 @@ def test_runs_after_a_compaction_made_by_a_launch_of_group_sums(gc, orc, monkeyp
             assert np.array_equal(net.categories(), ref["active_ids"][n - 1])
             assert same_floats(net.activations(every), ref["kept"][n - 1][1])
             assert same_floats(net.activations_noalloc(every[::7]), ref["kept"][n - 1][1][::7])
+
+
+def test_rows_read_back_after_a_layer_was_replaced(gc, orc):
+    """Rows may be read until the network is inspected again: a layer that has been handed over anew since the run does not
+    show in them, whatever its groups are."""
+    print("rows read back after a layer was replaced", flush=True)
+    rng = np.random.default_rng(12)
+    N, B, L = 1024, 700, 4      # (2.9 MB: past the size up to which whole rows are read)
+    layers = [radix_like_csr(rng, N, 16 << l) for l in range(L)]
+    feats = (rng.random((B, N)) < 0.4).astype(np.float32)
+    want = orc.infer(feats, layers, -0.3, prune=False)["y"]
+    every = np.arange(B, dtype=np.int32)
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        net.run(prune=False)
+        for k in range(3):
+            net.set_layer_csr(L - 1, *radix_like_csr(rng, N, 32 << k))
+            if k != 1:
+                net.layer_plan(L - 1)      # (waits for its inspection)
+            assert same_floats(net.activations(every), want)
+        net.inspect()
+        with pytest.raises(gc.SpdnnError):
+            net.activations(every)
