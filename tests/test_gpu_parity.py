@@ -2462,3 +2462,28 @@ def test_rows_read_back_after_a_layer_was_replaced(gc, orc):
         net.inspect()
         with pytest.raises(gc.SpdnnError):
             net.activations(every)
+
+
+def test_waiting_for_counts_leaves_the_processor_alone(gc):
+    """While the counts of a launch are outstanding (the device is held back for 15 ms, less than what one layer of wide rows
+    can take) the calling thread sleeps, whether or not something is queued behind that launch; its timers are as before then."""
+    import ctypes
+    import time
+    slack = lambda: ctypes.CDLL(None).prctl(30, 0, 0, 0, 0)      # (PR_GET_TIMERSLACK)
+    print("waiting for counts", flush=True)
+    rng = np.random.default_rng(5)
+    with gc.Network(1024, 300, 6, bias=-0.3) as net:
+        for l in range(6):
+            net.set_layer_csr(l, *radix_like_csr(rng, 1024, 16 << (l % 3)))
+        net.inspect()
+        net.synth_features(3, 300, 0.3, 0.6)
+        net.run(prune=True)
+        before, shares = slack(), []
+        for _ in range(5):
+            hold_device(0.015)
+            t, c = time.perf_counter(), time.thread_time()
+            net.run(prune=True, n_layers=3)
+            shares.append((time.thread_time() - c) / (time.perf_counter() - t))
+            assert time.perf_counter() - t > 0.014
+        print("share of a processor:", shares, flush=True)
+        assert sorted(shares)[2] < 0.6 and slack() == before
