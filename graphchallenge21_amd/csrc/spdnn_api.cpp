@@ -2055,11 +2055,11 @@ struct ResidentSig {
     bool operator==(const ResidentSig& o) const { return ok == o.ok && full == o.full && ngroups == o.ngroups && wmode == o.wmode; }
 };
 // Where bands of one exact weight run as tiles.  Up to 1024 neurons against QUAD, 32 entries, us per layer: 1024 neurons
-// 300 rows 4.8 and 5.7, 2000 4.9 and 5.6, 4352 9.6 and 11.9, 40000 39 and 54, 60000 63 and 80; 768 neurons 3.7 and 4.5
-// at 300, 30 and 41 at 40000; 512 2.7 and 3.3 at 300, 8.3 and 10.8 at 16000, 30 and 37 at 60000; 256 15 and 19 at 60000.
-// Launches of 12 to 16 rows (20, below 768 neurons) for every CU stay with QUAD, where they have always run and the
-// tests look for them (1024 neurons, 3840 rows: 6.3 against 5.1).  Wider bands have no QUAD form; tiles against one walk
-// per layer: 2048 neurons 9.4 and 9.0 at 300 rows, 9.7 and 18 at 4096, 136 and 197 at 60000; 1536 neurons 103 and 148.
+// 300 rows 5.0 and 6.3, 2000 5.2 and 5.9, 4352 9.8 and 12.7, 40000 40.5 and 61, 60000 64 and 88; 768 neurons 3.9 and 4.9
+// at 300, 31 and 47 at 40000; 512 2.9 and 3.3 at 300, 8.7 and 11.6 at 16000, 31 and 39 at 60000; 256 1.9 and 2.7 at 300,
+// 16 and 20 at 60000; with 8 and 16 entries 0.5 - 0.9 of QUAD.  One
+// range stays with QUAD: launches of 12 to 16 rows (20, below 768 neurons) for every CU, where QUAD has always run and the
+// tests look for it (1024 neurons, 3840 rows: 5.1 against 6.3).
 static bool tiles_by_size(const spdnn_net* n) {
     const int cu = n->n_cu;
     return n->N > 1024 || n->carried < 12 * cu || n->carried >= (n->N >= 768 ? 16 : 20) * cu;
@@ -2078,6 +2078,28 @@ static ResidentSig resident_sig(const spdnn_net* n, int l, bool tiles = true) { 
         if (g.rows == 0 || n->RB % g.rows != 0) g.ok = 0;
     }
     return g;
+}
+
+// Whether k layers of tiles in one launch take less than a walk for each (bands wider than 1024 neurons, which have no QUAD
+// form).  A layer of tiles takes the same time for one row as for sixteen of every CU; a walk takes as long as its launch up to
+// 256 rows, and from there on the time of its bytes.  us per layer, tiles and walks, 32 entries: 2304 neurons 64 rows 10.0 and
+// 6.4, 512 10.0 and 9.2, 768 10.2 and 12.0, 4096 10.3 and 20, 4352 19.9 and 20.3, 16000 39 and 62; 2048 neurons 300 rows 9.0
+// and 8.9, 2000 9.0 and 10.4; 1280 neurons 64 rows 5.7 and 5.5, 512 5.7 and 6.9; 8 entries, 2304 neurons 64 rows 7.0 and 5.9, 2048
+// neurons 300 rows 6.2 and 7.3.  The launch itself, the count behind it and the rows in and out take 8 us while they stay on
+// chip, 36 (of 14 million values) to 110 (of 37 million) from memory (less where no look comes between and the walk does
+// not find its rows on chip either: 60 layers of 24000 x 1536, four in tiles and one alone in turn, 3.81 ms against 4.96); eight layers
+// of 4352 rows of 2304 neurons 203 us against 185, of 768 rows of 2048 90 and 99.  moving: rows are dying, and the host looks behind every walk, up to 25 us more
+// until the counts settle, and few rows may soon be fewer (24 layers of 64 rows, 2048 neurons: 8 entries 181 us against 212, 32
+// entries 257 and 219; four layers at a time of 16000 x 2304 1.30 ms against 1.21).
+static bool wide_tiles_pay(const spdnn_net* n, int steps, int k, bool moving) {
+    const int rows = n->carried, rounds = (rows / 16 + n->n_cu - 1) / n->n_cu;
+    const double values = 1e-6 * (double)rows * (double)n->N;
+    steps = steps <= 24 ? 24 : steps <= 32 ? 32 : steps <= 36 ? 36 : 48;   // (what band_tile_resident_kernel runs)
+    const double walk = rows <= 256 || (moving && rows <= 512) ? (steps == 32 ? 6.1 : 5.7) : rows <= 512 ? 5.0 + (1.4 + 0.042 * steps) * values
+                        : rows <= 2048 ? (n->N > 2048 ? 11.2 : 9.3) + 0.3 * values : 6.0 + 1.5 * values;
+    const double tile = rounds * (0.4 + (1.4 + 0.062 * steps) * n->N / 1024.0);
+    const double launch = 8.0 + 2.6 * std::max(0.0, values - 2.5);
+    return (moving ? std::min(100.0, launch) - std::min(25.0, 2.5 * k) : std::min(70.0, launch)) + k * tile < k * walk;
 }
 
 // The band resident kernels find the QUAD or TILE form of their j-th layer j strides behind that of their first: whether
@@ -2382,7 +2404,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 const bool wide_rows = rsig.rows >= 16 && rsig.ok < 3;
                 // (band quads: a layer inside the launch takes 0.88 of its time alone at 60000 rows, 0.76 at 6000, and rows in
                 // and out cost the launch what 1.5 layers take at either size: worth it from 16 and from 6 layers)
-                // (band tiles: from 4; 120 layers that keep 40000 of 60000 rows take 8.4 ms with 3 or 4, 8.6 with 8, 8.7 with 16)
+                // (band tiles: from 4, where wide_tiles_pay does not say otherwise)
                 auto shortest = [&](const ResidentSig& g) {
                     if (persist_asked || wide_rows) return 2;
                     if (g.ok < 3) return 8;
@@ -2417,7 +2439,9 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // faster one - measured per layer at batch 60000: N=2048 376 against 337 us, N=4096 1232 against 948; at 2048
                 // rows 13 against 38 and 42 against 57)
                 const bool too_large = !persist_asked && rsig.ok == 2 && !wide_rows && n->carried >= n->tiled_min_rows;
-                if (k >= rmin && !too_large) { c = k; resident = true; }
+                const bool pays = rsig.ok != 4 || n->N <= 1024 || persist_asked || n->tile_mode == 2 ||
+                                  wide_tiles_pay(n, rsig.ngroups, k, opt.prune && st.c_prune <= 1);
+                if (k >= rmin && !too_large && pays) { c = k; resident = true; }
             }
             const bool pair = !fb && !resident && !chain && !head && is_pair(l);
             if (pair) c = 2;
@@ -2707,7 +2731,8 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             bool worth = (double)st.newest_count <= (double)thr * (double)n->carried;
             if (!worth && thr >= 0.75f && st.newest_count > 0 && st.l <= last && nb * n->RB < n->carried) {   // (fewer rounds of workgroups)
                 const LayerPlan& q = n->layers[(size_t)st.l];
-                const bool tiles = !st.sums && persist_on && n->resident_mode && resident_sig(n, st.l).ok == 4;
+                const bool tiles = !st.sums && persist_on && n->resident_mode && resident_sig(n, st.l).ok == 4 &&
+                                   (n->N <= 1024 || wide_tiles_pay(n, q.tile_steps, last - st.l + 1, false));
                 auto layer_us = [&](int rows) {
                     return st.sums ? sums_layer_us(st.sums, rows, n->n_cu, true) : tiles ? band_tile_layer_us(n->N, q.tile_steps, rows, n->n_cu) : 0.0;
                 };

@@ -2487,3 +2487,36 @@ def test_waiting_for_counts_leaves_the_processor_alone(gc):
             assert time.perf_counter() - t > 0.014
         print("share of a processor:", shares, flush=True)
         assert sorted(shares)[2] < 0.6 and slack() == before
+
+
+@pytest.mark.parametrize("N,B,K,pattern,prune,kinds", [
+    (2304, 64, 32, "0" * 24, False, []),                       # a walk costs its launch, a layer of tiles what 4096 rows cost
+    (2304, 3000, 32, "0" * 24, False, ["band tiles"]),
+    (2304, 4300, 32, "0" * 8, False, []),                      # a second round for 256 rows
+    (2048, 300, 32, "0" * 24, False, []),
+    (2048, 300, 8, "0" * 24, False, ["band tiles"]),
+    (1280, 64, 32, "0" * 24, False, []),
+    (1536, 64, 16, "0" * 24, False, ["band tiles"]),
+    (2048, 2000, 32, "1" + "0" * 4, False, []),                # too few layers for the rows in and out
+    (2048, 2000, 32, "1" + "0" * 23, False, ["band tiles"]),
+])
+def test_where_band_layers_run_in_tiles(gc, orc, monkeypatch, capfd, N, B, K, pattern, prune, kinds):
+    """Band layers of one weight ("0") and of several ("1") run in the launches that measured faster at their size; whatever
+    they run in, the values are those of one launch per layer."""
+    print("launches of bands N=%d B=%d K=%d %s" % (N, B, K, pattern), flush=True)
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    with gc.Network(N, B, len(pattern), bias=-0.3) as net:
+        for l, kind in enumerate(pattern):
+            rp, c, v = orc.gen_layer_csr(11, l % 6, N, K, 2.0 / K)
+            if kind == "1":
+                v = (v * np.tile(np.float32([0.5, 2.0]), len(v) // 2)).astype(np.float32)
+            net.set_layer_csr(l, rp, c, v)
+        net.inspect()
+        net.synth_features(3, B, 0.4, 0.6)
+        ask = np.arange(0, B, 1 + B // 500, dtype=np.int32)
+        net.run(prune=prune, fuse_layers=1)
+        want, cats = net.activations(ask), net.categories()
+        _launch_kinds(capfd)
+        net.run(prune=prune)
+        assert [k for k, _ in _launch_kinds(capfd)] == kinds
+        assert np.array_equal(net.categories(), cats) and same_floats(net.activations(ask), want)
