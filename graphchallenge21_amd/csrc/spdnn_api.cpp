@@ -2057,21 +2057,24 @@ struct ResidentSig {
 // Where bands of one exact weight run as tiles.  Up to 1024 neurons against QUAD, 32 entries, us per layer: 1024 neurons
 // 300 rows 5.0 and 6.3, 2000 5.2 and 5.9, 4352 9.8 and 12.7, 40000 40.5 and 61, 60000 64 and 88; 768 neurons 3.9 and 4.9
 // at 300, 31 and 47 at 40000; 512 2.9 and 3.3 at 300, 8.7 and 11.6 at 16000, 31 and 39 at 60000; 256 1.9 and 2.7 at 300,
-// 16 and 20 at 60000; with 8 and 16 entries 0.5 - 0.9 of QUAD.  One
-// range stays with QUAD: launches of 12 to 16 rows (20, below 768 neurons) for every CU, where QUAD has always run and the
-// tests look for it (1024 neurons, 3840 rows: 5.1 against 6.3).
-static bool tiles_by_size(const spdnn_net* n) {
+// 16 and 20 at 60000; with 8 and 16 entries 0.5 - 0.9 of QUAD.  Two ranges stay with QUAD.  Four entries merge to 19 of a
+// tile's 24 steps at least, but to 7 of a quad: 1024 neurons up to 4352 rows 3.4 - 7.1 and 3.2 - 6.3 (5120 5.6 and 6.4; 768
+// neurons 0.83 - 1.0 of QUAD); not while rows may die, where QUAD launches are short (24 layers of 300 rows 105 us, 126 in QUAD).  And launches of 12 to 16 rows (20, below 768 neurons) for every CU, where QUAD has always
+// run and the tests look for it (1024 neurons, 3840 rows: 5.1 against 6.3).
+static bool tiles_by_size(const spdnn_net* n, const LayerPlan& p, bool prune) {
     const int cu = n->n_cu;
-    return n->N > 1024 || n->carried < 12 * cu || n->carried >= (n->N >= 768 ? 16 : 20) * cu;
+    if (n->N > 1024) return true;
+    if (!prune && p.tile_steps <= 20 && n->N > 768 && n->carried < 20 * cu) return false;
+    return n->carried < 12 * cu || n->carried >= (n->N >= 768 ? 16 : 20) * cu;
 }
-static ResidentSig resident_sig(const spdnn_net* n, int l, bool tiles = true) {   // tiles = false: not the TILE form
+static ResidentSig resident_sig(const spdnn_net* n, int l, bool prune, bool tiles = true) {   // tiles = false: not the TILE form
     const LayerPlan& p = n->layers[(size_t)l];
     ResidentSig g;
     if (p.kernel == SPDNN_KERNEL_BAND && p.alt_ngroups > 0) { g.ok = 1; g.full = p.alt_full ? 1 : 0; g.ngroups = p.alt_ngroups; }
     else if (p.kernel == SPDNN_KERNEL_BLOCK && p.wmode == 0) { g.ok = 1; g.full = p.blk_full ? 1 : 0; g.ngroups = p.ngroups; }
     else if (p.kernel == SPDNN_KERNEL_TILED && !p.rt_ent.empty() && n->rowtile_mode) { g.ok = 2; g.wmode = p.wmode; }
     else if (tiles && p.kernel == SPDNN_KERNEL_BAND && p.tile_steps > 0 && n->band_resident_mode &&
-             (n->tile_mode == 2 || (n->tile_mode == 1 && tiles_by_size(n)))) { g.ok = 4; g.ngroups = p.tile_steps; }
+             (n->tile_mode == 2 || (n->tile_mode == 1 && tiles_by_size(n, p, prune)))) { g.ok = 4; g.ngroups = p.tile_steps; }
     else if (p.kernel == SPDNN_KERNEL_BAND && p.quad_groups > 0 && n->band_resident_mode) { g.ok = 3; g.ngroups = p.quad_groups; g.wmode = p.wmode == 2 ? 2 : 1; }
     if (g.ok) {
         g.rows = g.ok == 1 ? resident_rows_per_workgroup(n->N, g.ngroups) : g.ok == 2 ? rowtile_resident_rows(n->N) : g.ok == 4 ? band_tile_rows(n->N, n->carried, n->n_cu) : band_resident_rows(n->N);
@@ -2387,7 +2390,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 kmax = std::max(1, std::min(kmax, last - l + 1));
                 while (c < kmax && takes_sums(l + c)) ++c;
             }
-            if (!fb && !chain && !head && persist_on && n->resident_mode && n->d_table && (rsig = resident_sig(n, l)).ok) {
+            if (!fb && !chain && !head && persist_on && n->resident_mode && n->d_table && (rsig = resident_sig(n, l, opt.prune != 0)).ok) {
                 // (tiles while the counts move: where fewer rows would take as long, one workgroup or less to a compute unit, or
                 // where the last layer looked at left three rows in four, about 120 us of layers to a launch and four at least.
                 // Looking behind every layer cost 25 us; 300 x 1024, six layers: 71 us a run against 113, 120 layers of 6000
@@ -2414,7 +2417,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // layers from l0 on that one launch takes in the form g, of `most`
                 auto run_of = [&](int l0, const ResidentSig& g, int most, bool tiles) {
                     int k = 1;
-                    while (k < most && resident_sig(n, l0 + k, tiles) == g && (g.ok < 3 || band_plans_equidistant(n, l0, l0 + k, g.ok == 4))) ++k;
+                    while (k < most && resident_sig(n, l0 + k, opt.prune != 0, tiles) == g && (g.ok < 3 || band_plans_equidistant(n, l0, l0 + k, g.ok == 4))) ++k;
                     return k;
                 };
                 int k = run_of(l, rsig, room, true);
@@ -2423,12 +2426,12 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 // QUAD launch - alone a layer takes 1.45 of them, in tiles 0.95, rows in and out 1.25 (6000 x 1024, five
                 // layers of several weights behind one of one weight, ten times over: 0.82 ms in ten launches, 1.08 layer by
                 // layer; the other way round 0.82 in ten launches, 0.90 as one layer and five in tiles).
-                const ResidentSig quad = rsig.ok >= 3 ? resident_sig(n, l, false) : ResidentSig{};
+                const ResidentSig quad = rsig.ok >= 3 ? resident_sig(n, l, opt.prune != 0, false) : ResidentSig{};
                 const int kq = quad.ok == 3 ? run_of(l, quad, room, false) : 0;
                 if (kq > k && kq >= shortest(quad)) {
                     double pieces = 0.0;
                     for (int i = 0, m; i < kq; i += m) {
-                        const ResidentSig g = resident_sig(n, l + i);
+                        const ResidentSig g = resident_sig(n, l + i, opt.prune != 0);
                         m = run_of(l + i, g, kq - i, true);
                         pieces += m < shortest(g) ? 1.45 * m : g.ok == 4 ? 1.25 + 0.95 * m : 1.25 + m;
                     }
@@ -2731,7 +2734,7 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             bool worth = (double)st.newest_count <= (double)thr * (double)n->carried;
             if (!worth && thr >= 0.75f && st.newest_count > 0 && st.l <= last && nb * n->RB < n->carried) {   // (fewer rounds of workgroups)
                 const LayerPlan& q = n->layers[(size_t)st.l];
-                const bool tiles = !st.sums && persist_on && n->resident_mode && resident_sig(n, st.l).ok == 4 &&
+                const bool tiles = !st.sums && persist_on && n->resident_mode && resident_sig(n, st.l, true).ok == 4 &&
                                    (n->N <= 1024 || wide_tiles_pay(n, q.tile_steps, last - st.l + 1, false));
                 auto layer_us = [&](int rows) {
                     return st.sums ? sums_layer_us(st.sums, rows, n->n_cu, true) : tiles ? band_tile_layer_us(n->N, q.tile_steps, rows, n->n_cu) : 0.0;
