@@ -2423,17 +2423,22 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                 int k = run_of(l, rsig, room, true);
                 // Bands under one weight have both forms, other bands the QUAD form alone.  Where a run of layers is a mixture of
                 // the two, tiles would cut it into pieces: taken as QUAD throughout if that costs less, counted in layers of a
-                // QUAD launch - alone a layer takes 1.45 of them, in tiles 0.95, rows in and out 1.25 (6000 x 1024, five
-                // layers of several weights behind one of one weight, ten times over: 0.82 ms in ten launches, 1.08 layer by
-                // layer; the other way round 0.82 in ten launches, 0.90 as one layer and five in tiles).
+                // QUAD launch - alone a layer takes 1.45 of them, rows in and out 1.25, and a layer in tiles counts 0.95, so that
+                // pieces of ten layers and more run in tiles.  Layers of one other and m of one weight over and over, pieces
+                // against QUAD throughout, m = 5, 10, 24 (and what a layer in tiles takes of one in QUAD): 32 entries, 1024 neurons
+                // 6000 rows 0.88, 0.80, 0.74 (0.70), 300 rows 0.93, 0.89, 0.86 (0.80); 8 entries 0.99, 0.86, 0.79 and 1.05, 1.00,
+                // 0.97; 768 neurons 4352 rows, 32 entries 0.98, 0.86, 0.78.  Where several narrow workgroups share a CU and one
+                // round of them holds all rows the pieces' launches weigh more: 0.97, sixteen layers (512 neurons 6000 rows,
+                // 32 entries 1.25, 1.04, 0.97 and m = 16 0.99; 8 entries 1.35, 1.08, 0.97; 256 neurons 6000 rows 1.18, 1.06, 0.95).
                 const ResidentSig quad = rsig.ok >= 3 ? resident_sig(n, l, opt.prune != 0, false) : ResidentSig{};
                 const int kq = quad.ok == 3 ? run_of(l, quad, room, false) : 0;
                 if (kq > k && kq >= shortest(quad)) {
+                    const double tile = n->N < 768 && n->carried >= 16 * n->n_cu && one_round ? 0.97 : 0.95;
                     double pieces = 0.0;
                     for (int i = 0, m; i < kq; i += m) {
                         const ResidentSig g = resident_sig(n, l + i, opt.prune != 0);
                         m = run_of(l + i, g, kq - i, true);
-                        pieces += m < shortest(g) ? 1.45 * m : g.ok == 4 ? 1.25 + 0.95 * m : 1.25 + m;
+                        pieces += m < shortest(g) ? 1.45 * m : g.ok == 4 ? 1.25 + tile * m : 1.25 + m;
                     }
                     if (1.25 + kq <= pieces) { rsig = quad; k = kq; }
                 }

@@ -2502,6 +2502,9 @@ def test_waiting_for_counts_leaves_the_processor_alone(gc):
     (1024, 300, 4, "0" * 8, False, ["band quads"]),            # most of a tile's steps are padding
     (1024, 300, 4, "0" * 8, True, ["band tiles"]),
     (768, 300, 4, "0" * 8, False, ["band tiles"]),
+    (512, 6000, 32, "1" + "0" * 11, False, ["band quads"]),    # two workgroups to a CU, one round
+    (512, 6000, 32, "1" + "0" * 19, False, ["band tiles"]),
+    (1024, 6000, 32, "1" + "0" * 11, False, ["band tiles"]),
 ])
 def test_where_band_layers_run_in_tiles(gc, orc, monkeypatch, capfd, N, B, K, pattern, prune, kinds):
     """Band layers of one weight ("0") and of several ("1") run in the launches that measured faster at their size; whatever
