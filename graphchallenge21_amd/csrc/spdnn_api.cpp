@@ -869,13 +869,15 @@ int alloc_feature_buffers(spdnn_net* n) {
     return SPDNN_OK;
 }
 
-PlanLayout plan_layout(const LayerPlan& p) {
+// (streamed plans run layer by layer: no launch there reads the records of tiles, 64 bytes a neuron that would cross the link
+// with every layer)
+PlanLayout plan_layout(const LayerPlan& p, bool streamed) {
     PlanLayout y;
     const size_t len[kPlanArrays] = {p.pairs.size() * 4,    p.ell_col.size() * 4,  p.rowlen.size() * 4,   p.wv.size() * 4,
                                      p.dst.size() * 4,      p.blk_cols.size() * 4, p.blk_cnt.size() * 4,  p.alt_cols.size() * 4,
                                      p.alt_cnt.size() * 4,  p.alt_dst.size() * 4,  p.alt_wv.size() * 4,
                                      p.rt_ent.size() * 4,   p.quad_col.size() * 4, p.quad_w.size() * 4,   p.sum_cols.size() * 2,
-                                     p.tile_rec.size() * 4};
+                                     streamed ? 0 : p.tile_rec.size() * 4};
     for (int k = 0; k < kPlanArrays; ++k) {
         y.off[k] = y.bytes;
         y.len[k] = len[k];
@@ -919,13 +921,13 @@ int upload_plans(spdnn_net* n) {
     const size_t L = (size_t)n->L;
     n->lay.assign(L, PlanLayout{});
     size_t total = 0, largest = 0;
+    const bool streamed = n->plan_window >= 2 && (size_t)n->plan_window < L;
     for (size_t l = 0; l < L; ++l) {
-        n->lay[l] = plan_layout(n->layers[l]);
+        n->lay[l] = plan_layout(n->layers[l], streamed);
         total += n->lay[l].bytes;
         largest = std::max(largest, n->lay[l].bytes);
     }
     n->dl.assign(L, DevLayer{});
-    const bool streamed = n->plan_window >= 2 && (size_t)n->plan_window < L;
     if (!streamed) {
         HIPCHK(dev_malloc(&n->arena, std::max<size_t>(total, 256)));
         std::vector<char> blob(largest);

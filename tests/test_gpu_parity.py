@@ -2526,3 +2526,27 @@ def test_where_band_layers_run_in_tiles(gc, orc, monkeypatch, capfd, N, B, K, pa
         net.run(prune=prune)
         assert [k for k, _ in _launch_kinds(capfd)] == kinds
         assert np.array_equal(net.categories(), cats) and same_floats(net.activations(ask), want)
+
+
+@pytest.mark.parametrize("N,K", [(256, 8), (1024, 32), (2048, 32), (2304, 4)])
+def test_streamed_plans_leave_out_what_only_resident_launches_read(gc, orc, N, K):
+    """The records of tiles (64 bytes a neuron) are on the device where a launch of several layers can read them, and do not
+    cross the link with every layer where plans are streamed; the rows are the same."""
+    print("streamed plans of bands N=%d K=%d" % (N, K), flush=True)
+    B, L = 300, 6
+    feats = orc.gen_features(3, N, 0, B, 0.4, 0.6)
+    got = []
+    for window in (0, 3):
+        with gc.Network(N, B, L, bias=-0.3) as net:
+            net.set_plan_window(window)
+            net.synth_layers(5, nnz_per_row=K, value=2.0 / K)
+            net.inspect()
+            net.set_features_dense(feats)
+            for fuse in (0, 2):
+                net.run(prune=False, fuse_layers=fuse)
+                got.append(net.activations(np.arange(B, dtype=np.int32)))
+            w, device, pinned = net.plan_memory()
+            assert w == window and same_floats(got[0], got[-1])
+            if window:
+                assert pinned == resident - L * 64 * N and device == window * pinned // L
+            resident = device
