@@ -2933,9 +2933,11 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     // copy command, and no copy in device memory in between), the host copies them out while the next slots are filled.
     // Behind a layer of equal groups a group's value goes over the link once, a sixteenth of the row, and the host writes it
     // to the group's neurons: what is left is the rate at which the host's threads write (9 MB 0.16
-    // ms, 0.28 with whole rows over the link; 29 MB 0.29, 0.72; 590 MB into a fresh array 6.3, 12.2).
+    // ms, 0.28 with whole rows over the link; 29 MB 0.29, 0.72; 590 MB into a fresh array 6.3, 12.2).  Not where the calling
+    // thread is alone with them: it writes from the list of groups slower than it copies (64 KB 24 us, 23 as whole rows; 1 MB 71 -
+    // 76, 64; 2 MB 121 - 129, 110; with the crew, 2.1 MB, 67 - 74 and 97 - 115).
     const size_t row_bytes = (size_t)n->N * 4, id_bytes = (size_t)nrows * 4;
-    int groups = n->pinned_staging ? output_groups(n) : 0;
+    int groups = n->pinned_staging && (size_t)nrows * row_bytes >= kCrewMinBytes ? output_groups(n) : 0;
     StageLease lease(n->stream);
     const size_t lent_bytes = groups ? (size_t)groups * 4 : row_bytes;
     int rc = lend_staging(n, (size_t)nrows * lent_bytes, lent_bytes, &lease);

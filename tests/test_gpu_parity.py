@@ -2367,8 +2367,10 @@ def test_slabs_of_group_sums(gc, orc, monkeypatch, capfd, N, B, kind, rl, S):
 
 
 @pytest.mark.parametrize("N,B,asked,window", [
-    (512, 40, 70, 0),         # one piece, written by the calling thread
-    (1008, 900, 1300, 0),     # past the size from which the writing is shared out
+    (512, 40, 70, 0),         # too little for more than the calling thread: whole rows
+    (1008, 900, 1300, 0),     # past the size from which the writing is shared out, and the rows go by group
+    (1024, 900, 511, 0),      # the last that goes as whole rows
+    (1024, 900, 512, 0),      # 2 MiB, the first by group
     (1024, 6000, 5000, 0),    # 20 MB, written past the caches
     (16384, 300, 520, 0),     # 34 MB, several pieces
     (1024, 700, 900, 3),      # streamed plans: another layer's plan may lie where this layer's did
