@@ -4349,9 +4349,13 @@ hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const i
     return hipGetLastError();
 }
 
-hipError_t launch_fill_i32(int32_t* p, int n, int32_t v, hipStream_t s) {
-    if (n <= 0 || !p) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(fill_i32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
+hipError_t launch_fill_i32(int32_t* p, size_t n, int32_t v, hipStream_t s) {
+    if (n == 0 || !p) return hipErrorInvalidValue;
+    for (size_t at = 0; at < n;) {   // (the kernel counts in int)
+        const int part = (int)std::min<size_t>(n - at, (size_t)1 << 30);
+        hipLaunchKernelGGL(fill_i32_kernel, dim3((part + 255) / 256), dim3(256), 0, s, p + at, part, v);
+        at += (size_t)part;
+    }
     return hipGetLastError();
 }
 

@@ -403,7 +403,7 @@ hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const i
                               int nreq, int N, int rl, const int32_t* active, int stamp, float* rowmajor,
                               hipStream_t s, int cols = -1, int stride = 1);   // cols >= 0: columns phys_of_col[0], [stride], ... only
 
-hipError_t launch_fill_i32(int32_t* p, int n, int32_t v, hipStream_t s);
+hipError_t launch_fill_i32(int32_t* p, size_t n, int32_t v, hipStream_t s);
 hipError_t launch_iota_gid(int32_t* gid, int rows, int batch, hipStream_t s);
 // where[g] = physical row (< carried) whose global id is g, -1 if none, for g in [0, batch)
 hipError_t launch_row_table(const int32_t* gid, int carried, int batch, int32_t* where, hipStream_t s);

@@ -2520,12 +2520,12 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
             n->stamp += c;
             if (!group && !counts_clear) {
                 const int from = st.count_pending ? std::max(first, l - 1) : l;   // (launches of several layers have stored theirs)
-                HIPCHK(launch_fill_i32(n->d_counts + from, last - from + 1, 0, n->stream));
+                HIPCHK(launch_fill_i32(n->d_counts + from, (size_t)(last - from + 1), 0, n->stream));
                 counts_clear = true;
             }
             if (persist && !persist_clear) {
-                HIPCHK(launch_fill_i32(n->d_done + (size_t)first * n->done_stride, nl * n->done_stride, 0, n->stream));
-                HIPCHK(launch_fill_i32(reinterpret_cast<int32_t*>(n->d_ctl), (int)((size_t)nl * sizeof(PersistCtl) / 4), 0, n->stream));
+                HIPCHK(launch_fill_i32(n->d_done + (size_t)first * n->done_stride, (size_t)nl * n->done_stride, 0, n->stream));
+                HIPCHK(launch_fill_i32(reinterpret_cast<int32_t*>(n->d_ctl), (size_t)nl * sizeof(PersistCtl) / 4, 0, n->stream));
                 persist_clear = true;
             }
             if (opt.time_layers) HIPCHK(hipEventRecord(n->ev_layer[(size_t)(2 * l)], n->stream));

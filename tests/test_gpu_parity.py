@@ -2552,3 +2552,27 @@ def test_streamed_plans_leave_out_what_only_resident_launches_read(gc, orc, N, K
             if window:
                 assert pinned == resident - L * 64 * N and device == window * pinned // L
             resident = device
+
+
+def test_row_blocks_times_layers_beyond_an_int(gc, monkeypatch):
+    """A persistent launch's words per layer and row block are cleared for the whole call: 65535 row blocks through 32769
+    layers are 2^31 + 32767 of them.  The rows die in the second layer, so that nearly all of the depth is the clearing."""
+    print("row blocks times layers beyond an int", flush=True)
+    monkeypatch.setenv("SPDNN_ROWS_PER_LANE", "1")
+    monkeypatch.setenv("SPDNN_BAND_RESIDENT", "0")
+    monkeypatch.setenv("SPDNN_REGION_PAIRING", "0")
+    N, B, L = 256, 64 * 65535, 32769
+    with gc.Network(N, B, L, bias=-0.9) as net:
+        net.synth_layers(3, nnz_per_row=4, value=0.5)
+        net.inspect()
+        print("  inspected", flush=True)
+        net.synth_features(3, B, 0.05, 0.05)
+        print("  features set", flush=True)
+        net.run(prune=True, n_layers=3, fuse_layers=1)
+        want = [net.active_count(l) for l in range(3)]
+        assert 0 < want[0] < B and want[2] == 0
+        for n in (3, L):
+            r = net.run(prune=True, n_layers=n, fuse_layers=2)
+            print("  run of", n, flush=True)
+            assert r.persistent_launches >= 1 and r.persistent_fallbacks == 0 and r.active_rows == 0
+            assert [net.active_count(l) for l in range(3)] == want
