@@ -3365,13 +3365,12 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(
 }
 
 __global__ void unpack_rows_kernel(Feat y, const int32_t* __restrict__ phys_of_col,
-                                   const int32_t* __restrict__ row_ids, const int32_t* __restrict__ where, int N, int RB,
+                                   const int32_t* __restrict__ phys, int N, int RB,
                                    const int32_t* __restrict__ active, int stamp, float* __restrict__ rowmajor, int cols,
                                    int stride) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= cols) return;
-    const int id = row_ids[blockIdx.y];
-    const int pr = where ? where[id] : id;
+    const int pr = phys[blockIdx.y];
     float x = 0.0f;
     // a row that the last layer did not stamp is all zero by definition (its block may have been
     // skipped, leaving stale data in the buffer)
@@ -4339,12 +4338,12 @@ hipError_t launch_pack_rows(const float* rowmajor, const Feat& y, const int32_t*
     return hipGetLastError();
 }
 
-hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* row_ids, const int32_t* where, int nreq,
+hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* phys, int nreq,
                               int N, int rl, const int32_t* active, int stamp, float* rowmajor, hipStream_t s, int cols, int stride) {
     if (cols < 0) cols = N;
     if (nreq <= 0 || nreq > 65535 || N <= 0 || cols == 0 || cols > N || stride < 1) return hipErrorInvalidValue;
     dim3 grid((cols + 255) / 256, nreq);
-    hipLaunchKernelGGL(unpack_rows_kernel, grid, dim3(256), 0, s, y, phys_of_col, row_ids, where, N, 64 * rl, active,
+    hipLaunchKernelGGL(unpack_rows_kernel, grid, dim3(256), 0, s, y, phys_of_col, phys, N, 64 * rl, active,
                        stamp, rowmajor, cols, stride);
     return hipGetLastError();
 }

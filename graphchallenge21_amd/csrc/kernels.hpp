@@ -396,12 +396,10 @@ hipError_t launch_synth_features(const Feat& y, const int32_t* col_of_phys, int 
 hipError_t launch_pack_rows(const float* rowmajor, const Feat& y, const int32_t* phys_of_col, int N,
                             int64_t row0, int nrows, int rl, int32_t* nonfinite, hipStream_t s);
 
-// Row-block layout to row-major for a list of rows: physical rows, or with `where` (see launch_row_table) global ids
-// (physical row -1 gives a zero row).
+// Row-block layout to row-major for a list of physical rows (-1 gives a zero row).
 // `active`/`stamp`: rows whose stamp differs read back as zero rows (stamp 0 = no check).
-hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* row_ids, const int32_t* where,
-                              int nreq, int N, int rl, const int32_t* active, int stamp, float* rowmajor,
-                              hipStream_t s, int cols = -1, int stride = 1);   // cols >= 0: columns phys_of_col[0], [stride], ... only
+hipError_t launch_unpack_rows(const Feat& y, const int32_t* phys_of_col, const int32_t* phys, int nreq, int N, int rl,
+                              const int32_t* active, int stamp, float* rowmajor, hipStream_t s, int cols = -1, int stride = 1);   // cols >= 0: columns phys_of_col[0], [stride], ... only
 
 hipError_t launch_fill_i32(int32_t* p, size_t n, int32_t v, hipStream_t s);
 hipError_t launch_iota_gid(int32_t* gid, int rows, int batch, hipStream_t s);

@@ -2975,7 +2975,7 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
     auto rows_in = [&](int k) { return std::min(per, nrows - k * per); };
     if (!pinned) {
         for (int k = 0; k < K; ++k) {
-            HIPCHK(launch_unpack_rows(n->cur, lab, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+            HIPCHK(launch_unpack_rows(n->cur, lab, d_phys + (size_t)k * per, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
                                       n->d_stage, n->stream));
             HIPCHK(hipMemcpyAsync(rowmajor + (size_t)k * per * n->N, n->d_stage, (size_t)rows_in(k) * row_bytes, hipMemcpyDeviceToHost, n->stream));
         }
@@ -3010,7 +3010,7 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
             HIPCHK(ready(arrived++));
             crew.wait(k - kStageSlots);
         }
-        HIPCHK(launch_unpack_rows(n->cur, cols, d_phys + (size_t)k * per, nullptr, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
+        HIPCHK(launch_unpack_rows(n->cur, cols, d_phys + (size_t)k * per, rows_in(k), n->N, n->rl, n->d_active, n->last_stamp,
                                   (float*)lease.at(k), n->stream, groups ? groups : n->N, groups ? 16 : 1));
         HIPCHK(hipEventRecord(n->ev_stage[k % kStageSlots], n->stream));
     }
@@ -3051,7 +3051,7 @@ static int spdnn_get_activations_noalloc_impl(spdnn_net* n, const int32_t* rows,
         const int m = std::min(chunk, nrows - i0);
         HIPCHK(hipMemcpyAsync(d_ids, rows + i0, (size_t)m * 4, hipMemcpyHostToDevice, n->stream));
         HIPCHK(launch_lookup_rows(d_ids, m, d_where, d_phys, n->stream));
-        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys, nullptr, m, n->N, n->rl, n->d_active, n->last_stamp, d_out, n->stream));
+        HIPCHK(launch_unpack_rows(n->cur, lab, d_phys, m, n->N, n->rl, n->d_active, n->last_stamp, d_out, n->stream));
         HIPCHK(hipMemcpyAsync(rowmajor + (size_t)i0 * n->N, d_out, (size_t)m * row_bytes, hipMemcpyDeviceToHost, n->stream));
         HIPCHK(hipStreamSynchronize(n->stream));  // the staging rows are reused by the next pass
     }

@@ -1946,7 +1946,7 @@ def test_tiles_add_in_ascending_order_over_the_whole_range(gc, orc, monkeypatch,
 
 @pytest.mark.parametrize("N,B,kind", [(1024, 4100, "band tiles"), (768, 4100, "band tiles"), (1024, 3800, "band quads"), (512, 4100, "band quads")])
 def test_where_resident_launches_run_in_tiles_by_default(gc, monkeypatch, capfd, N, B, kind):
-    """By default from 768 neurons and sixteen rows for every compute unit."""
+    """Launches of 12 to 16 rows (to 20, below 768 neurons) for every compute unit keep the QUAD form by default."""
     monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
     with gc.Network(N, B, 8, bias=-0.3) as net:
         net.synth_layers(3, nnz_per_row=32, value=0.0625)
@@ -2035,7 +2035,7 @@ def test_run_that_ends_in_an_error_inside_group_sums(gc, orc, monkeypatch, calls
 
 @pytest.mark.parametrize("L,asked", [(300, 300), (255, 1000), (256, 255)])
 def test_more_layers_than_one_launch_in_tiles_holds(gc, L, asked):
-    """A caller may ask for launches of any number of layers: those in tiles, which hold 254, are cut.  Against one launch
+    """A caller may ask for launches of any number of layers, in tiles too (more than a byte counts).  Against one launch
     per layer."""
     print("tiles, %d layers in launches of up to %d" % (L, asked), flush=True)
     N, B = 1024, 4200
@@ -2060,7 +2060,7 @@ def test_more_layers_than_one_launch_in_tiles_holds(gc, L, asked):
     (1024, 4200, "011111" * 3, 3, 3),     # behind one layer of one weight those of several, too few for a launch of their own
     (768, 4200, "100000" * 3, 3, 3),      # the other way round: alone the first layer would be left over
     (1024, 4200, "1" + "0" * 17, 1, 2),   # long enough in tiles: the first layer alone
-    (512, 900, "011111" * 2, 2, 2),       # narrower layers keep the QUAD form anyway
+    (512, 900, "011111" * 2, 2, 2),       # narrower layers, few rows
 ])
 def test_resident_launches_of_bands_of_one_weight_among_others(gc, orc, N, B, pattern, resident, launches):
     """Band layers of one power-of-two weight (which have a TILE form) among band layers of several (which do not): one
