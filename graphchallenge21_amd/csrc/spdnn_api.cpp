@@ -24,8 +24,10 @@
 #include <thread>
 #include <vector>
 
-#include <emmintrin.h>
 #include <sys/prctl.h>
+#if defined(__SSE2__)
+#include <emmintrin.h>
+#endif
 
 #include "../../include/spdnn.h"
 #include "inspector.hpp"
@@ -682,12 +684,20 @@ int output_groups(spdnn_net* n) {
     }
     return G;
 }
-// A row from its group values.  `stream`: past the caches (a transfer larger than those; rows start at 16 bytes)
+// A row from its group values.  `stream`: past the caches (a transfer larger than those; rows start at 16 bytes), where the
+// processor has such stores; end_stream makes them visible to other threads.
 void expand_row(float* out, const float* sums, const uint16_t* group, int N, bool stream) {
     int j = 0;
+#if defined(__SSE2__)
     if (stream)
         for (; j + 4 <= N; j += 4) _mm_stream_ps(out + j, _mm_setr_ps(sums[group[j]], sums[group[j + 1]], sums[group[j + 2]], sums[group[j + 3]]));
+#endif
     for (; j < N; ++j) out[j] = sums[group[j]];
+}
+void end_stream() {
+#if defined(__SSE2__)
+    _mm_sfence();
+#endif
 }
 // Part `part` of CopyCrew::kParts of a piece of `bytes`
 void copy_part(void* dst, const void* src, size_t bytes, int part) {
@@ -2991,7 +3001,7 @@ static int spdnn_get_activations_impl(spdnn_net* n, const int32_t* rows, int nro
         const int lo = (int)((int64_t)rows_in(k) * part / CopyCrew::kParts), hi = (int)((int64_t)rows_in(k) * (part + 1) / CopyCrew::kParts);
         for (int i = lo; i < hi; ++i)
             expand_row(to + (size_t)i * n->N, (const float*)lease.at(k) + (size_t)i * groups, n->group_of.data(), n->N, stream);
-        if (stream) _mm_sfence();
+        if (stream) end_stream();
     });
     const int32_t* cols = lab;
     if (groups) {   // the column of a group's first output
