@@ -2676,8 +2676,10 @@ static int spdnn_run_impl(spdnn_net* n, const spdnn_run_options* opt_in, spdnn_r
                                           n->d_alive_gid, n->stream));
                 HIPCHK(hipMemcpyAsync(n->d_counts + l, n->d_count, 4, hipMemcpyDeviceToDevice, n->stream));
             }
-            // (behind a head the next launch skips the rows that died by itself: nobody needs their number before that)
-            const bool look_later = head && opt.prune && sums_slab_rows(st.sums, n->carried, n->n_cu, true) != 0;
+            // (behind a head the next launch skips the rows that died by itself: nobody needs their number before that.  Where
+            // the layer in front of the head is still to be counted that is done here, and the head with it: the next launch
+            // counts one layer back)
+            const bool look_later = head && opt.prune && !st.count_pending && sums_slab_rows(st.sums, n->carried, n->n_cu, true) != 0;
             if (fused_count && group && look_later) {
                 if (polled && st.pub.n > 0) recs.push_back({(int)(st.pub.src - n->d_counts), st.pub.n, -1});
                 st.pub = Publish{};

@@ -2415,7 +2415,7 @@ def test_runs_after_a_compaction_made_by_a_launch_of_group_sums(gc, orc, monkeyp
     N, B, L = 512, 6000, 25 if how == "all rows die" else 13
     layers = [radix_like_csr(rng, N, 16 << (l % 4)) for l in range(L)]
     if how == "another class behind":
-        layers[7:] = [random_csr(rng, N, rng.integers(20, 40, size=N), "uniform") for _ in range(L - 7)]
+        layers[7:] = [sort_rows(random_csr(rng, N, rng.integers(20, 40, size=N), "uniform")) for _ in range(L - 7)]
     if how == "all rows die":
         layers[7] = (layers[7][0], layers[7][1], -layers[7][2])
     feats = (rng.random((B, N)) < np.where(rng.random((B, 1)) < 0.3, 0.5, 0.2)).astype(np.float32)
@@ -2576,3 +2576,34 @@ def test_row_blocks_times_layers_beyond_an_int(gc, monkeypatch):
             print("  run of", n, flush=True)
             assert r.persistent_launches >= 1 and r.persistent_fallbacks == 0 and r.active_rows == 0
             assert [net.active_count(l) for l in range(3)] == want
+
+
+@pytest.mark.parametrize("B", [1500, 700])     # (with more and with fewer rows than group sums take many of to a workgroup)
+@pytest.mark.parametrize("front", ["band", "band of several weights", "unstructured"])
+def test_layers_in_front_of_group_sums_are_counted(gc, orc, monkeypatch, capfd, B, front):
+    """The layer in front of a run of group sums is a launch of its own, counted by what comes behind it: with its count lost
+    the layers behind would have no rows, and the run no categories."""
+    print("layers in front of group sums, %s, %d rows" % (front, B), flush=True)
+    monkeypatch.setenv("SPDNN_RUN_VERBOSE", "1")
+    rng = np.random.default_rng(21)
+    N, L = 512, 9
+    layers = [radix_like_csr(rng, N, 16 << (l % 4)) for l in range(L)]
+    for l in (0, 4):
+        rp, c, v = sort_rows(random_csr(rng, N, rng.integers(20, 40, size=N), "uniform")) if front == "unstructured" else orc.gen_layer_csr(11, l, N)
+        layers[l] = (rp, c, (v * np.tile(np.float32([0.5, 2.0]), len(v) // 2)).astype(np.float32) if front == "band of several weights" else v)
+    feats = (rng.random((B, N)) < np.where(rng.random((B, 1)) < 0.8, rng.uniform(0.4, 0.6, (B, 1)), 0.2)).astype(np.float32)
+    ref = orc.infer(feats, layers, -0.3, prune=False, keep=set(range(L)))
+    every = np.arange(B, dtype=np.int32)
+    with gc.Network(N, B, L, bias=-0.3) as net:
+        for l, csr in enumerate(layers):
+            net.set_layer_csr(l, *csr)
+        net.inspect()
+        net.set_features_dense(feats)
+        for n in (4, L, 4, L):
+            _launch_kinds(capfd)
+            r = net.run(prune=True, n_layers=n, compact_threshold=1e-6 if n == 4 else 0.75)
+            assert [k for k, _ in _launch_kinds(capfd) if k.startswith("head")] == ["head, lists"] * (1 if n == 4 else 2)
+            assert [net.active_count(l) for l in range(n)] == [len(a) for a in ref["active_ids"][:n]]
+            assert r.active_rows == len(ref["active_ids"][n - 1]) > B // 2
+            assert np.array_equal(net.categories(), ref["active_ids"][n - 1])
+            assert same_floats(net.activations(every), ref["kept"][n - 1][1])
