@@ -97,8 +97,9 @@ typedef struct spdnn_run_options {
                                   - resident launches where consecutive layers have a BLOCK form with one exact weight
                                     (RadiX-Net layers) or are TILED layers, at most 4096 neurons wide, or are BAND layers
                                     at most 1024 neurons wide (from 6 layers on, from 16 at 16384 rows and more; under one
-                                    power-of-two weight up to 2304 neurons, from 4 layers on, on the matrix cores but
-                                    for launches of 12 - 16 rows per compute unit): a workgroup keeps 32, 16, 8 or 4 rows
+                                    power-of-two weight from 4 layers on and on the matrix cores, but for launches of 12 - 16
+                                    rows per compute unit, to 20 below 768 neurons; such layers of up to 2304 neurons
+                                    where that is faster than a launch per layer): a workgroup keeps 32, 16, 8 or 4 rows
                                     in LDS through up to 64 layers (SPDNN_RESIDENT=0: never; SPDNN_BAND_RESIDENT=0: not
                                     the BAND layers);
                                     three or more consecutive layers with such a BLOCK form, of any width up to 65536, carry
@@ -336,8 +337,9 @@ int spdnn_get_categories(spdnn_net* net, int32_t* ids, int64_t cap, int64_t* n);
  * The rows go through pinned slots that the networks of a process share: four of at most 16 MiB (or of one row, where that
  * is more) for each transfer under way, at most two such sets kept when none is, one of at most 16 MiB when the last
  * network has been destroyed.  Where no memory can be pinned (or SPDNN_PINNED_STAGING=0) they go through pageable memory.
- * Behind a layer of equal groups (a BLOCK form with one exact weight, plans resident) one value per group goes over the
- * link and the host's threads write it to the group's neurons (SPDNN_GROUP_SUMS=0: whole rows). */
+ * Behind a layer of equal groups (a BLOCK form with one exact weight, plans resident) 2 MiB of rows and more go as one value
+ * per group over the link and the host's threads write it to the group's neurons (SPDNN_GROUP_SUMS=0: whole rows; so do
+ * rows read after a layer has been handed over anew). */
 int spdnn_get_activations(spdnn_net* net, const int32_t* rows, int nrows, float* rowmajor);
 
 /* spdnn_get_activations for callers that cannot allocate device memory (tight serving loops,
