@@ -1117,6 +1117,14 @@ hipError_t labelling_dev(spdnn_net* n, int layers_done, const int32_t** out) {
     return hipSuccess;
 }
 
+// To be called before the plans of layers [first, first + count) are written anew: rows that a run left in front of one of
+// them may still be read until the next inspection, and lie in the labelling of the plan that is about to go.
+hipError_t keep_labelling(spdnn_net* n, int first, int count) {
+    const int32_t* kept = nullptr;
+    if (!n->have_features || n->cur_layer < first || n->cur_layer >= first + count) return hipSuccess;
+    return labelling_dev(n, n->cur_layer, &kept);
+}
+
 // The carried rows have moved (or are about to, in a launch that has just been queued) and d_gid_tmp holds their ids: the
 // one place where the two change, so that no compaction leaves reset_state without the mark that d_gid has to be written anew.
 void take_moved_ids(spdnn_net* n) {
@@ -1302,6 +1310,7 @@ static int spdnn_set_layer_csr_impl(spdnn_net* n, int layer, const int32_t* rowp
     auto vv = std::make_shared<std::vector<float>>();
     const std::string err = normalize_csr(n->N, rowptr, col, val, *rp, *cc, *vv);
     if (!err.empty()) return fail(SPDNN_E_ARG, err);
+    HIPCHK(keep_labelling(n, layer, 1));
     if (n->pending[(size_t)layer]) {  // the layer is being replaced: never race with its earlier job
         n->pool->wait_all();
         std::fill(n->pending.begin(), n->pending.end(), 0);
@@ -1323,6 +1332,7 @@ static int spdnn_load_layer_tsv_impl(spdnn_net* n, int layer, const char* path) 
 static int spdnn_load_layers_tsv_impl(spdnn_net* n, const char* data_dir, int first, int count) {
     if (!n || !data_dir) return fail(SPDNN_E_ARG, "NULL argument");
     if (first < 0 || count < 0 || first + count > n->L) return fail(SPDNN_E_ARG, "layer range out of bounds");
+    HIPCHK(keep_labelling(n, first, count));
     n->pool->wait_all();
     std::fill(n->pending.begin(), n->pending.end(), 0);
     n->inspected = false;
@@ -1405,6 +1415,7 @@ static int spdnn_synth_layers_impl(spdnn_net* n, uint64_t seed, int first, int c
     if (first < 0 || count < 0 || first + count > n->L) return fail(SPDNN_E_ARG, "layer range out of bounds");
     if (nnz_per_row < 1 || nnz_per_row > n->N || !std::isfinite(value))
         return fail(SPDNN_E_ARG, "bad nnz_per_row or value");
+    HIPCHK(keep_labelling(n, first, count));
     n->pool->wait_all();
     std::fill(n->pending.begin(), n->pending.end(), 0);
     n->inspected = false;

@@ -2607,3 +2607,33 @@ def test_layers_in_front_of_group_sums_are_counted(gc, orc, monkeypatch, capfd, 
             assert r.active_rows == len(ref["active_ids"][n - 1]) > B // 2
             assert np.array_equal(net.categories(), ref["active_ids"][n - 1])
             assert same_floats(net.activations(every), ref["kept"][n - 1][1])
+
+
+def test_rows_read_in_front_of_a_layer_that_was_replaced(gc, orc):
+    """Rows of a run that ended in front of a layer may be read until the network is inspected again, whatever that layer
+    has become since: they lie in the labelling its plan had."""
+    print("rows read in front of a layer that was replaced", flush=True)
+    rng = np.random.default_rng(14)
+    N, B, L = 1024, 200, 4
+    layers = [radix_like_csr(rng, N, 16 << l) for l in range(L)]
+    feats = (rng.random((B, N)) < 0.4).astype(np.float32)
+    want = orc.infer(feats, layers, -0.3, prune=False, keep={1})["kept"][1][1]
+    every = np.arange(B, dtype=np.int32)
+    for how in ("csr", "all", "first read after"):
+        with gc.Network(N, B, L, bias=-0.3) as net:
+            for l, csr in enumerate(layers):
+                net.set_layer_csr(l, *csr)
+            net.inspect()
+            net.set_features_dense(feats)
+            net.run(prune=False, n_layers=2)
+            for k in range(3):
+                if how == "all":
+                    net.synth_layers(5 + k, nnz_per_row=32, value=0.0625)
+                else:
+                    net.set_layer_csr(2, *radix_like_csr(rng, N, 32 << k))
+                if how == "first read after" and k == 0:
+                    continue
+                assert same_floats(net.activations(every), want)       # (its inspection may be under way)
+                net.layer_plan(2)
+                assert same_floats(net.activations(every), want)
+                assert same_floats(net.activations_noalloc(every), want)
