@@ -2615,9 +2615,10 @@ def test_rows_read_in_front_of_a_layer_that_was_replaced(gc, orc):
     print("rows read in front of a layer that was replaced", flush=True)
     rng = np.random.default_rng(14)
     N, B, L = 1024, 200, 4
-    layers = [radix_like_csr(rng, N, 16 << l) for l in range(L)]
+    layers = [orc.gen_layer_csr(11, l, N) for l in range(L)]      # (bands, each behind an order of its own)
     feats = (rng.random((B, N)) < 0.4).astype(np.float32)
     want = orc.infer(feats, layers, -0.3, prune=False, keep={1})["kept"][1][1]
+    assert (want[:, 1:] != want[:, :-1]).any(axis=1).all()      # (another labelling shows in every row)
     every = np.arange(B, dtype=np.int32)
     for how in ("csr", "all", "first read after"):
         with gc.Network(N, B, L, bias=-0.3) as net:
@@ -2626,14 +2627,15 @@ def test_rows_read_in_front_of_a_layer_that_was_replaced(gc, orc):
             net.inspect()
             net.set_features_dense(feats)
             net.run(prune=False, n_layers=2)
+            before = net.input_labelling(2)
             for k in range(3):
                 if how == "all":
-                    net.synth_layers(5 + k, nnz_per_row=32, value=0.0625)
+                    net.synth_layers(12 + k)
                 else:
-                    net.set_layer_csr(2, *radix_like_csr(rng, N, 32 << k))
+                    net.set_layer_csr(2, *orc.gen_layer_csr(12 + k, 2, N))
                 if how == "first read after" and k == 0:
                     continue
                 assert same_floats(net.activations(every), want)       # (its inspection may be under way)
-                net.layer_plan(2)
+                assert not np.array_equal(net.input_labelling(2), before)      # (waits for the inspection)
                 assert same_floats(net.activations(every), want)
                 assert same_floats(net.activations_noalloc(every), want)
